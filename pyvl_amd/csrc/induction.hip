@@ -5,6 +5,8 @@
 #include "pvl_internal.hpp"
 #include "induction_core.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -592,7 +594,8 @@ __global__ void __launch_bounds__(256) chain_segment_kernel(unsigned n_seg, cons
                                                             const uint32_t *__restrict__ seg_line,
                                                             const double *__restrict__ nodes,
                                                             const double *__restrict__ gamma, unsigned n_active,
-                                                            double tol, SegRec *__restrict__ out)
+                                                            double tol, SegRec *__restrict__ out,
+                                                            double *__restrict__ seg_gamma)
 {
     const unsigned j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n_seg)
@@ -609,33 +612,216 @@ __global__ void __launch_bounds__(256) chain_segment_kernel(unsigned n_seg, cons
     if (r.len < tol)
         r.ex = r.ey = r.ez = r.len = 0.0;
     const uint32_t l = ln & kInvalidId;
-    const double g = l < n_active ? gamma[l] : 0.0;
-    r.gamma = (ln & kReversed) ? -g : g;
+    double g = l < n_active ? gamma[l] : 0.0;
+    g = (ln & kReversed) ? -g : g;
+    r.pad = 0.0;
+    const double l2 = r.len * r.len;
+    constexpr double fa[kFarTerms] = {kFar1, kFar2, kFar3, kFar4, kFar5, kFar6, kFar7};
+    double q = r.len * g;
+    r.c[0] = q;
+#pragma unroll
+    for (int k = 0; k < kFarTerms; ++k)
+    {
+        q = q * l2;
+        r.c[k + 1] = fa[k] * q;
+    }
     out[j] = r;
+    seg_gamma[j] = g;
 }
 
-// PPL points per lane; the workgroup's four waves take the pieces of the item's chunk in
-// turn; per-wave sums are combined in LDS in wave order and written per chunk (no atomics).
-// Along a piece, the end node's dr = p - r becomes the next segment's dr1 (the reference form
-// also carries |dr|^2), so each segment record is one 64-byte scalar load and the accurate
-// forms spend ~66 VALU instructions per pair (cross_m).  The segment loop is unrolled by two
-// so that the carried terms are renamed, not copied.  Capped at 64 VGPRs (a few SGPRs spill to
-// VGPR lanes, none to memory): five workgroups per CU on the side stream (five waves per SIMD)
-// leave each SIMD 192 VGPRs, room for two 96-VGPR waves of the library stream's kernels.
-template <int PREC, int PPL>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8)))
-    chain_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, const double *__restrict__ nodes,
-                          const ChainPiece *__restrict__ pieces, unsigned n_pieces, unsigned cr,
-                          const SegRec *__restrict__ segs, unsigned pieces_per_chunk, double *__restrict__ partial,
-                          double tol, unsigned pblocks, unsigned n_items)
+// Segments of a piece that are active at cr filled rows.
+__device__ __forceinline__ unsigned active_segments(const ChainPiece &pc, unsigned cr)
 {
-    __shared__ double red[4][3][kWave * PPL];
+    if (!pc.row1)
+        return pc.n_seg;
+    const unsigned avail = cr - (pc.row1 - 1);
+    return pc.n_seg < avail ? pc.n_seg : avail;
+}
+
+// Axis-aligned box of the wave's points (64 PPL of them), the same in every lane.
+struct PointBox
+{
+    double lo[3], hi[3];
+};
+__device__ __forceinline__ double wave_uniform(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int PPL>
+__device__ __forceinline__ PointBox point_box(const double (&px)[PPL], const double (&py)[PPL], const double (&pz)[PPL])
+{
+    PointBox b;
+    const double *c[3] = {px, py, pz};
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+    {
+        double lo = c[k][0], hi = c[k][0];
+#pragma unroll
+        for (int i = 1; i < PPL; ++i)
+            lo = fmin(lo, c[k][i]), hi = fmax(hi, c[k][i]);
+        for (int off = 32; off > 0; off >>= 1)
+        {
+            lo = fmin(lo, __shfl_xor(lo, off));
+            hi = fmax(hi, __shfl_xor(hi, off));
+        }
+        b.lo[k] = wave_uniform(lo), b.hi[k] = wave_uniform(hi);
+    }
+    return b;
+}
+// True when every point of the box is at least s.reach from the lines' box: the far form then
+// holds for every pair (SegBox::reach).  False for anything that is not a number.
+__device__ __forceinline__ bool box_far(const PointBox &b, const SegBox &s)
+{
+    double d2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+    {
+        const double g = fmax(fmax(s.lo[k] - b.hi[k], b.lo[k] - s.hi[k]), 0.0);
+        d2 = fma(g, g, d2);
+    }
+    return __builtin_amdgcn_ballot_w64(d2 >= s.reach * s.reach) != 0;
+}
+
+// v += w K of a segment in the far form (induction_core.hpp) for a lane's PPL points, a = p - r1
+// before and p - r2 after; step by step over the points, whose chains of dependent operations
+// then fill each other's latency.
+template <int PPL>
+__device__ __forceinline__ void far_add(const SegRec &r, const double (&px)[PPL], const double (&py)[PPL],
+                                        const double (&pz)[PPL], double (&ax)[PPL], double (&ay)[PPL],
+                                        double (&az)[PPL], double tol2, double (&vx)[PPL], double (&vy)[PPL],
+                                        double (&vz)[PPL])
+{
+    double bx[PPL], by[PPL], bz[PPL], q[PPL], cx[PPL], cy[PPL], cz[PPL], h2[PPL], u[PPL], f[PPL];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i)
+    {
+        bx[i] = px[i] - r.nx, by[i] = py[i] - r.ny, bz[i] = pz[i] - r.nz;
+        q[i] = fma(ax[i], bx[i], fma(ay[i], by[i], az[i] * bz[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < PPL; ++i)
+    {
+        cx[i] = fma(ay[i], r.ez, -(az[i] * r.ey));
+        cy[i] = fma(az[i], r.ex, -(ax[i] * r.ez));
+        cz[i] = fma(ax[i], r.ey, -(ay[i] * r.ex));
+        ax[i] = bx[i], ay[i] = by[i], az[i] = bz[i];
+    }
+#pragma unroll
+    for (int i = 0; i < PPL; ++i)
+    {
+        q[i] = far_rcp(q[i]);
+        h2[i] = fma(cx[i], cx[i], fma(cy[i], cy[i], cz[i] * cz[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < PPL; ++i)
+        u[i] = q[i] * (q[i] * h2[i]), f[i] = r.c[kFarTerms];
+#pragma unroll
+    for (int k = kFarTerms - 1; k >= 0; --k)
+#pragma unroll
+        for (int i = 0; i < PPL; ++i)
+            f[i] = fma(f[i], u[i], r.c[k]);
+#pragma unroll
+    for (int i = 0; i < PPL; ++i)
+    {
+        // the angle's sign: K = -(dr1 x e) angle / h
+        const double wm = h2[i] < tol2 ? 0.0 : -(q[i] * f[i]);
+        vx[i] = fma(wm, cx[i], vx[i]);
+        vy[i] = fma(wm, cy[i], vy[i]);
+        vz[i] = fma(wm, cz[i], vz[i]);
+    }
+}
+
+// Head of each piece: its active segments, start and bounds; one lane per segment.
+__global__ void __launch_bounds__(256) chain_head_kernel(unsigned n_pieces, const ChainPiece *__restrict__ pieces,
+                                                           unsigned cr, const double *__restrict__ nodes,
+                                                           const SegRec *__restrict__ segs, ChainHead *__restrict__ out,
+                                                           unsigned *__restrict__ queue)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *queue = 0u;
+    constexpr unsigned L = kChainPiece;
+    static_assert((L & (L - 1)) == 0 && L <= 64, "the pieces of a wave");
+    const unsigned k = blockIdx.x * (256 / L) + threadIdx.x / L, lane = threadIdx.x % L;
+    if (k >= n_pieces)
+        return;
+    const ChainPiece pc = pieces[k];
+    const unsigned n = active_segments(pc, cr);
+    ChainHead hd;
+    hd.first_seg = pc.first_seg, hd.n_seg = n;
+    SegBox &b = hd.box;
+    b.reach = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        hd.start[c] = b.lo[c] = b.hi[c] = nodes[3 * pc.start_node + c];
+    if (lane < n)
+    {
+        const SegRec &r = segs[pc.first_seg + lane];
+        const double e[3] = {r.nx, r.ny, r.nz};
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            b.lo[c] = fmin(b.lo[c], e[c]), b.hi[c] = fmax(b.hi[c], e[c]);
+        b.reach = far_reach(r.len);
+    }
+    for (int off = L / 2; off > 0; off >>= 1)
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            b.lo[c] = fmin(b.lo[c], __shfl_xor(b.lo[c], off, L));
+            b.hi[c] = fmax(b.hi[c], __shfl_xor(b.hi[c], off, L));
+        }
+        b.reach = fmax(b.reach, __shfl_xor(b.reach, off, L));
+    }
+    if (lane == 0)
+        out[k] = hd;
+}
+
+// Waits until the far form's part of a record is in scalar registers (SegRec::len is not part
+// of it), with nothing moved across.
+__device__ __forceinline__ void arrived(const SegRec &r)
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(r.nx), "s"(r.ny), "s"(r.nz), "s"(r.ex), "s"(r.ey), "s"(r.ez), "s"(r.c[0]), "s"(r.c[1]),
+                 "s"(r.c[2]), "s"(r.c[3]), "s"(r.c[4]), "s"(r.c[5]), "s"(r.c[6]), "s"(r.c[7]));
+}
+
+// A lane has PPL points, a wave 64 PPL, a workgroup four times that; the waves of a workgroup walk
+// the same pieces, a chunk of them (every n_chunks-th piece, so that the pieces near the points are
+// spread over the chunks) per item, so that a segment's record is read into the scalar
+// cache once for four waves (with a piece per wave the records' latency held the kernel at twice
+// its issue time).  Sums are written per chunk (no atomics, no exchange between waves).
+// Bound by VALU issue: 37 slots per pair in the far form (induction_core.hpp), 73 in the general
+// one.  A piece whose box is far enough from the box of the wave's points takes the far form for
+// all its segments without any test inside the loop (93 to 95 % of the pairs of a 400-row wake);
+// the end node's dr = p - r is the next segment's dr1.  Work items are (point block, piece chunk)
+// pairs, taken from a grid that may be smaller than their number (side stream).
+template <int PREC, int PPL>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+    chain_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, const ChainHead *__restrict__ heads,
+                          unsigned n_pieces, const SegRec *__restrict__ segs, const double *__restrict__ seg_gamma,
+                          unsigned n_chunks, double *__restrict__ partial, double tol, unsigned pblocks,
+                          unsigned n_items, unsigned *__restrict__ queue)
+{
     const unsigned w = wave_id(), lane = lane_id();
     const double tol2 = tol * tol;
-    for (unsigned item = blockIdx.x; item < n_items; item += gridDim.x)
+    __shared__ unsigned s_item;
+    for (;;)
     {
+        if (threadIdx.x == 0)
+            s_item = atomicAdd(queue, 1u);
+        __syncthreads();
+        const unsigned item = __builtin_amdgcn_readfirstlane(s_item);
+        __syncthreads(); // s_item is rewritten for the next item
+        if (item >= n_items)
+            return;
         const unsigned chunk = item / pblocks;
-        const unsigned p0 = (item - chunk * pblocks) * (kWave * PPL) + lane;
+        const unsigned w0 = ((item - chunk * pblocks) * 4 + w) * (kWave * PPL);
+        if (w0 >= n_pts)
+            continue;
+        const unsigned p0 = w0 + lane;
         double px[PPL], py[PPL], pz[PPL], vx[PPL], vy[PPL], vz[PPL];
 #pragma unroll
         for (int i = 0; i < PPL; ++i)
@@ -645,19 +831,14 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))
             px[i] = pts[3 * pc + 0], py[i] = pts[3 * pc + 1], pz[i] = pts[3 * pc + 2];
             vx[i] = 0.0, vy[i] = 0.0, vz[i] = 0.0;
         }
-        const unsigned k0 = chunk * pieces_per_chunk;
-        const unsigned k1 = (k0 + pieces_per_chunk) < n_pieces ? (k0 + pieces_per_chunk) : n_pieces;
-        for (unsigned k = k0 + w; k < k1; k += 4)
+        PointBox box;
+        if constexpr (PREC != PVL_FP64_REF_FORM)
+            box = point_box<PPL>(px, py, pz);
+        for (unsigned k = chunk; k < n_pieces; k += n_chunks)
         {
-            const ChainPiece pc = pieces[k];
-            unsigned n = pc.n_seg;
-            if (pc.row1)
-            {
-                const unsigned avail = cr - (pc.row1 - 1);
-                n = n < avail ? n : avail;
-            }
-            const double sx = nodes[3 * pc.start_node + 0], sy = nodes[3 * pc.start_node + 1],
-                         sz = nodes[3 * pc.start_node + 2];
+            const ChainHead &hd = heads[k];
+            const unsigned n = hd.n_seg;
+            const double sx = hd.start[0], sy = hd.start[1], sz = hd.start[2];
             double ax[PPL], ay[PPL], az[PPL], aq[PPL]; // aq (|p - node|^2) only for the reference form
 #pragma unroll
             for (int i = 0; i < PPL; ++i)
@@ -665,74 +846,88 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))
                 ax[i] = px[i] - sx, ay[i] = py[i] - sy, az[i] = pz[i] - sz;
                 aq[i] = PREC == PVL_FP64_REF_FORM ? ax[i] * ax[i] + ay[i] * ay[i] + az[i] * az[i] : 0.0;
             }
-            const SegRec *sg = segs + pc.first_seg;
-#pragma unroll 2
-            for (unsigned j = 0; j < n; ++j)
-            {
-                const SegRec r = sg[j];
+            const SegRec *sg = segs + hd.first_seg;
+            const double *gg = seg_gamma + hd.first_seg;
+            // one segment in the general form, and on to its end node
+            auto general = [&](unsigned j, const double *table) {
+                const double nx = sg[j].nx, ny = sg[j].ny, nz = sg[j].nz;
+                const double ex = sg[j].ex, ey = sg[j].ey, ez = sg[j].ez, len = sg[j].len, gamma = gg[j];
 #pragma unroll
                 for (int i = 0; i < PPL; ++i)
                 {
-                    const double bx = px[i] - r.nx, by = py[i] - r.ny, bz = pz[i] - r.nz;
                     bool cut;
                     if constexpr (PREC == PVL_FP64_REF_FORM)
                     {
+                        const double bx = px[i] - nx, by = py[i] - ny, bz = pz[i] - nz;
                         const double bq = bx * bx + by * by + bz * bz;
                         const double m =
-                            pair_m<PREC>(r.ex, r.ey, r.ez, r.len, ax[i], ay[i], az[i], aq[i], bx, by, bz, bq, tol, tol2, cut);
-                        const double kx = cut ? 0.0 : (ay[i] * r.ez - az[i] * r.ey) * m;
-                        const double ky = cut ? 0.0 : (az[i] * r.ex - ax[i] * r.ez) * m;
-                        const double kz = cut ? 0.0 : (ax[i] * r.ey - ay[i] * r.ex) * m;
-                        vx[i] = vx[i] + r.gamma * kx;
-                        vy[i] = vy[i] + r.gamma * ky;
-                        vz[i] = vz[i] + r.gamma * kz;
+                            pair_m<PREC>(ex, ey, ez, len, ax[i], ay[i], az[i], aq[i], bx, by, bz, bq, tol, tol2, cut);
+                        const double kx = cut ? 0.0 : (ay[i] * ez - az[i] * ey) * m;
+                        const double ky = cut ? 0.0 : (az[i] * ex - ax[i] * ez) * m;
+                        const double kz = cut ? 0.0 : (ax[i] * ey - ay[i] * ex) * m;
+                        vx[i] = vx[i] + gamma * kx;
+                        vy[i] = vy[i] + gamma * ky;
+                        vz[i] = vz[i] + gamma * kz;
                         aq[i] = bq;
+                        ax[i] = bx, ay[i] = by, az[i] = bz;
                     }
                     else
                     {
                         double cx, cy, cz;
                         const double m =
-                            cross_m<PREC>(r.ex, r.ey, r.ez, r.len, ax[i], ay[i], az[i], tol2, cx, cy, cz, cut);
-                        const double wm = cut ? 0.0 : r.gamma * m;
+                            cross_m<PREC, 2>(ex, ey, ez, len, ax[i], ay[i], az[i], tol2, cx, cy, cz, cut, table);
+                        const double wm = cut ? 0.0 : gamma * m;
                         vx[i] = fma(wm, cx, vx[i]);
                         vy[i] = fma(wm, cy, vy[i]);
                         vz[i] = fma(wm, cz, vz[i]);
+                        ax[i] = px[i] - nx, ay[i] = py[i] - ny, az[i] = pz[i] - nz;
+                        __builtin_amdgcn_sched_barrier(0); // one point after the other: fewer registers
                     }
-                    ax[i] = bx, ay[i] = by, az[i] = bz;
                 }
+            };
+            bool far = false;
+            if constexpr (PREC != PVL_FP64_REF_FORM)
+                far = box_far(box, hd.box);
+            if (far)
+            {
+                // the next segment's record is on its way to scalar registers while this one is
+                // worked on (scalar loads return out of order, so a wait is for all of them: the
+                // one for the next record stands at the end of this one's work)
+                auto work = [&](const SegRec &r) { far_add<PPL>(r, px, py, pz, ax, ay, az, tol2, vx, vy, vz); };
+                SegRec r = sg[0], q;
+                arrived(r);
+                unsigned j = 0;
+                for (; j + 1 < n; j += 2)
+                {
+                    q = sg[j + 1];
+                    __builtin_amdgcn_sched_barrier(0);
+                    work(r);
+                    arrived(q);
+                    r = sg[j + 2 < n ? j + 2 : j];
+                    __builtin_amdgcn_sched_barrier(0);
+                    work(q);
+                    arrived(r);
+                }
+                if (j < n)
+                    work(r);
+            }
+            else
+            {
+                const double *table = PREC == PVL_FP64 ? atan_table() : nullptr;
+                for (unsigned j = 0; j < n; ++j)
+                    general(j, table);
             }
         }
 #pragma unroll
         for (int i = 0; i < PPL; ++i)
         {
-            red[w][0][i * kWave + lane] = vx[i];
-            red[w][1][i * kWave + lane] = vy[i];
-            red[w][2][i * kWave + lane] = vz[i];
-        }
-        __syncthreads();
-        if (w == 0)
-        {
-#pragma unroll
-            for (int i = 0; i < PPL; ++i)
+            const unsigned p = p0 + i * kWave;
+            if (p < n_pts)
             {
-                const unsigned p = p0 + i * kWave;
-                if (p >= n_pts)
-                    continue;
-                const unsigned q = i * kWave + lane;
-                double sx2 = red[0][0][q], sy2 = red[0][1][q], sz2 = red[0][2][q];
-                for (int u = 1; u < 4; ++u)
-                {
-                    sx2 = sx2 + red[u][0][q];
-                    sy2 = sy2 + red[u][1][q];
-                    sz2 = sz2 + red[u][2][q];
-                }
                 double *dst = partial + ((size_t)chunk * n_pts + p) * 3;
-                dst[0] = sx2;
-                dst[1] = sy2;
-                dst[2] = sz2;
+                dst[0] = vx[i], dst[1] = vy[i], dst[2] = vz[i];
             }
         }
-        __syncthreads(); // red is rewritten by the next item
     }
 }
 
@@ -816,47 +1011,47 @@ int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, 
 }
 
 int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_line, const double *nodes,
-                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, hipStream_t s)
+                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, double *seg_gamma,
+                   hipStream_t s)
 {
     if (n_seg == 0)
         return PVL_OK;
     chain_segment_kernel<<<(n_seg + 255) / 256, 256, 0, s>>>(n_seg, seg_ab, seg_line, nodes, gamma, n_active_lines,
-                                                             tol, out);
+                                                             tol, out, seg_gamma);
     PVL_HIP(hipGetLastError());
     return PVL_OK;
 }
 
 constexpr int kChainPPL = 2;
+constexpr unsigned kChainPoints = 4 * kWave * kChainPPL; // per workgroup
+constexpr unsigned kChainItems = 4608;
 
 unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces)
 {
-    // aim at >= ~2048 work items while keeping >= 8 pieces (>= 2 per wave) per chunk
-    const unsigned ppg = kWave * kChainPPL;
-    const unsigned pblocks = (n_pts + ppg - 1) / ppg;
-    unsigned n_chunks = (2048 + pblocks - 1) / pblocks;
-    const unsigned max_chunks = (n_pieces + 7) / 8;
-    if (n_chunks > max_chunks)
-        n_chunks = max_chunks;
-    if (n_chunks < 1)
-        n_chunks = 1;
-    const unsigned ppc = (n_pieces + n_chunks - 1) / n_chunks;
-    return ppc ? (n_pieces + ppc - 1) / ppc : 1;
+    // kChainItems work items (six per workgroup of the side stream: the last ones claimed are
+    // the kernel's tail), a chunk of at least 8 pieces each.  More items cost more partial sums
+    // (24 bytes per point and chunk, written and read once).
+    const unsigned pblocks = (n_pts + kChainPoints - 1) / kChainPoints;
+    const unsigned max_chunks = std::max(1u, (n_pieces + 7) / 8);
+    return std::min(max_chunks, std::max(1u, kChainItems / pblocks));
 }
 
 int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nodes, const ChainPiece *pieces,
-                            unsigned n_pieces, unsigned cr, const SegRec *segs, int precision, double tol,
-                            double work, hipStream_t s, double *partial, unsigned max_groups)
+                            unsigned n_pieces, unsigned cr, const SegRec *segs, const double *seg_gamma,
+                            ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial,
+                            unsigned max_groups)
 {
     const unsigned n_chunks = chain_velocity_chunks(n_pts, n_pieces);
-    const unsigned ppc = (n_pieces + n_chunks - 1) / n_chunks;
-    const unsigned ppg = kWave * kChainPPL;
-    const unsigned pblocks = (n_pts + ppg - 1) / ppg;
+    const unsigned pblocks = (n_pts + kChainPoints - 1) / kChainPoints;
     const unsigned n_items = pblocks * n_chunks;
     const unsigned grid = max_groups && max_groups < n_items ? max_groups : n_items;
+    unsigned *queue = (unsigned *)(heads + n_pieces); // one spare head
+    chain_head_kernel<<<(n_pieces * kChainPiece + 255) / 256, 256, 0, s>>>(n_pieces, pieces, cr, nodes, segs, heads, queue);
+    PVL_HIP(hipGetLastError());
     ProfScope prof("wake_self_velocity", work, s);
     dispatch_precision(precision, [&](auto P) {
         chain_velocity_kernel<decltype(P)::value, kChainPPL><<<grid, kBlock, 0, s>>>(
-            n_pts, pts, nodes, pieces, n_pieces, cr, segs, ppc, partial, tol, pblocks, n_items);
+            n_pts, pts, heads, n_pieces, segs, seg_gamma, n_chunks, partial, tol, pblocks, n_items, queue);
     });
     PVL_HIP(hipGetLastError());
     return PVL_OK;

@@ -93,6 +93,31 @@ template <bool SGPR_COEF = false> __device__ __forceinline__ double atan_poly64(
     return fma(a * s, p, a);
 }
 
+// The same polynomial with its coefficients loaded (scalar loads): for a less often taken branch
+// beside a loop that needs the scalar registers itself.  atan_table() at the branch's start gives
+// an address that is opaque to the compiler, which would otherwise hoist the loads out of it.
+static __constant__ double kAtanTable[17] = {
+    -4.7926633120228785553e-5, 4.800660567800612957e-4,  -2.2725728333658927666e-3, 6.8183912427924839848e-3,
+    -1.4739706399322470277e-2, 2.4909137877934616446e-2, -3.5142229350564300719e-2, 4.3938991765738211806e-2,
+    -5.1356486201903778769e-2, 5.8483233451193392607e-2, -6.6598275562737410628e-2, 7.6913027337110721971e-2,
+    -9.090805442522420044e-2,  1.1111104041852547122e-1, -1.4285713995249626285e-1, 1.9999999993898812193e-1,
+    -3.3333333333288106455e-1};
+__device__ __forceinline__ const double *atan_table()
+{
+    const double *t = kAtanTable;
+    asm volatile("" : "+s"(t));
+    return t;
+}
+__device__ __forceinline__ double atan_poly64_table(double a, const double *t)
+{
+    const double s = a * a;
+    double p = t[0];
+#pragma unroll
+    for (int k = 1; k < 17; ++k)
+        p = fma(p, s, t[k]);
+    return fma(a * s, p, a);
+}
+
 __device__ __forceinline__ float atan_poly32(float a)
 {
     const float s = a * a;
@@ -127,14 +152,19 @@ __device__ __forceinline__ double pvl_atan2(double y, double x)
 
 // atan2(-ay, x) for ay >= 0 (the segment's angle below: its sine is never positive), as
 // pvl_atan2 without the sign transfer.
-template <bool SGPR_COEF = false> __device__ __forceinline__ double pvl_atan2_neg(double ay, double x)
+template <int COEF = 0>
+__device__ __forceinline__ double pvl_atan2_neg(double ay, double x, const double *table = nullptr)
 {
     const double ax = fabs(x);
     const double mn = fmin(ax, ay), mx = fmax(ax, ay);
     double r = __builtin_amdgcn_rcp(mx);
     r = fma(r, fma(-mx, r, 1.0), r);
     const double a = mn * r;
-    double t = atan_poly64<SGPR_COEF>(a);
+    double t;
+    if constexpr (COEF == 2)
+        t = atan_poly64_table(a, table);
+    else
+        t = atan_poly64<COEF == 1>(a);
     t = (ay > ax) ? (1.57079632679489661923 - t) : t;
     t = (x < 0.0) ? (3.14159265358979323846 - t) : t;
     return -t;
@@ -166,7 +196,7 @@ __device__ __forceinline__ double pvl_rsqrt(double x)
 // q2 likewise (each dot product left to right, no FMA, as the reference), e = the unit
 // direction.  The cut-off is decided here.  Split from line_m so that a walk along a chain of
 // segments can reuse one endpoint's terms for the next segment (bit-identical values).
-template <int PREC, bool SGPR_COEF = false>
+template <int PREC, int COEF = 0>
 __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double len, double d1x, double d1y,
                                          double d1z, double q1, double d2x, double d2y, double d2z, double q2,
                                          double tol, double tol2, bool &cut)
@@ -198,7 +228,7 @@ __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double
         {
             const double ih = pvl_rsqrt(h2);
             const double h = h2 * ih;
-            const double dphi = pvl_atan2_neg<SGPR_COEF>(len * h, fma(t1, t2, h2));
+            const double dphi = pvl_atan2_neg<COEF>(len * h, fma(t1, t2, h2));
             m = dphi * ih;
         }
         else
@@ -225,9 +255,10 @@ __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double
 // shorter than tol has direction 0 and length 0 (chain records), so c = 0, h^2 = 0 and it is
 // cut, as the reference's length test cuts it.  A cut pair's m may be NaN or Inf; the caller
 // replaces the pair's value by 0.
-template <int PREC>
+template <int PREC, int COEF = 0>
 __device__ __forceinline__ double cross_m(double ex, double ey, double ez, double len, double d1x, double d1y,
-                                          double d1z, double tol2, double &cx, double &cy, double &cz, bool &cut)
+                                          double d1z, double tol2, double &cx, double &cy, double &cz, bool &cut,
+                                          const double *table = nullptr)
 {
     cx = fma(d1y, ez, -(d1z * ey));
     cy = fma(d1z, ex, -(d1x * ez));
@@ -240,7 +271,7 @@ __device__ __forceinline__ double cross_m(double ex, double ey, double ez, doubl
     {
         const double ih = pvl_rsqrt(h2);
         const double h = h2 * ih;
-        return pvl_atan2_neg(len * h, fma(t1, t2, h2)) * ih;
+        return pvl_atan2_neg<COEF>(len * h, fma(t1, t2, h2), table) * ih;
     }
     else
     {
@@ -252,8 +283,35 @@ __device__ __forceinline__ double cross_m(double ex, double ey, double ez, doubl
     }
 }
 
+// Far form of angle / h, for pairs whose point is further than about four segment lengths from
+// the segment's midpoint: with A = len h and B = dr1 . dr2 = h^2 + t1 t2 the angle is
+// atan(A / B), and angle / h = (len / B) (1 + s P(s)), s = (len / B)^2 h^2 -- a function of
+// h^2 alone, so neither the square root nor the octant logic of atan2 is needed, and a short
+// P suffices.  B = |m|^2 - len^2 / 4 for the distance m from the midpoint, so |m| >= 4 len makes
+// B positive and gives s <= 0.0645, over which the degree-6 P below has a relative error of
+// 4.6e-16 (tools/fit_atan.py 6 double 0.0645; the general form's polynomial: 1.1e-15).  1/B is
+// the hardware reciprocal and one Newton step, as in pvl_atan2.  Callers decide by the boxes of
+// a wave's points and of a group of lines, so the evaluation itself carries no test.
+constexpr int kFarTerms = 7;
+constexpr double kFar1 = -3.3333333333275589419e-1, kFar2 = 1.9999999977026864496e-1,
+                 kFar3 = -1.4285711189790686119e-1, kFar4 = 1.1110912812573140192e-1,
+                 kFar5 = -9.0840857012789507027e-2, kFar6 = 7.5620986412452229467e-2,
+                 kFar7 = -5.3494538871327659169e-2;
+// Distance of a point from a line of length len from which on the far form holds (4 len from the
+// midpoint, and a margin for the rounding of the boxes).  Lines cut by length (len 0) and lengths
+// whose 15th powers could leave the range of a double take the general form for every point.
+__device__ __forceinline__ double far_reach(double len)
+{
+    return (len >= 1e-12 && len <= 1e12) ? 4.000001 * len : __builtin_inf();
+}
+__device__ __forceinline__ double far_rcp(double b)
+{
+    const double r = __builtin_amdgcn_rcp(b);
+    return fma(r, fma(-b, r, 1.0), r);
+}
+
 // Scalar factor of K (angle / h; the cut-off is decided here) and dr1 = p - r1.
-template <int PREC, bool SGPR_COEF = false>
+template <int PREC, int COEF = 0>
 __device__ __forceinline__ double line_m(const LineGeom &g, double px, double py, double pz, double tol, double tol2,
                                          double &d1x, double &d1y, double &d1z, bool &cut)
 {
@@ -261,7 +319,7 @@ __device__ __forceinline__ double line_m(const LineGeom &g, double px, double py
     const double d2x = px - g.r2x, d2y = py - g.r2y, d2z = pz - g.r2z;
     const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
     const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
-    return pair_m<PREC, SGPR_COEF>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2, tol, tol2, cut);
+    return pair_m<PREC, COEF>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2, tol, tol2, cut);
 }
 
 // K(line, p).  The reference form keeps the reference's cross product and products; the
@@ -311,7 +369,7 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     {
         double d1x, d1y, d1z;
         bool cut;
-        const double m = line_m<PREC, true>(g, px, py, pz, tol, tol2, d1x, d1y, d1z, cut);
+        const double m = line_m<PREC, 1>(g, px, py, pz, tol, tol2, d1x, d1y, d1z, cut);
         const double cx = fma(d1y, g.ez, -(d1z * g.ey));
         const double cy = fma(d1z, g.ex, -(d1x * g.ez));
         const double cz = fma(d1x, g.ey, -(d1y * g.ex));

@@ -122,32 +122,52 @@ int point_velocity_reduce(unsigned n_pts, unsigned n_chunks, const double *parti
 // piece with row1 > 0 runs streamwise from node row row1 - 1 and only its first cr - (row1 - 1)
 // segments are active at cr filled rows.  Walking a piece, each node's p - r (and, in the
 // reference form, |p - r|^2) is formed once and serves both segments that meet there.
-constexpr unsigned kChainPiece = 32;
+constexpr unsigned kChainPiece = 16;
 struct ChainPiece
 {
     uint32_t start_node, first_seg, n_seg, row1;
 };
 // Per-step segment record: end node, unit direction and length (the reference's line
-// prologue, src/core/flow_solver.c:95-103, in the chain's direction) and circulation.
-struct alignas(16) SegRec
+// prologue, src/core/flow_solver.c:95-103, in the chain's direction), and the far form's
+// coefficients with the segment's length and circulation multiplied in
+// (induction_core.hpp): w = r (c[0] + u (c[1] + ...)), r = 1/B, u = r^2 h^2.
+struct alignas(128) SegRec
 {
     double nx, ny, nz;
     double ex, ey, ez;
-    double len, gamma;
+    double len, pad;
+    double c[8];
 };
-static_assert(sizeof(SegRec) == 64, "SegRec layout");
+static_assert(sizeof(SegRec) == 128, "SegRec layout");
+// Bounds of a group of lines: the box of their end points, and the distance from which on the
+// far form holds for each of them (infinite when one of them has to take the general form).
+struct SegBox
+{
+    double lo[3], hi[3], reach;
+};
+// Per-step head of a piece: its active segments, its start node's position and its bounds.
+struct alignas(32) ChainHead
+{
+    uint32_t first_seg, n_seg;
+    double start[3];
+    SegBox box;
+};
+// Workgroups per CU of the self-induction on the side stream.
+constexpr int kChainSideGroups = 3;
 // Line circulations gamma_l = sum of +-Gamma over the surfaces holding line l, lines < n_active.
 int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, double *gamma, hipStream_t s);
-// SegRec of n_seg segments (seg_ab: node pairs; seg_line: mesh line | bit 31 when the chain runs
-// against the line's direction); lines >= n_active_lines carry no circulation.
+// SegRec and circulation (seg_gamma) of n_seg segments (seg_ab: node pairs; seg_line: mesh line |
+// bit 31 when the chain runs against the line's direction); lines >= n_active_lines carry no
+// circulation.
 int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_line, const double *nodes,
-                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, hipStream_t s);
+                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, double *seg_gamma,
+                   hipStream_t s);
 unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces);
 // Partial sums per piece chunk (3 n_pts doubles each, in chunk order; point_velocity_reduce adds
 // them); work = pairs evaluated, for the profiler.
 int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nodes, const ChainPiece *pieces,
-                            unsigned n_pieces, unsigned cr, const SegRec *segs, int precision, double tol,
-                            double work, hipStream_t s, double *partial, unsigned max_groups);
+                            unsigned n_pieces, unsigned cr, const SegRec *segs, const double *seg_gamma,
+                            ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial, unsigned max_groups);
 
 // Single-workgroup LU panel (lu_panel_f64.hip / lu_panel_f32.hip): factors the m x jb panel
 // at P (row stride lda; matrix rows row_base..) with partial pivoting, piv[row_base + j]

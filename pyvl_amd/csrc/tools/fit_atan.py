@@ -3,7 +3,8 @@
 atan(a) ~= a + a * s * P(s), s = a^2, 0 <= a <= 1, minimising the maximum relative error
 of atan (Lawson's iteratively reweighted least squares on Chebyshev nodes, in 60-digit
 arithmetic), then checks the double/float Horner evaluation against mpmath.  Prints the
-coefficients as C literals.  Usage: python fit_atan.py DEGREE_P [float]
+coefficients as C literals.  With SMAX < 1 the fit covers s = a^2 <= SMAX only (the far form
+of the induction kernels).  Usage: python fit_atan.py DEGREE_P [float|double [SMAX]]
 """
 import sys
 
@@ -13,8 +14,8 @@ import numpy as np
 mp.mp.dps = 60
 
 
-def fit(deg, n_nodes=400, iters=60):
-    nodes = [(1 - mp.cos(mp.pi * (k + mp.mpf(0.5)) / n_nodes)) / 2 for k in range(n_nodes)]  # s in (0,1)
+def fit(deg, smax=1, n_nodes=400, iters=60):
+    nodes = [smax * (1 - mp.cos(mp.pi * (k + mp.mpf(0.5)) / n_nodes)) / 2 for k in range(n_nodes)]  # s in (0, smax)
     g = []
     w_rel = []
     for s in nodes:
@@ -46,10 +47,10 @@ def fit(deg, n_nodes=400, iters=60):
     return [coef[j] for j in range(deg + 1)], max(err)
 
 
-def check(coef, dtype):
+def check(coef, dtype, smax=1):
     rng = np.random.default_rng(0)
     a = np.concatenate([np.linspace(0, 1, 200001), rng.uniform(0, 1, 200000), 10.0 ** -rng.uniform(0, 12, 20000)])
-    a = a.astype(dtype)
+    a = (a * np.sqrt(float(smax))).astype(dtype)
     c = [dtype(float(x)) for x in coef]
     s = a * a
     p = np.full_like(a, c[-1])
@@ -67,8 +68,9 @@ def check(coef, dtype):
 if __name__ == "__main__":
     deg = int(sys.argv[1])
     dtype = np.float32 if len(sys.argv) > 2 and sys.argv[2] == "float" else np.float64
-    coef, err = fit(deg)
+    smax = mp.mpf(sys.argv[3]) if len(sys.argv) > 3 else 1
+    coef, err = fit(deg, smax)
     print(f"// degree {deg}: minimax relative error of the polynomial {float(err):.3e}, "
-          f"{dtype.__name__} Horner {check(coef, dtype):.3e}")
+          f"{dtype.__name__} Horner {check(coef, dtype, smax):.3e}")
     for x in coef:
         print(f"    {mp.nstr(x, 20, min_fixed=-1, max_fixed=-1)},")

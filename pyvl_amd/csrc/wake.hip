@@ -66,6 +66,8 @@ struct pvl_wake
     ChainPiece *d_pieces = nullptr;
     std::vector<uint32_t> pieces_at; // [R+1] pieces active with r ring rows filled
     SegRec *d_segrec = nullptr;      // [n_seg] per-step records
+    double *d_seggamma = nullptr;    // [n_seg] their circulations
+    ChainHead *d_heads = nullptr;    // [pieces] per-step heads
     bool pending = false;
     int pending_prec = 0;
     unsigned pending_na = 0, pending_npts = 0, pending_chunks = 0;
@@ -359,6 +361,8 @@ int build_chains(pvl_wake *w, const std::vector<uint32_t> &lines)
     PVL_HIP(hipMalloc((void **)&w->d_seg_line, sizeof(uint32_t) * sl.size()));
     PVL_HIP(hipMalloc((void **)&w->d_pieces, sizeof(ChainPiece) * pieces.size()));
     PVL_HIP(hipMalloc((void **)&w->d_segrec, sizeof(SegRec) * sl.size()));
+    PVL_HIP(hipMalloc((void **)&w->d_seggamma, sizeof(double) * sl.size()));
+    PVL_HIP(hipMalloc((void **)&w->d_heads, sizeof(ChainHead) * (pieces.size() + 1)));
     PVL_HIP(hipMemcpy(w->d_seg_ab, ab.data(), sizeof(uint32_t) * ab.size(), hipMemcpyHostToDevice));
     PVL_HIP(hipMemcpy(w->d_seg_line, sl.data(), sizeof(uint32_t) * sl.size(), hipMemcpyHostToDevice));
     PVL_HIP(hipMemcpy(w->d_pieces, pieces.data(), sizeof(ChainPiece) * pieces.size(), hipMemcpyHostToDevice));
@@ -477,6 +481,8 @@ int pvl_wake_destroy(pvl_wake *w)
     (void)hipFree(w->d_seg_line);
     (void)hipFree(w->d_pieces);
     (void)hipFree(w->d_segrec);
+    (void)hipFree(w->d_seggamma);
+    (void)hipFree(w->d_heads);
     pvl_mesh_destroy(w->full);
     pvl_mesh_destroy(w->row0);
     (void)hipFree(w->d_te_nodes);
@@ -559,10 +565,10 @@ static int self_partials(pvl_wake *w, unsigned n_pts, const double *pts, int pre
     if (int st = line_circulations(w->full, na, w->d_circ[w->cur], w->d_sgamma, s))
         return st;
     if (int st = chain_segments(w->n_seg, w->d_seg_ab, w->d_seg_line, w->d_upos, w->d_sgamma, na, w->tol, w->d_segrec,
-                                s))
+                                w->d_seggamma, s))
         return st;
-    return chain_velocity_partials(n_pts, pts, w->d_upos, w->d_pieces, w->pieces_at[ar], ar, w->d_segrec, precision,
-                                   w->tol, (double)n_pts * (double)na, s, w->d_spartial, max_groups);
+    return chain_velocity_partials(n_pts, pts, w->d_upos, w->d_pieces, w->pieces_at[ar], ar, w->d_segrec,
+                                   w->d_seggamma, w->d_heads, precision, w->tol, (double)n_pts * (double)na, s, w->d_spartial, max_groups);
 }
 
 // Orders the library stream after a started self-induction (its inputs may be overwritten
@@ -611,7 +617,7 @@ int pvl_wake_begin_update(pvl_wake *w, int mode, int precision)
     // wake nodes (pvl_wake_update evaluates at a copy of the same values)
     PVL_HIP(hipEventRecord(w->ev_ready, stream()));
     PVL_HIP(hipStreamWaitEvent(s, w->ev_ready, 0));
-    if (int st = self_partials(w, n_old, w->d_upos, precision, s, (unsigned)side_groups(5)))
+    if (int st = self_partials(w, n_old, w->d_upos, precision, s, (unsigned)side_groups(kChainSideGroups)))
         return st;
     PVL_HIP(hipEventRecord(w->ev_done, s));
     w->pending = true;
