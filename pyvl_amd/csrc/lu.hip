@@ -603,219 +603,340 @@ template <int P> __device__ __forceinline__ float quad_bcast(float v)
 }
 
 // Panel step WITHOUT interchanges (pivoting modes "none" and "auto"), fused: the LU of the
-// 64 x 64 diagonal block, L21 = A21 U11^-1 and U12 = L11^-1 A12 in one launch.  A workgroup
-// has 6 waves, each holding 16 rows or columns with 4 lanes per row / column (lane p of a quad
-// holds entries 4k + p, k = 0..15, in registers):
-//   waves 0-3  its own copy of the diagonal block (wave w: rows 16w .. 16w + 15),
-//   wave 4     panel rows jb + 16g .. jb + 16g + 15 below the diagonal block (L21),
-//   wave 5     columns jb + 16g .. jb + 16g + 15 of the panel's row block right of it (U12).
-// Step j: the quad owning diagonal row j has published it and 1/u_jj in LDS (as soon as step
-// j - 1 finalised it); after one barrier every later diagonal row and every row below forms
-// its multiplier (owner lane of column j), broadcasts it over the quad (DPP) and subtracts it
-// times row j, and the diagonal rows publish their multipliers l_ij, which the U12 columns
-// apply one step later (x_i -= l_i,j-1 x_j-1).  The diagonal waves carry the step-to-step
-// chain and run at the highest priority; the other two waves fill in behind them.  Per element the
-// operations and their order are those of the right-looking column sweep (dgetf2 without
-// interchanges, dtrsm).  The copies of the diagonal block agree (same arithmetic
-// everywhere).  Every workgroup reads A11 at its start, so L11 \ U11 is stored by the LAST
-// workgroup to finish (status[4] counts finished workgroups and is reset to 0 by that
-// workgroup; no workgroup waits for another); workgroup 0 stores the identity interchanges.
-// Only the last panel can be narrower than 64 (jb < 64 implies m == jb: no rows below, no
-// columns right): it is padded with identity rows and columns.
-// status[2]: smallest zero-pivot column (atomicMin); status[3] |= 1 when partial pivoting
-// would interchange: a sub-diagonal |a| above |pivot| at its column's elimination, or a zero
-// or NaN pivot.
-constexpr int kNopivRows = 16;   // rows below (and columns right) per workgroup
-constexpr int kNopivThreads = 384;
-
-// Registers and LDS rings of panel_nopiv_kernel (one instance per lane).
-template <typename T> struct NopivLane
+// 64 x 64 diagonal block, L21 = A21 U11^-1 and U12 = L11^-1 A12 in one launch.  A workgroup has 8
+// waves and its own copy of the diagonal block in LDS:
+//   waves 0-3  the diagonal block in slabs of 16 columns, wave w owning slab w,
+//   waves 4, 5 16 panel rows each below the diagonal block (L21),
+//   waves 6, 7 16 columns each of the panel's row block right of it (U12).
+// Stage s (one barrier each): waves w >= s bring their slab up to date with slab s - 1 (the
+// slab's 16 rows of U by substitution, the rows below on MFMA), then wave s factors slab s with
+// one row per lane and the slab's columns in registers, the pivot row broadcast with readlane; the
+// row and column waves follow one slab behind, each slab of theirs updated on MFMA with the ones
+// before it and finished by substitution (a quad of lanes per row or column).
+// Bound by the dependent chain of the 64 columns; a column costs ~270 cycles (readlanes, updates,
+// the reciprocal's chain) and a slab ~1,600 cycles of update ahead of its factorisation.  With
+// a barrier and an LDS round trip of the pivot row per column (~1,200 cycles) the step took 37 us.
+// The copies of the diagonal block agree (same arithmetic everywhere).  Every workgroup reads A11
+// at its start, so L11 \ U11 is stored by the LAST workgroup to finish (status[4] counts finished
+// workgroups and is reset to 0 by that workgroup; no workgroup waits for another); workgroup 0
+// stores the identity interchanges.  Only the last panel can be narrower than 64 (jb < 64 implies
+// m == jb: no rows below, no columns right): it is padded with identity rows and columns.
+// status[2]: smallest zero-pivot column (atomicMin); status[3] |= 1 when partial pivoting would
+// interchange: a sub-diagonal |a| above |pivot| at its column's elimination, or a zero or NaN
+// pivot.
+constexpr int kNopivRows = 32; // rows below (and columns right) per workgroup
+constexpr int kNopivThreads = 512;
+constexpr int kSlab = 16;
+constexpr int kNopivLd = NB + 1;    // row stride of the diagonal block and of the row strips
+constexpr int kNopivLdY = kSlab + 1; // row stride of the column strips
+constexpr size_t nopiv_lds_elems()
 {
-    static constexpr int KQ = NB / 4;
-    T v[KQ];       // diagonal row, row below, or column right (by role)
-    T (*Urow)[NB]; // row j of U11, column 4k + p at p * KQ + k
-    T (*Lcol)[NB]; // column j of L11, row 4k + p at p * KQ + k
-    T *Uinv;
-    int role;      // 0 diagonal block, 1 row below, 2 column right
-    int p, rd, jb, row_base, first_zero;
-    bool live, due;
-};
-
-// Publish diagonal row J (final once step J - 1 is done) and 1/u_JJ into ring slot J & 1.
-template <int J, typename T> __device__ __forceinline__ void nopiv_publish(NopivLane<T> &L)
-{
-    constexpr int KQ = NopivLane<T>::KQ;
-    constexpr int kj = J >> 2, pj = J & 3, s = J & 1;
-    if (L.rd == J)
-    {
-#pragma unroll
-        for (int k = 0; k < KQ; ++k)
-            L.Urow[s][L.p * KQ + k] = L.v[k];
-        if (L.p == pj)
-            L.Uinv[s] = T(1) / L.v[kj];
-    }
+    return (size_t)NB * kNopivLd + 2 * (kSlab * kNopivLd) + 2 * (NB * kNopivLdY) + NB;
 }
 
-// Step J of panel_nopiv_kernel (J a compile-time constant: every register index is static).
-template <int J, typename T> __device__ __forceinline__ void nopiv_step(NopivLane<T> &L)
+// 1/x to half an ulp and a little: the hardware estimate (2^-24 in FP64), one third-order step,
+// and the specials (0, infinities, NaN) as a division gives them.
+__device__ __forceinline__ double fast_recip(double x)
 {
-    constexpr int KQ = NopivLane<T>::KQ;
-    constexpr int kj = J >> 2, pj = J & 3, s = J & 1;
-    const int p = L.p;
-    __syncthreads();
-    if (L.role != 2)
-    {
-        const T ujj = L.Urow[s][pj * KQ + kj];
-        const T inv = L.Uinv[s];
-        const double pa = fabs((double)ujj);
-        T u[KQ];
-#pragma unroll
-        for (int k = kj; k < KQ; ++k)
-            u[k] = L.Urow[s][p * KQ + k];
-        if (L.role == 0)
-        {
-            if (J < L.jb && ujj == T(0) && L.first_zero == 0)
-                L.first_zero = L.row_base + J + 1;
-            if (L.rd > J)
-            {
-                const T own = L.v[kj];
-                T l = own * inv;
-                if (p == pj)
-                {
-                    L.due |= J < L.jb && (!(fabs((double)own) <= pa) || !(pa > 0.0));
-                    L.v[kj] = l;
-                    L.Lcol[s][(L.rd & 3) * KQ + (L.rd >> 2)] = l;
-                }
-                l = quad_bcast<pj>(l);
-#pragma unroll
-                for (int k = kj; k < KQ; ++k)
-                {
-                    const T v = fma(-l, u[k], L.v[k]);
-                    L.v[k] = (k > kj || p > pj) ? v : L.v[k];
-                }
-            }
-            if constexpr (J + 1 < NB)
-                nopiv_publish<J + 1>(L);
-        }
-        else
-        {
-            const T own = L.v[kj];
-            T l = own * inv;
-            if (p == pj)
-            {
-                L.due |= L.live && (!(fabs((double)own) <= pa) || !(pa > 0.0));
-                L.v[kj] = l;
-            }
-            l = quad_bcast<pj>(l);
-#pragma unroll
-            for (int k = kj; k < KQ; ++k)
-            {
-                const T v = fma(-l, u[k], L.v[k]);
-                L.v[k] = (k > kj || p > pj) ? v : L.v[k];
-            }
-        }
-    }
-    else if constexpr (J >= 1)
-    {
-        // U12 columns: apply column J - 1 of L11 (published last step)
-        constexpr int t = J - 1, kt = t >> 2, pt = t & 3;
-        const T yt = quad_bcast<pt>(L.v[kt]);
-#pragma unroll
-        for (int k = kt; k < KQ; ++k)
-        {
-            const T v = fma(-L.Lcol[t & 1][p * KQ + k], yt, L.v[k]);
-            L.v[k] = (k > kt || p > pt) ? v : L.v[k];
-        }
-    }
-    // Keep this step's updates here: the rows below and U12 columns are otherwise only read
-    // by the final stores, and the compiler would sink their FMAs past the barriers.
-#pragma unroll
-    for (int k = 0; k < KQ; ++k)
-        asm volatile("" : "+v"(L.v[k]));
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return __builtin_amdgcn_div_fixup(fma(r, fma(e, e, e), r), x, 1.0);
+}
+__device__ __forceinline__ float fast_recip(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_amdgcn_div_fixupf(fmaf(r, fmaf(-x, r, 1.0f), r), x, 1.0f);
 }
 
-template <typename T, int... J> __device__ __forceinline__ void nopiv_steps(NopivLane<T> &L, std::integer_sequence<int, J...>)
+// Orders a wave's own LDS accesses across its lanes.
+__device__ __forceinline__ void wave_lds_fence()
 {
-    (nopiv_step<J>(L), ...);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// At most 96 VGPRs (5 waves per SIMD): two of its waves then fit on a SIMD beside four waves
-// of the side stream's point-velocity kernel.
+// C -= A B for one 16 x 16 tile in LDS, K = 16, on MFMA; strides lda, ldb, ldc.
 template <typename T>
-__global__ void __launch_bounds__(kNopivThreads) __attribute__((amdgpu_waves_per_eu(5))) panel_nopiv_kernel(T *__restrict__ P, int lda, int m, int jb,
-                                                                    int row_base, int *__restrict__ piv,
-                                                                    int *__restrict__ status)
+__device__ __forceinline__ void tile_update(T *C, int ldc, const T *A, int lda, const T *B, int ldb, int lane)
 {
-    constexpr int KQ = NB / 4;
-    __shared__ T Urow[2][NB];
-    __shared__ T Lcol[2][NB];
-    __shared__ T Uinv[2];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int g = blockIdx.x;
-    NopivLane<T> L;
-    L.Urow = Urow, L.Lcol = Lcol, L.Uinv = Uinv;
-    L.role = w < 4 ? 0 : w - 3;
-    L.p = lane & 3;
-    L.rd = L.role == 0 ? 16 * w + (lane >> 2) : -1; // diagonal-block row of this quad
-    L.jb = jb, L.row_base = row_base, L.first_zero = 0, L.due = false;
-    const int rc = jb + kNopivRows * g + (lane >> 2); // panel row below / column right
-    L.live = L.role != 0 && rc < m;                   // (m - jb rows below, m - jb columns right)
-    const int p = L.p, rd = L.rd;
-    if (L.role == 0)
+    using acc_t = typename Mfma<T>::acc_t;
+    const int lr = lane & 15, lk = lane >> 4;
+    acc_t c;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        c[v] = C[Mfma<T>::out_row(lk, v) * ldc + lr];
+#pragma unroll
+    for (int kk = 0; kk < kSlab; kk += 4)
+        c = Mfma<T>::mma(-A[lr * lda + kk + lk], B[(kk + lk) * ldb + lr], c);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        C[Mfma<T>::out_row(lk, v) * ldc + lr] = c[v];
+}
+
+template <typename T> __device__ __forceinline__ T quad_bcast_sel(T v, int p)
+{
+    switch (p)
+    {
+    case 0: return quad_bcast<0>(v);
+    case 1: return quad_bcast<1>(v);
+    case 2: return quad_bcast<2>(v);
+    default: return quad_bcast<3>(v);
+    }
+}
+
+// X = L^-1 X for a 16 x 16 tile X in LDS and the unit lower L (16 x 16, stride ldl): lane
+// 4 c + p holds rows p, p + 4, .. of column c (dtrsm's column sweep).
+template <typename T>
+__device__ __forceinline__ void tile_solve_lower(T *X, int ldx, const T *L, int ldl, int lane)
+{
+    const int c = lane >> 2, p = lane & 3;
+    T x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        x[q] = X[(4 * q + p) * ldx + c];
+#pragma unroll
+    for (int t = 0; t < kSlab - 1; ++t)
+    {
+        const int kt = t >> 2, pt = t & 3;
+        const T xt = quad_bcast_sel(x[kt], pt);
+#pragma unroll
+        for (int q = kt; q < 4; ++q)
+        {
+            const T v = fma(-L[(4 * q + p) * ldl + t], xt, x[q]);
+            x[q] = (q > kt || p > pt) ? v : x[q];
+        }
+        if (pt == 3)
+            __builtin_amdgcn_sched_barrier(0); // bounds how far ahead the LDS reads (registers) run
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        X[(4 * q + p) * ldx + c] = x[q];
+}
+
+// X = X U^-1 for a 16 x 16 tile X in LDS and the upper U (stride ldu, reciprocal diagonal inv):
+// lane 4 r + p holds columns p, p + 4, .. of row r.  Returns true when an entry exceeds its
+// column's pivot in magnitude (or the pivot is zero or NaN).
+template <typename T>
+__device__ __forceinline__ bool tile_solve_upper(T *X, int ldx, const T *U, int ldu, const T *inv, int lane)
+{
+    const int r = lane >> 2, p = lane & 3;
+    int due = 0;
+    T x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        x[q] = X[r * ldx + 4 * q + p];
+#pragma unroll
+    for (int t = 0; t < kSlab; ++t)
+    {
+        const int kt = t >> 2, pt = t & 3;
+        const double pa = fabs((double)U[t * ldu + t]);
+        const T own = x[kt];
+        T l = own * inv[t];
+        if (p == pt)
+        {
+            due |= (int)(!(fabs((double)own) <= pa) | !(pa > 0.0));
+            x[kt] = l;
+        }
+        asm volatile("" : "+v"(due));
+        l = quad_bcast_sel(l, pt);
+#pragma unroll
+        for (int q = kt; q < 4; ++q)
+        {
+            const T v = fma(-l, U[t * ldu + 4 * q + p], x[q]);
+            x[q] = (q > kt || p > pt) ? v : x[q];
+        }
+        if (pt == 3)
+            __builtin_amdgcn_sched_barrier(0); // bounds how far ahead the LDS reads (registers) run
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        X[r * ldx + 4 * q + p] = x[q];
+    return due != 0;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kNopivThreads) __attribute__((amdgpu_waves_per_eu(6)))
+    panel_nopiv_kernel(T *__restrict__ P, int lda, int m, int jb, int row_base, int *__restrict__ piv,
+                       int *__restrict__ status)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int LD = kNopivLd, LY = kNopivLdY;
+    T *S = (T *)smem_raw; // the diagonal block
+    T *inv = S + NB * LD + 2 * (kSlab * LD) + 2 * (NB * LY);
+    const int tid = threadIdx.x, lane = tid & 63, g = blockIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int strip = (w >> 1) & 1; // 0: rows below (waves 4, 5), 1: columns right (waves 6, 7)
+    T *X = S + NB * LD + (strip == 0 ? (w & 1) * (kSlab * LD) : 2 * (kSlab * LD) + (w & 1) * (NB * LY));
+    const int i0 = jb + kNopivRows * g + kSlab * (w & 1); // the strip's first row or column
+    const bool has_strip = w >= 4 && i0 < m;              // wave-uniform
+    int due = 0;
+    int first_zero = 0;
+    if (w < 4)
         main_stream_priority<3>();
     else
         main_stream_priority<2>();
-#pragma unroll
-    for (int k = 0; k < KQ; ++k)
+    // Loads are unconditional, from addresses clamped into the panel (no branch per element, all
+    // in flight together); identity padding of a narrow last panel, zeros past the strips' end.
+    // A strip's element i of this lane: row i0 + i, column lane below; row 4 i + lane / 16, column
+    // i0 + lane % 16 to the right.
+    const int srow = strip == 0 ? i0 : lane >> 4, scol = strip == 0 ? lane : i0 + (lane & 15);
+    const int rstep = strip == 0 ? 1 : 4, xstep = strip == 0 ? LD : 4 * LY;
+    const int x0 = strip == 0 ? lane : (lane >> 4) * LY + (lane & 15);
     {
-        const int c = 4 * k + p;
-        if (L.role == 0)
-            L.v[k] = (rd < jb && c < jb) ? P[(size_t)rd * lda + c] : (rd == c ? T(1) : T(0));
-        else if (L.role == 1)
-            L.v[k] = L.live ? P[(size_t)rc * lda + c] : T(0);
-        else
-            L.v[k] = L.live ? P[(size_t)c * lda + rc] : T(0);
-    }
-    nopiv_publish<0>(L);
-    nopiv_steps(L, std::make_integer_sequence<int, NB>{});
-    if (L.role != 0 && L.live)
-    {
+        constexpr int NV = NB * NB / kNopivThreads;
+        const int r0 = tid / NB, c = tid % NB;
+        T v[NV];
 #pragma unroll
-        for (int k = 0; k < KQ; ++k)
+        for (int i = 0; i < NV; ++i)
+            v[i] = P[(size_t)min(r0 + i * (kNopivThreads / NB), jb - 1) * lda + min(c, jb - 1)];
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
         {
-            const int c = 4 * k + p;
-            if (L.role == 1)
-                P[(size_t)rc * lda + c] = L.v[k];
-            else
-                P[(size_t)c * lda + rc] = L.v[k];
+            const int r = r0 + i * (kNopivThreads / NB);
+            S[r * LD + c] = (r < jb && c < jb) ? v[i] : (r == c ? T(1) : T(0));
         }
     }
-    if (g == 0 && L.role == 0)
+    if (has_strip)
     {
-        if (rd < jb && p == 0)
-            piv[row_base + rd] = row_base + rd;
-        if (threadIdx.x == 0 && L.first_zero)
-            atomicMin(&status[2], L.first_zero);
+        const T *src = P + (size_t)min(srow, m - 1) * lda + min(scol, m - 1);
+        // (rows past the matrix: the row strips' last rows only, read again from its last row)
+        T v[kSlab];
+#pragma unroll
+        for (int i = 0; i < kSlab; ++i)
+            v[i] = src[(size_t)(min(srow + rstep * i, m - 1) - min(srow, m - 1)) * lda];
+#pragma unroll
+        for (int i = 0; i < kSlab; ++i)
+            X[x0 + xstep * i] = (srow + rstep * i < m && scol < m) ? v[i] : T(0);
     }
-    if (__ballot(L.due) && lane == 0)
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s <= 4; ++s)
+    {
+        const int t0 = kSlab * (s - 1); // the slab finished in the stage before
+        // opaque per stage: LDS addresses are formed where they are used instead of all being
+        // kept in registers (and spilled) across the stages
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
+        if (w < 4)
+        {
+            if (s >= 1 && w >= s)
+            {
+                tile_solve_lower(S + t0 * LD + kSlab * w, LD, S + t0 * LD + t0, LD, lane);
+                wave_lds_fence();
+#pragma unroll 1
+                for (int i = s; i < 4; ++i)
+                    tile_update(S + kSlab * i * LD + kSlab * w, LD, S + kSlab * i * LD + t0, LD,
+                                S + t0 * LD + kSlab * w, LD, lane);
+                wave_lds_fence();
+            }
+            if (w == s)
+            {
+                const int c0 = kSlab * s, row = c0 + lane;
+                const bool ok = row < NB;
+                T v[kSlab];
+#pragma unroll
+                for (int c = 0; c < kSlab; ++c)
+                    v[c] = ok ? S[row * LD + c0 + c] : T(0);
+                T u = bcast_lane(v[0], 0), r = fast_recip(u);
+#pragma unroll
+                for (int j = 0; j < kSlab; ++j)
+                {
+                    const double pa = fabs((double)u);
+                    const bool below = lane > j;
+                    const T own = below ? v[j] : T(0);
+                    const T l = own * r;
+                    // (identity padding past jb: a pivot of 1 over zeros, never due)
+                    due |= (int)(below & ok & (!(fabs((double)own) <= pa) | !(pa > 0.0)));
+                    asm volatile("" : "+v"(due)); // now, or every column's operands stay in registers for it
+                    if (lane == j)
+                        inv[c0 + j] = r;
+                    if (j + 1 < kSlab)
+                    {
+                        // the next pivot and its reciprocal first, from its row's entries (the
+                        // same operations as in its own lane): the other columns' updates fill
+                        // that chain's latency
+                        const T ujk = bcast_lane(v[j + 1], j);
+                        u = fma(-(bcast_lane(v[j], j + 1) * r), ujk, bcast_lane(v[j + 1], j + 1));
+                        r = fast_recip(u);
+                        v[j + 1] = fma(-l, ujk, v[j + 1]);
+                    }
+#pragma unroll
+                    for (int k = j + 2; k < kSlab; ++k)
+                        v[k] = fma(-l, bcast_lane(v[k], j), v[k]);
+                    v[j] = below ? l : v[j];
+                    __builtin_amdgcn_sched_barrier(0); // or the broadcasts of several columns pile up in SGPRs
+                }
+                if (ok)
+                {
+#pragma unroll
+                    for (int c = 0; c < kSlab; ++c)
+                        S[row * LD + c0 + c] = v[c];
+                }
+                wave_lds_fence();
+                const unsigned long long z = __ballot(lane < kSlab && S[(c0 + lane % kSlab) * (LD + 1)] == T(0));
+                if (z && first_zero == 0)
+                    first_zero = row_base + c0 + (int)__builtin_ctzll(z) + 1;
+            }
+        }
+        else if (s >= 1 && has_strip)
+        {
+            if (strip == 0)
+            {
+#pragma unroll 1
+                for (int t = 0; t < s - 1; ++t)
+                {
+                    tile_update(X + t0, LD, X + kSlab * t, LD, S + kSlab * t * LD + t0, LD, lane);
+                    wave_lds_fence();
+                }
+                const bool d = tile_solve_upper(X + t0, LD, S + t0 * LD + t0, LD, inv + t0, lane);
+                due |= (int)(d && i0 + (lane >> 2) < m);
+            }
+            else
+            {
+#pragma unroll 1
+                for (int t = 0; t < s - 1; ++t)
+                {
+                    tile_update(X + t0 * LY, LY, S + t0 * LD + kSlab * t, LD, X + kSlab * t * LY, LY, lane);
+                    wave_lds_fence();
+                }
+                tile_solve_lower(X + t0 * LY, LY, S + t0 * LD + t0, LD, lane);
+            }
+            wave_lds_fence();
+        }
+        __syncthreads();
+    }
+    if (has_strip)
+    {
+#pragma unroll
+        for (int i = 0; i < kSlab; ++i)
+            if (srow + rstep * i < m && scol < m)
+                P[(size_t)(srow + rstep * i) * lda + scol] = X[x0 + xstep * i];
+    }
+    if (g == 0)
+    {
+        if (tid < jb)
+            piv[row_base + tid] = row_base + tid;
+        if (lane == 0 && first_zero)
+            atomicMin(&status[2], first_zero);
+    }
+    if (__ballot(due) && lane == 0)
         atomicOr(&status[3], 1);
     // This workgroup's read of A11 is complete (its values fed every step).  The workgroup
     // that finishes last stores L11 \ U11 over A11 and resets the counter.
     __shared__ int last;
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (tid == 0)
         last = atomicAdd(&status[4], 1) == (int)gridDim.x - 1;
     __syncthreads();
-    if (last && L.role == 0)
+    if (last)
     {
-#pragma unroll
-        for (int k = 0; k < KQ; ++k)
+        for (int idx = tid; idx < NB * NB; idx += kNopivThreads)
         {
-            const int c = 4 * k + p;
-            if (rd < jb && c < jb)
-                P[(size_t)rd * lda + c] = L.v[k];
+            const int r = idx / NB, c = idx % NB;
+            if (r < jb && c < jb)
+                P[(size_t)r * lda + c] = S[r * LD + c];
         }
-        if (threadIdx.x == 0)
+        if (tid == 0)
             atomicExch(&status[4], 0);
     }
 }
@@ -1966,6 +2087,8 @@ template <typename T> int factor_impl(int n, T *A, int *piv, int *info_out, bool
     {
         PVL_HIP(hipFuncSetAttribute((const void *)panel_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds));
+        PVL_HIP(hipFuncSetAttribute((const void *)panel_nopiv_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)(sizeof(T) * nopiv_lds_elems())));
         attr_set[sizeof(T) == 8] = true;
     }
     PanelX<T> *X = (PanelX<T> *)g_ws.panelx;
@@ -2029,8 +2152,8 @@ template <typename T> int factor_impl(int n, T *A, int *piv, int *info_out, bool
         {
             T *P = A + (size_t)k * n + k;
             ProfScope prof(sizeof(T) == 8 ? "lu_panel_f64" : "lu_panel_f32");
-            panel_nopiv_kernel<T><<<std::max(1, (m - jb + kNopivRows - 1) / kNopivRows), kNopivThreads, 0,
-                                     stream()>>>(P, n, m, jb, k, piv, status);
+            panel_nopiv_kernel<T><<<std::max(1, (m - jb + kNopivRows - 1) / kNopivRows), kNopivThreads,
+                                     sizeof(T) * nopiv_lds_elems(), stream()>>>(P, n, m, jb, k, piv, status);
             PVL_HIP(hipGetLastError());
         }
         else if (nbf == kPanelWgCols && m <= panel_wg_rows(sizeof(T)))
