@@ -17,9 +17,10 @@
 //                  update after each outer block of 256 columns, and the updates inside an
 //                  outer block with a side of 2048 or more, are plain GEMMs and go to rocBLAS
 //                  (dgemm / sgemm, no atomics), which runs m x m x 256 ~1.4x faster.
-// Solves: one workgroup for systems whose right-hand sides fit its LDS (trsv_wg_kernel),
-// else one launch per triangle with a workgroup per block row that waits on the flags of
-// the blocks before it (trsv_flow_kernel).
+// Solves: a single right-hand side one launch per triangle with a workgroup per 64 rows
+// (trsv1_kernel); several, one workgroup where they fit its LDS (trsv_wg_kernel), else one launch
+// per triangle with a workgroup per block row that waits on the flags of the blocks before it
+// (trsv_flow_kernel).
 #include "pvl_internal.hpp"
 #include "lu_common.hpp"
 
@@ -599,6 +600,21 @@ template <int P> __device__ __forceinline__ double quad_bcast(double v)
 template <int P> __device__ __forceinline__ float quad_bcast(float v)
 {
     constexpr int ctrl = P | (P << 2) | (P << 4) | (P << 6);
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xF, 0xF, false));
+}
+
+// Value of the lane whose number differs in the quad's bits M (DPP quad_perm).
+template <int M> __device__ __forceinline__ double quad_xor(double v)
+{
+    constexpr int ctrl = (0 ^ M) | ((1 ^ M) << 2) | ((2 ^ M) << 4) | ((3 ^ M) << 6);
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xF, 0xF, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xF, 0xF, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int M> __device__ __forceinline__ float quad_xor(float v)
+{
+    constexpr int ctrl = (0 ^ M) | ((1 ^ M) << 2) | ((2 ^ M) << 4) | ((3 ^ M) << 6);
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xF, 0xF, false));
 }
 
@@ -1548,43 +1564,6 @@ __global__ void __launch_bounds__(NT) trsv_flow_kernel(const T *__restrict__ A, 
         __hip_atomic_store(&flag[t], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// s4[j] += sum over c in [c0, c1), c = lane mod 64, of arow[j][c] * x[c], for four factor rows:
-// each lane walks its columns in increasing order (the association of a lane-strided dot
-// product); the loads of four columns per row are issued before their FMAs, so that 16 of a
-// lane's loads are in flight at once (the single-workgroup solves are bound by how many bytes
-// one CU keeps in flight, not by arithmetic).
-template <typename T>
-__device__ __forceinline__ void dot4_lane_strided(const T *const (&arow)[4], const T *__restrict__ x, int c0, int c1,
-                                                  int lane, T (&s4)[4])
-{
-    constexpr int U = 4;
-    for (int cb = c0 + lane; cb < c1; cb += 64 * U)
-    {
-        T av[U][4], xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            const int c = cb + 64 * u;
-            const bool ok = c < c1;
-            const int cc = ok ? c : cb; // cb < c1: an in-range column
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                av[u][j] = arow[j][cc];
-            xv[u] = ok ? x[cc] : T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            if (cb + 64 * u < c1)
-            {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    s4[j] = fma(av[u][j], xv[u], s4[j]);
-            }
-        }
-    }
-}
-
 // Whole triangular solve in ONE workgroup (512 threads, at most 96 VGPRs: it fits on a CU
 // beside the side stream's point-velocity waves) for small systems: x (n x nrhs) lives in LDS; blocks of 64
 // rows are taken in solve order, each first reduced by the already solved part (dot products
@@ -1676,126 +1655,200 @@ __global__ void __launch_bounds__(kTrsvWgThreads) __attribute__((amdgpu_waves_pe
         B[i] = x[i];
 }
 
-// Single right-hand side, whole triangular solve in ONE workgroup with look-ahead (the time
-// loop's solve).  Blocks of BS rows are solved in order; block s's reduction by the solved
-// part is split into the blocks solved up to s - 2 ("old", a dot product over contiguous
-// factor rows, as in trsv_wg_kernel) and block s - 1 ("new").  While wave 0 solves block s
-// (the new part from the staged off-diagonal block, then substitution with the staged
-// diagonal block, LAPACK dtrsv order), waves 1-7 stage block s + 1's diagonal block and its
-// off-diagonal block against block s, and form its old part: only wave 0's short chain is
-// on the critical path.  Each row is reduced once by old + new (one subtraction per block,
-// as a blocked dtrsv).  BS = 32 keeps the LDS (x and four BS x (BS + 1) tiles: 42 KB for
-// n = 1,024 in FP64) small enough to share a CU with the side stream's workgroups.
-constexpr int kTrsvLaThreads = 512;
-constexpr int kTrsvLaBs = 32;
-constexpr size_t kTrsvLaMaxX = 32 * 1024; // x in LDS: n <= 4,096 (FP64)
-template <typename T, bool LOWER, int BS>
-__global__ void __launch_bounds__(kTrsvLaThreads) __attribute__((amdgpu_waves_per_eu(5)))
-    trsv_la_kernel(const T *__restrict__ A, int lda, int n, T *__restrict__ b)
+// Single right-hand side (the time loop's solve): one triangle per launch, a workgroup per block of
+// 64 rows.  A block's solution is published in `out`, whose entries hold a signalling NaN until
+// then (kUnsolved, which no arithmetic returns): whoever needs block k polls its 64 values
+// themselves, one memory round trip instead of a flag's and the data's.  Every wave streams its 16
+// rows of the factor block by block, the next block's loads in flight while x of this one is
+// polled; a row's part of a block is a dot product of its own, added to the row's sum, and the
+// sum is subtracted once (a blocked dtrsv's order).  Wave 0 then solves with the diagonal block,
+// lane = row, coefficients from LDS eight columns ahead, x_k broadcast with readlane.  The upper
+// block's columns are scaled by 1/u_kk beforehand (u_ik / u_kk, off the critical path), so that the
+// chain has no division and the quotients are formed once at the end: one more rounding per
+// coefficient, a relative perturbation of U by half an ulp.
+// Bound by the chain of blocks, ~2.5 us each: poll, last block's dot products, 64 substitution
+// steps, store.  At n = 1,024 in FP64 a solve took 420 us in one workgroup per triangle (bound by
+// how fast one CU streams the factor).
+// Workgroups take solve-order indices from a ticket counter, so every smaller index belongs to a
+// workgroup already running; the one with the last ticket resets the counter.  Each workgroup
+// puts its block of `reset` (the other triangle's buffer) back to kUnsolved.  Waits are bounded: a
+// timed-out wait is recorded in the pinned host word kAsyncErrorWord and the workgroup writes NaN.
+constexpr int kAsyncErrorWord = 8;
+template <typename T> struct Unsolved;
+template <> struct Unsolved<double>
+{
+    static constexpr unsigned long long bits = 0x7FF4C0DEC0DE5EEDull;
+};
+template <> struct Unsolved<float>
+{
+    static constexpr unsigned bits = 0x7FA0C0DEu;
+};
+template <typename T> __device__ __forceinline__ bool is_unsolved(T v)
+{
+    return __builtin_bit_cast(typename Bits<T>::U, v) == Unsolved<T>::bits;
+}
+template <typename T> __global__ void __launch_bounds__(256) unsolved_kernel(T *__restrict__ p, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n)
+        p[i] = __builtin_bit_cast(T, Unsolved<T>::bits);
+}
+
+template <typename T, bool LOWER>
+__global__ void __launch_bounds__(256)
+    trsv1_kernel(const T *__restrict__ A, int lda, int n, const T *__restrict__ in, const int *__restrict__ perm,
+                 T *__restrict__ out, T *__restrict__ final_out, T *__restrict__ reset,
+                 unsigned *__restrict__ ticket, int *__restrict__ host)
 {
     main_stream_priority<3>();
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T *x = (T *)smem_raw; // n
-    __shared__ T Dt[2][BS][BS + 1], Ot[2][BS][BS + 1], sold[2][BS];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int nb = (n + BS - 1) / BS;
-    auto blk = [&](int s) { return LOWER ? s : nb - 1 - s; };
-    for (int i = tid; i < n; i += kTrsvLaThreads)
-        x[i] = b[i];
-    // helpers' work for solve step s (block blk(s)), done during step s - 1 (or up front for
-    // s = 0): stage the diagonal block and the off-diagonal block against blk(s - 1), and the
-    // old part over the blocks solved at steps <= s - 2
-    auto prepare = [&](int s, int htid, int hw, int nhw) {
-        const int ib = blk(s), r0 = ib * BS, nr = min(BS, n - r0);
-        const int buf = s & 1;
-        for (int idx = htid; idx < BS * BS; idx += nhw * 64)
-        {
-            const int r = idx / BS, c = idx % BS;
-            Dt[buf][r][c] = (r < nr && c < nr) ? A[(size_t)(r0 + r) * lda + r0 + c] : (r == c ? T(1) : T(0));
-        }
-        if (s >= 1)
-        {
-            const int p0 = blk(s - 1) * BS, np = min(BS, n - p0);
-            for (int idx = htid; idx < BS * BS; idx += nhw * 64)
-            {
-                const int r = idx / BS, c = idx % BS;
-                Ot[buf][r][c] = (r < nr && c < np) ? A[(size_t)(r0 + r) * lda + p0 + c] : T(0);
-            }
-        }
-        // old columns: blocks solved at steps <= s - 2
-        int c0 = 0, c1 = 0;
-        if (s >= 2)
-        {
-            if (LOWER)
-                c0 = 0, c1 = (s - 1) * BS;
-            else
-                c0 = (nb - s + 1) * BS, c1 = n;
-        }
-        for (int g = hw; g < BS / 4; g += nhw)
-        {
-            const int ra = 4 * g;
-            const T *arow[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                arow[j] = A + (size_t)(r0 + min(ra + j, nr - 1)) * lda;
-            T s4[4] = {T(0), T(0), T(0), T(0)};
-            dot4_lane_strided<T>(arow, x, c0, c1, lane, s4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-            {
-                T s2 = s4[j];
-                for (int off = 32; off > 0; off >>= 1)
-                    s2 += __shfl_xor(s2, off);
-                if (lane == 0)
-                    sold[buf][ra + j] = s2;
-            }
-        }
-    };
-    __syncthreads();
-    prepare(0, tid, wv, 8);
-    __syncthreads();
-    for (int s = 0; s < nb; ++s)
+    constexpr int BS = NB, LD = NB + 1;
+    __shared__ T D[BS][LD];
+    __shared__ T xs[4][BS];
+    __shared__ T sums[BS];
+    __shared__ int s_t, s_ok;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nblk = (n + BS - 1) / BS;
+    if (tid == 0)
     {
-        const int buf = s & 1;
-        if (wv == 0)
-        {
-            const int ib = blk(s), r0 = ib * BS, nr = min(BS, n - r0);
-            const int r = lane < BS ? lane : BS - 1;
-            T snew = T(0);
-            if (s >= 1)
-            {
-                const int p0 = blk(s - 1) * BS;
-                T a0 = T(0), a1 = T(0);
-#pragma unroll 4
-                for (int k = 0; k < BS; k += 2)
-                {
-                    a0 = fma(Ot[buf][r][k], x[min(p0 + k, n - 1)], a0);
-                    a1 = fma(Ot[buf][r][k + 1], x[min(p0 + k + 1, n - 1)], a1);
-                }
-                snew = a0 + a1;
-            }
-            T v = lane < nr ? x[r0 + lane] - (sold[buf][r] + snew) : T(0);
-            const T dd = Dt[buf][r][r];
-            for (int kk = 0; kk < BS; ++kk)
-            {
-                const int k = LOWER ? kk : BS - 1 - kk;
-                if (!LOWER && lane == k)
-                    v = v / dd;
-                const T vk = bcast_lane(v, k);
-                if (LOWER ? (lane > k && lane < BS) : lane < k)
-                    v = fma(-Dt[buf][r][k], vk, v);
-            }
-            if (lane < nr)
-                x[r0 + lane] = v;
-        }
-        else if (s + 1 < nb)
-        {
-            prepare(s + 1, tid - 64, wv - 1, 7);
-        }
-        __syncthreads();
+        const int tk = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tk == nblk - 1)
+            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_t = tk;
+        s_ok = 1;
     }
-    for (int i = tid; i < n; i += kTrsvLaThreads)
-        b[i] = x[i];
+    __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(s_t); // solve order
+    const int ib = LOWER ? t : nblk - 1 - t;
+    const int r0 = ib * BS, nr = min(BS, n - r0);
+    // this lane's row and its columns q, q + 4, .. of each block
+    const int q = lane & 3, row = 16 * w + (lane >> 2);
+    const T *Ar = A + (size_t)(r0 + min(row, nr - 1)) * lda;
+    auto block_col = [&](int k) { return (LOWER ? k : nblk - 1 - k) * BS; };
+    T cur[16], nxt[16];
+    auto fetch = [&](T(&v)[16], int c0) {
+        const int last = min(BS, n - c0) - 1;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            v[i] = Ar[c0 + min(q + 4 * i, last)];
+    };
+    // the diagonal block and the right-hand side
+    T dv[16];
+    fetch(dv, r0);
+    const bool live = lane < nr;
+    const int src = r0 + (live ? lane : 0);
+    const T bv = in[perm ? perm[src] : src];
+    if (t > 0)
+        fetch(cur, block_col(0));
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+    {
+        const int c = q + 4 * i;
+        D[row][c] = (row < nr && c < nr) ? dv[i] : (row == c ? T(1) : T(0));
+    }
+    __syncthreads();
+    const T diag = D[lane][lane];
+    if constexpr (!LOWER)
+    {
+        __syncthreads(); // diag is read by every wave before the columns are scaled
+        T u[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            u[i] = D[q + 4 * i][q + 4 * i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (q + 4 * i > row)
+                D[row][q + 4 * i] = D[row][q + 4 * i] / u[i];
+    }
+    T acc = T(0);
+    bool ok = true;
+    for (int k = 0; k < t; ++k)
+    {
+        const int c0 = block_col(k), nc = min(BS, n - c0);
+        if (k + 1 < t)
+            fetch(nxt, block_col(k + 1));
+        T xv = T(0);
+        if (lane < nc)
+        {
+            unsigned spins = 0;
+            const unsigned long long w0 = wall_clock64();
+            for (;;)
+            {
+                xv = xload(&out[c0 + lane]);
+                if (!is_unsolved(xv))
+                    break;
+                if (!ok || ((++spins & 255u) == 0 && wall_clock64() - w0 > kWaitTicks))
+                {
+                    ok = false;
+                    break;
+                }
+            }
+        }
+        xs[w][lane] = xv;
+        wave_lds_fence();
+        T p0 = T(0), p1 = T(0);
+#pragma unroll
+        for (int i = 0; i < 16; i += 2)
+        {
+            p0 = fma(cur[i], xs[w][q + 4 * i], p0);
+            p1 = fma(cur[i + 1], xs[w][q + 4 * i + 4], p1);
+        }
+        acc = acc + (p0 + p1);
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            cur[i] = nxt[i];
+    }
+    if (!ok)
+    {
+        s_ok = 0;
+        __hip_atomic_store(&host[kAsyncErrorWord], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    acc = acc + quad_xor<1>(acc);
+    acc = acc + quad_xor<2>(acc);
+    if (q == 0)
+        sums[row] = acc;
+    __syncthreads();
+    if (w != 0)
+        return;
+    T x = live ? bv - sums[lane] : T(0), res = T(0);
+    constexpr int KC = 8;
+    T lc[KC], ln[KC];
+#pragma unroll
+    for (int u = 0; u < KC; ++u)
+        lc[u] = D[lane][LOWER ? u : BS - 1 - u];
+    for (int kc = 0; kc < BS; kc += KC)
+    {
+        if (kc + KC < BS)
+        {
+#pragma unroll
+            for (int u = 0; u < KC; ++u)
+                ln[u] = D[lane][LOWER ? kc + KC + u : BS - 1 - (kc + KC + u)];
+        }
+#pragma unroll
+        for (int u = 0; u < KC; ++u)
+        {
+            const int k = LOWER ? kc + u : BS - 1 - (kc + u);
+            // the lane's own value is final at its step; what later steps do to it is not used
+            const T xk = bcast_lane(x, k);
+            res = lane == k ? x : res;
+            x = fma(-lc[u], xk, x);
+        }
+#pragma unroll
+        for (int u = 0; u < KC; ++u)
+            lc[u] = ln[u];
+    }
+    if constexpr (!LOWER)
+        res = res / diag;
+    if (!s_ok)
+        res = T(NAN);
+    if (live)
+    {
+        xstore(&out[r0 + lane], res);
+        if (final_out)
+            final_out[r0 + lane] = res;
+        reset[r0 + lane] = __builtin_bit_cast(T, Unsolved<T>::bits);
+    }
 }
 
 // R = B - A X on FP64 MFMA (v_mfma_f64_16x16x4f64), for the refinement's FP64 residuals: a
@@ -1955,7 +2008,6 @@ __global__ void status_to_host_kernel(const int *__restrict__ status, int *__res
 
 // A timed-out wait of the single-launch solve (err[5]) is recorded in the pinned host word
 // kAsyncErrorWord, where it stays until the host takes it at its next synchronisation.
-constexpr int kAsyncErrorWord = 8;
 __global__ void record_async_error_kernel(const int *__restrict__ err, int *__restrict__ host)
 {
     main_stream_priority();
@@ -2264,6 +2316,7 @@ struct pvl_lu
     float *dinv = nullptr; // FP32: inverses of the 128 x 128 diagonal blocks of L and U
     bool dinv_valid = false;
     unsigned *flow = nullptr; // tickets and block flags of the single-launch solves
+    void *single = nullptr;   // 2 n (T): exchange buffers of the single-right-hand-side solve
     unsigned epoch = 0;       // flag value of the latest solve launch
 };
 
@@ -2312,6 +2365,19 @@ template <typename T> int solve_impl(pvl_lu *h, T *B, int nrhs)
     if (int st = ensure_ws())
         return st;
     T *work = (T *)h->work;
+    if (nrhs == 1)
+    {
+        ProfScope prof(sizeof(T) == 8 ? "lu_trsv_f64" : "lu_trsv_f32");
+        const T *Ap = (const T *)h->lu;
+        T *y = (T *)h->single, *x = y + n;
+        const int nb = (n + NB - 1) / NB;
+        trsv1_kernel<T, true><<<nb, 256, 0, stream()>>>(Ap, n, n, B, h->perm, y, (T *)nullptr, x, h->flow + 2,
+                                                        g_status_host_dev);
+        trsv1_kernel<T, false><<<nb, 256, 0, stream()>>>(Ap, n, n, y, nullptr, x, B, y, h->flow + 3,
+                                                         g_status_host_dev);
+        PVL_HIP(hipGetLastError());
+        return PVL_OK;
+    }
     for (int q0 = 0; q0 < nrhs; q0 += kMaxRhs)
     {
         const int nq = std::min(kMaxRhs, nrhs - q0);
@@ -2327,15 +2393,7 @@ template <typename T> int solve_impl(pvl_lu *h, T *B, int nrhs)
         }
         PVL_HIP(hipGetLastError());
         const size_t xbytes = sizeof(T) * (size_t)n * nq;
-        if (nq == 1 && xbytes <= kTrsvLaMaxX)
-        {
-            ProfScope prof(sizeof(T) == 8 ? "lu_trsv_f64" : "lu_trsv_f32");
-            const T *Ap = (const T *)h->lu;
-            trsv_la_kernel<T, true, kTrsvLaBs><<<1, kTrsvLaThreads, xbytes, stream()>>>(Ap, n, n, work);
-            trsv_la_kernel<T, false, kTrsvLaBs><<<1, kTrsvLaThreads, xbytes, stream()>>>(Ap, n, n, work);
-            PVL_HIP(hipGetLastError());
-        }
-        else if (xbytes <= (size_t)kTrsvWgBytes)
+        if (xbytes <= (size_t)kTrsvWgBytes)
         {
             ProfScope prof(sizeof(T) == 8 ? "lu_trsv_f64" : "lu_trsv_f32");
             const T *Ap = (const T *)h->lu;
@@ -2384,6 +2442,12 @@ int alloc_handle(pvl_lu *h, int n, int prec)
     PVL_HIP(hipMalloc(&h->work, es * (size_t)n * kMaxRhs));
     const int nblk = (n + NB - 1) / NB;
     PVL_HIP(hipMalloc(&h->flow, sizeof(unsigned) * (kFlowHeader + nblk)));
+    PVL_HIP(hipMalloc(&h->single, 2 * es * (size_t)n));
+    if (prec == PVL_FP64)
+        unsolved_kernel<double><<<(2 * n + 255) / 256, 256, 0, stream()>>>((double *)h->single, 2 * n);
+    else
+        unsolved_kernel<float><<<(2 * n + 255) / 256, 256, 0, stream()>>>((float *)h->single, 2 * n);
+    PVL_HIP(hipGetLastError());
     return device_fill32(h->flow, 0u, sizeof(unsigned) * (kFlowHeader + nblk));
 }
 
@@ -2437,6 +2501,7 @@ int pvl_lu_destroy(pvl_lu *h)
     (void)hipFree(h->work);
     (void)hipFree(h->dinv);
     (void)hipFree(h->flow);
+    (void)hipFree(h->single);
     delete h;
     return PVL_OK;
 }
