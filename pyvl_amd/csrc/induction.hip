@@ -59,6 +59,55 @@ __global__ void __launch_bounds__(256) line_geom_kernel(unsigned n_lines, const 
     out[i] = g;
 }
 
+// Record of the accurate forms (LineMid) with the line's circulation, the sum over the surfaces
+// holding the line of +-Gamma_s in increasing surface order.  A line cut by
+// length takes the far form everywhere (direction 0: every pair's c and h^2 are 0 and it is cut);
+// lengths whose squares could leave the range of a double never do.
+__global__ void __launch_bounds__(256) line_mid_kernel(unsigned n_lines, const uint32_t *__restrict__ lines,
+                                                      const double *__restrict__ pos, double tol,
+                                                      const uint32_t *__restrict__ loff,
+                                                      const uint32_t *__restrict__ lsurf,
+                                                      const double *__restrict__ circ, LineMid *__restrict__ out)
+{
+    main_stream_priority();
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_lines)
+        return;
+    const uint32_t p1 = lines[2 * i] & kInvalidId, p2 = lines[2 * i + 1] & kInvalidId;
+    const double ax = pos[3 * p1 + 0], ay = pos[3 * p1 + 1], az = pos[3 * p1 + 2];
+    const double bx = pos[3 * p2 + 0], by = pos[3 * p2 + 1], bz = pos[3 * p2 + 2];
+    const double dx = bx - ax, dy = by - ay, dz = bz - az;
+    LineMid g;
+    g.mx = 0.5 * (ax + bx), g.my = 0.5 * (ay + by), g.mz = 0.5 * (az + bz);
+    g.len = sqrt(dx * dx + dy * dy + dz * dz);
+    g.ex = dx / g.len;
+    g.ey = dy / g.len;
+    g.ez = dz / g.len;
+    const bool cut = g.len < tol;
+    if (cut)
+        g.ex = g.ey = g.ez = g.len = 0.0;
+    g.quarter = 0.25 * (g.len * g.len);
+    g.far_b = cut ? 0.0 : (g.len >= 1e-100 && g.len <= 1e100) ? 3.75 * (g.len * g.len) : __builtin_inf();
+    g.gamma = 0.0;
+    for (uint32_t k = loff[i]; k < loff[i + 1]; ++k)
+    {
+        const uint32_t e = lsurf[k];
+        const double c = circ[e & kInvalidId];
+        g.gamma = (e & kReversed) ? g.gamma - c : g.gamma + c;
+    }
+    out[i] = g;
+}
+
+// The record each precision's kernels read.
+template <int PREC> struct LineRecord
+{
+    using type = LineMid;
+};
+template <> struct LineRecord<PVL_FP64_REF_FORM>
+{
+    using type = LineGeom;
+};
+
 __device__ __forceinline__ unsigned wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
 __device__ __forceinline__ unsigned lane_id() { return threadIdx.x % kWave; }
 
@@ -342,25 +391,23 @@ __global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines,
 // does not depend on scheduling.  Work items are (64 PPL-point block, line chunk) pairs,
 // item = chunk * pblocks + block; workgroup b takes items b, b + gridDim.x, .. (a grid
 // smaller than the item count leaves CU slots to other work on the device; each item's
-// arithmetic is the same either way).  With PPL = 2 each lane runs two independent
-// evaluation chains per line (instruction-level parallelism) and every line's geometry,
-// loaded once into scalar registers, serves twice the points.
-// SITE only gives the free-wake self-induction launch its own symbol for profilers; it
-// uses PPL = 2, the other sites PPL = 1.  The self-induction kernel needs 60 VGPRs: five
-// workgroups per CU on the side stream (one wave each per SIMD) leave each SIMD 192 VGPRs
-// for the library stream's kernels.
-template <int SITE> constexpr int site_ppl() { return SITE == 1 ? 2 : 1; }
+// arithmetic is the same either way).  Bound by FP64 issue: 43 slots per far pair.  With PPL = 2
+// each lane runs two independent evaluation chains per line and every line's record, loaded once
+// into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.70 ms (1.45 ms
+// in the general form with one point per lane; one point per lane in this form 0.74 ms).
+// SITE only gives the free-wake self-induction launch its own symbol for profilers.
+constexpr int kPvPPL = 2;
 
 template <int PREC, int SITE>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SITE == 1 ? 4 : 6)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
     point_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, unsigned n_lines,
-                          const LineGeom *__restrict__ geom, const double *__restrict__ gamma,
-                          unsigned lines_per_chunk, double *__restrict__ partial, double tol, unsigned pblocks,
+                          const typename LineRecord<PREC>::type *__restrict__ geom, const double *__restrict__ gamma,
+                          const uint32_t *__restrict__ lines, const double *__restrict__ pos, unsigned lines_per_chunk, double *__restrict__ partial, double tol, unsigned pblocks,
                           unsigned n_items)
 {
     if constexpr (SITE == 0)
         main_stream_priority();
-    constexpr int PPL = site_ppl<SITE>();
+    constexpr int PPL = kPvPPL;
     __shared__ double red[4][3][kWave * PPL];
     const unsigned w = wave_id(), lane = lane_id();
     const double tol2 = tol * tol;
@@ -384,11 +431,11 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SIT
         const unsigned b = (a + per_wave) < l1 ? (a + per_wave) : l1;
         for (unsigned l = a; l < b; ++l)
         {
-            const LineGeom g = geom[l];
-            const double gl = gamma[l];
-#pragma unroll
-            for (int j = 0; j < PPL; ++j)
-                line_k_acc<PREC>(g, px[j], py[j], pz[j], tol, tol2, gl, vx[j], vy[j], vz[j]);
+            const auto g = geom[l];
+            if constexpr (PREC == PVL_FP64_REF_FORM)
+                line_k_acc<PREC, PPL>(g, gamma[l], px, py, pz, tol, tol2, vx, vy, vz);
+            else
+                line_k_acc<PREC, PPL>(g, lines + 2 * l, pos, px, py, pz, tol, tol2, vx, vy, vz);
         }
 #pragma unroll
         for (int j = 0; j < PPL; ++j)
@@ -939,33 +986,38 @@ namespace pvl
 // Point-velocity sum over the first n_active lines of the mesh (all lines for the public
 // entry point; the wake passes the prefix of lines its filled rows use -- the other lines
 // carry zero circulation).
-// Chunking: aim for >= ~4 workgroups per CU while keeping >= 64 lines per wave.
+// Chunking: aim for 4,096 workgroups of two points per lane while keeping >= 64 lines per wave.  Half
+// of that left the last round of waves half empty (30,000 points: 0.80 against 0.72 ms); twice of
+// it gains 3 % there and costs 1 % in a wake of 3,200 panels, in partial sums.  Where the partial sums and the line records of such a
+// plan would not fit pvl_point_velocity_noalloc's fixed scratch, the chunk count of 2,048 workgroups
+// of one point per lane, which is half as many.  One rule for both entry points: same sums.
 static bool self_site(const char *prof_name) { return std::strcmp(prof_name, "wake_self_velocity") == 0; }
-static unsigned site_points_per_group(const char *prof_name)
+constexpr unsigned kPvPoints = kWave * kPvPPL; // per workgroup
+
+static void plan_chunks(unsigned n_pts, unsigned n_active, unsigned *n_chunks_out, unsigned *lpc_out)
 {
-    return kWave * (self_site(prof_name) ? site_ppl<1>() : site_ppl<0>());
+    const auto plan = [&](unsigned groups, unsigned points, unsigned *lpc) {
+        const unsigned pblocks = (n_pts + points - 1) / points;
+        unsigned n_chunks = (groups + pblocks - 1) / pblocks;
+        const unsigned max_chunks = (n_active + 255) / 256;
+        if (n_chunks > max_chunks)
+            n_chunks = max_chunks;
+        if (n_chunks < 1)
+            n_chunks = 1;
+        if (n_chunks > 65535u)
+            n_chunks = 65535u;
+        *lpc = (n_active + n_chunks - 1) / n_chunks;
+        return (n_active + *lpc - 1) / *lpc;
+    };
+    *n_chunks_out = plan(4096, kPvPoints, lpc_out);
+    if (point_velocity_scratch(n_pts, n_active, *n_chunks_out) > PVL_NOALLOC_SCRATCH_BYTES)
+        *n_chunks_out = plan(2048, kWave, lpc_out);
 }
 
-static void plan_chunks(unsigned n_pts, unsigned n_active, unsigned ppg, unsigned *n_chunks_out, unsigned *lpc_out)
-{
-    const unsigned pblocks = (n_pts + ppg - 1) / ppg;
-    unsigned n_chunks = (2048 + pblocks - 1) / pblocks;
-    const unsigned max_chunks = (n_active + 255) / 256;
-    if (n_chunks > max_chunks)
-        n_chunks = max_chunks;
-    if (n_chunks < 1)
-        n_chunks = 1;
-    if (n_chunks > 65535u)
-        n_chunks = 65535u;
-    const unsigned lpc = (n_active + n_chunks - 1) / n_chunks;
-    *n_chunks_out = (n_active + lpc - 1) / lpc;
-    *lpc_out = lpc;
-}
-
-unsigned point_velocity_chunks(unsigned n_pts, unsigned n_active, const char *prof_name)
+unsigned point_velocity_chunks(unsigned n_pts, unsigned n_active)
 {
     unsigned nc, lpc;
-    plan_chunks(n_pts, n_active, site_points_per_group(prof_name), &nc, &lpc);
+    plan_chunks(n_pts, n_active, &nc, &lpc);
     return nc;
 }
 
@@ -975,26 +1027,34 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
                             const double *pts, int precision, unsigned n_active, const char *prof_name,
                             hipStream_t s, void *geom, double *gamma, double *partial, unsigned max_groups)
 {
-    LineGeom *g = (LineGeom *)geom;
-    line_geom_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, g);
-    PVL_HIP(hipGetLastError());
-    line_circulation_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_line_offsets, m->d_line_surfs,
-                                                                     circ, gamma);
+    if (precision == PVL_FP64_REF_FORM)
+    {
+        line_geom_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, (LineGeom *)geom);
+        PVL_HIP(hipGetLastError());
+        line_circulation_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_line_offsets,
+                                                                         m->d_line_surfs, circ, gamma);
+    }
+    else
+        line_mid_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, m->d_line_offsets,
+                                                               m->d_line_surfs, circ, (LineMid *)geom);
     PVL_HIP(hipGetLastError());
     unsigned n_chunks, lpc;
-    const unsigned ppg = site_points_per_group(prof_name);
-    plan_chunks(n_pts, n_active, ppg, &n_chunks, &lpc);
-    const unsigned pblocks = (n_pts + ppg - 1) / ppg;
+    plan_chunks(n_pts, n_active, &n_chunks, &lpc);
+    const unsigned pblocks = (n_pts + kPvPoints - 1) / kPvPoints;
     const unsigned n_items = pblocks * n_chunks;
     const unsigned grid = max_groups && max_groups < n_items ? max_groups : n_items;
     ProfScope prof(prof_name, (double)n_pts * (double)n_active, s);
     dispatch_precision(precision, [&](auto P) {
         if (self_site(prof_name))
             point_velocity_kernel<decltype(P)::value, 1>
-                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active, g, gamma, lpc, partial, tol, pblocks, n_items);
+                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active,
+                (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
+                m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
         else
             point_velocity_kernel<decltype(P)::value, 0>
-                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active, g, gamma, lpc, partial, tol, pblocks, n_items);
+                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active,
+                (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
+                m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
     });
     PVL_HIP(hipGetLastError());
     return PVL_OK;
@@ -1080,7 +1140,7 @@ int point_velocity_impl(const pvl_mesh *m, double tol, const double *pos, const 
                 return st;
         return PVL_OK;
     }
-    const unsigned n_chunks = point_velocity_chunks(n_pts, n_active, prof_name);
+    const unsigned n_chunks = point_velocity_chunks(n_pts, n_active);
     void *g = scratch(0, line_geom_bytes(n_active));
     double *gamma = (double *)scratch(1, sizeof(double) * n_active);
     double *partial = (double *)scratch(2, sizeof(double) * 3 * (size_t)n_pts * n_chunks);

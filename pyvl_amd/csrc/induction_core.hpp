@@ -199,7 +199,7 @@ __device__ __forceinline__ double pvl_rsqrt(double x)
 template <int PREC, int COEF = 0>
 __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double len, double d1x, double d1y,
                                          double d1z, double q1, double d2x, double d2y, double d2z, double q2,
-                                         double tol, double tol2, bool &cut)
+                                         double tol, double tol2, bool &cut, const double *table = nullptr)
 {
     const double t1 = ex * d1x + ey * d1y + ez * d1z;
     const double t2 = ex * d2x + ey * d2y + ez * d2z;
@@ -228,7 +228,7 @@ __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double
         {
             const double ih = pvl_rsqrt(h2);
             const double h = h2 * ih;
-            const double dphi = pvl_atan2_neg<COEF>(len * h, fma(t1, t2, h2));
+            const double dphi = pvl_atan2_neg<COEF>(len * h, fma(t1, t2, h2), table);
             m = dphi * ih;
         }
         else
@@ -378,29 +378,122 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     }
 }
 
-// v += w K(line, p): the point-velocity inner step (w = the line's circulation).  The
-// non-reference forms scale once (w m) and accumulate with FMAs.
-template <int PREC>
-__device__ __forceinline__ void line_k_acc(const LineGeom &g, double px, double py, double pz, double tol,
-                                           double tol2, double w, double &vx, double &vy, double &vz)
+// The accurate forms of the point-velocity sums, from line records about the midpoint: m = p - mid,
+// c = m x e (= dr1 x e: K's direction, |c| = h), B = dr1 . dr2 = |m|^2 - len^2 / 4, three operations
+// fewer per pair than from the end points.  From two lengths off the midpoint on
+// (B >= far_b = 3.75 len^2, for all points of a wave) the far form above holds with s <= 0.2845 and a
+// degree-10 P (relative error 3.2e-16: tools/fit_atan.py 10 double 0.2844); points in no particular
+// order make boxes useless, and the test costs one comparison per line.  Otherwise the whole wave
+// takes the general form, from the line's own end points (its h^2 is the reference's, rounding
+// included, which is what separates the two near a line).  43 issue slots per far pair, against
+// ~102 of the general form.
+struct LineMid
 {
-    if constexpr (PREC == PVL_FP64_REF_FORM)
+    double mx, my, mz;
+    double quarter; // len^2 / 4
+    double ex, ey, ez;
+    double len;
+    double far_b; // infinity: always the general form
+    double gamma; // the line's circulation (point-velocity sums)
+};
+static_assert(sizeof(LineMid) == sizeof(LineGeom), "one scratch size for both records");
+
+// angle / h (negative, as K's factor).
+__device__ __forceinline__ double mid_far(double b, double h2, double len)
+{
+    const double q = len * far_rcp(b);
+    const double u = (h2 * q) * q;
+    double p = -1.0530409925033454105e-2;
+    asm("v_fma_f64 %0, %0, %1, %2\n\t"
+        "v_fma_f64 %0, %0, %1, %3\n\t"
+        "v_fma_f64 %0, %0, %1, %4\n\t"
+        "v_fma_f64 %0, %0, %1, %5\n\t"
+        "v_fma_f64 %0, %0, %1, %6\n\t"
+        "v_fma_f64 %0, %0, %1, %7\n\t"
+        "v_fma_f64 %0, %0, %1, %8\n\t"
+        "v_fma_f64 %0, %0, %1, %9\n\t"
+        "v_fma_f64 %0, %0, %1, %10\n\t"
+        "v_fma_f64 %0, %0, %1, %11"
+        : "+v"(p)
+        : "v"(u), "s"(2.9501554043661432491e-2), "s"(-4.6025268387594494587e-2), "s"(5.7199422485590436944e-2),
+          "s"(-6.6394999569895820257e-2), "s"(7.6892308217604938091e-2), "s"(-9.0906782661688777695e-2),
+          "s"(1.1111100144380131558e-1), "s"(-1.4285713981516674141e-1), "s"(1.9999999995777831413e-1),
+          "s"(-3.3333333333312912204e-1));
+    return -fma(q * u, p, q);
+}
+
+// v[j] += gamma K(line, p[j]): the point-velocity inner step.  The non-reference forms scale once
+// and accumulate with FMAs.
+template <int PREC, int PPL>
+__device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, const double (&px)[PPL],
+                                           const double (&py)[PPL], const double (&pz)[PPL], double tol, double tol2,
+                                           double (&vx)[PPL], double (&vy)[PPL], double (&vz)[PPL])
+{
+#pragma unroll
+    for (int j = 0; j < PPL; ++j)
     {
         double kx, ky, kz;
-        line_k<PREC>(g, px, py, pz, tol, tol2, kx, ky, kz);
-        vx = vx + w * kx;
-        vy = vy + w * ky;
-        vz = vz + w * kz;
+        line_k<PREC>(g, px[j], py[j], pz[j], tol, tol2, kx, ky, kz);
+        vx[j] = vx[j] + gamma * kx;
+        vy[j] = vy[j] + gamma * ky;
+        vz[j] = vz[j] + gamma * kz;
+    }
+}
+// ab: the line's two end points in the mesh (read only when near), pos: their coordinates.
+template <int PREC, int PPL>
+__device__ __forceinline__ void line_k_acc(const LineMid &g, const uint32_t *ab, const double *pos,
+                                           const double (&px)[PPL], const double (&py)[PPL], const double (&pz)[PPL],
+                                           double tol, double tol2, double (&vx)[PPL], double (&vy)[PPL],
+                                           double (&vz)[PPL])
+{
+    double cx[PPL], cy[PPL], cz[PPL], b[PPL], w[PPL];
+    bool far = true;
+#pragma unroll
+    for (int j = 0; j < PPL; ++j)
+    {
+        const double mx = px[j] - g.mx, my = py[j] - g.my, mz = pz[j] - g.mz;
+        b[j] = fma(mx, mx, fma(my, my, fma(mz, mz, -g.quarter)));
+        far = far && b[j] >= g.far_b;
+        cx[j] = fma(my, g.ez, -(mz * g.ey));
+        cy[j] = fma(mz, g.ex, -(mx * g.ez));
+        cz[j] = fma(mx, g.ey, -(my * g.ex));
+    }
+    if (__builtin_amdgcn_ballot_w64(!far) == 0)
+    {
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
+        {
+            const double h2 = fma(cx[j], cx[j], fma(cy[j], cy[j], cz[j] * cz[j]));
+            const double f = g.gamma * mid_far(b[j], h2, g.len);
+            w[j] = h2 < tol2 ? 0.0 : f;
+        }
     }
     else
     {
-        double d1x, d1y, d1z;
-        bool cut;
-        const double m = line_m<PREC>(g, px, py, pz, tol, tol2, d1x, d1y, d1z, cut);
-        const double wm = cut ? 0.0 : w * m;
-        vx = fma(wm, fma(d1y, g.ez, -(d1z * g.ey)), vx);
-        vy = fma(wm, fma(d1z, g.ex, -(d1x * g.ez)), vy);
-        vz = fma(wm, fma(d1x, g.ey, -(d1y * g.ex)), vz);
+        const double *table = PREC == PVL_FP64 ? atan_table() : nullptr;
+        const double *r1 = pos + 3 * (size_t)(ab[0] & pvl::kInvalidId), *r2 = pos + 3 * (size_t)(ab[1] & pvl::kInvalidId);
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
+        {
+            const double d1x = px[j] - r1[0], d1y = py[j] - r1[1], d1z = pz[j] - r1[2];
+            const double d2x = px[j] - r2[0], d2y = py[j] - r2[1], d2z = pz[j] - r2[2];
+            const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
+            const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
+            bool cut;
+            const double f = g.gamma * pair_m<PREC, 2>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2,
+                                                       tol, tol2, cut, table);
+            w[j] = cut ? 0.0 : f;
+            cx[j] = fma(d1y, g.ez, -(d1z * g.ey));
+            cy[j] = fma(d1z, g.ex, -(d1x * g.ez));
+            cz[j] = fma(d1x, g.ey, -(d1y * g.ex));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < PPL; ++j)
+    {
+        vx[j] = fma(w[j], cx[j], vx[j]);
+        vy[j] = fma(w[j], cy[j], vy[j]);
+        vz[j] = fma(w[j], cz[j], vz[j]);
     }
 }
 

@@ -15,8 +15,6 @@ constexpr int kMaxDevices = 64;
 // Device address of `scratch` on each device, from hipGetSymbolAddress at set-up.
 void *g_scratch_dev[kMaxDevices] = {};
 
-constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
-
 } // namespace
 
 // Working memory of the no-allocation entry point, one copy per device, held until the
@@ -89,11 +87,10 @@ extern "C" int pvl_point_velocity_noalloc(const pvl_mesh *m, double tol, const d
     if (n_active == 0)
         return accumulate ? PVL_OK : device_fill32(out, 0u, sizeof(double) * 3 * (size_t)n_pts);
 
-    const unsigned n_chunks = point_velocity_chunks(n_pts, n_active, "point_velocity");
+    const unsigned n_chunks = point_velocity_chunks(n_pts, n_active);
     const size_t geom_bytes = align256(line_geom_bytes(n_active));
     const size_t gamma_bytes = align256(sizeof(double) * (size_t)n_active);
-    const size_t partial_bytes = sizeof(double) * 3 * (size_t)n_pts * n_chunks;
-    const size_t need = geom_bytes + gamma_bytes + partial_bytes;
+    const size_t need = point_velocity_scratch(n_pts, n_active, n_chunks);
     if (need > kScratchBytes)
     {
         set_error("pvl_point_velocity_noalloc: %u points x %u lines need %zu bytes of scratch, more than its fixed "

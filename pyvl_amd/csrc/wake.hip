@@ -526,7 +526,7 @@ static unsigned self_chunks(const pvl_wake *w, unsigned n_pts)
 {
     if (w->chains)
         return chain_velocity_chunks(n_pts, w->pieces_at[active_rows(w)]);
-    return point_velocity_chunks(n_pts, active_lines(w), "wake_self_velocity");
+    return point_velocity_chunks(n_pts, active_lines(w));
 }
 
 // Buffers of the self-induction: line circulations, segment records (chains) or line

@@ -7,13 +7,17 @@ the extension of the segments (cut off), segments shorter than the cut-off.
 Tolerance: the oracle's own rounding of h^2 and of a difference of two atan2 values is what
 separates the two (1e-12 of the largest velocity, the bound of the other parity tests)."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle import wake_oracle as WO
 from oracle import oracle as O
+from pyvl_amd import _lib
 from pyvl_amd import geometry as G
 from pyvl_amd.cvl import Mesh
+from pyvl_amd.device import DeviceArray
 from pyvl_amd.solver import FlowConditionsUniform, HeaveFrame, make_wing_wake_solver
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +57,45 @@ def test_free_wake_step_near_and_far_pieces(n_span, rows, flat):
     v = np.max(np.abs((ow.wake_positions[:, :, 1:] - pos[:, :, :-1]) / dt))
     assert np.max(np.abs(wp - ow.wake_positions)) <= dt * 1e-12 * v + 1e-14
     assert np.linalg.norm(wc - ow.circulation) <= 1e-12 * np.linalg.norm(ow.circulation)
+
+
+@pytest.mark.parametrize("n_pts", [1, 63, 64, 65, 127, 128, 129, 200])
+@pytest.mark.parametrize("lo,hi", [(2.05, 40.0), (1.9, 2.1), (0.05, 3.0)])
+def test_point_velocity_near_and_far_lines(n_pts, lo, hi):
+    """Sums whose waves are all far from a line, all at the border of the rule (two lengths from the
+    midpoint), or near: points around the lines of a small mesh with one zero-length line (a
+    collapsed panel edge), some of them on a line's extension (cut off)."""
+    rng = np.random.default_rng(n_pts)
+    pos, el, _ = G.flat_wing(3, 2, 3.0, 2.0)
+    pos[:, 2] += 0.05 * rng.normal(size=pos.shape[0])
+    pos[el[1][1]] = pos[el[1][0]]
+    m, t = Mesh(pos.shape[0], el), O.mesh_from_elements(pos.shape[0], el)
+    e = rng.integers(0, len(el), n_pts)
+    a, b = (pos[np.array([el[i][k] for i in e])] for k in (2, 3))
+    d = rng.normal(size=(n_pts, 3))
+    r = rng.uniform(lo, hi, (n_pts, 1)) * np.linalg.norm(b - a, axis=1, keepdims=True)
+    pts = 0.5 * (a + b) + r * d / np.linalg.norm(d, axis=1, keepdims=True)
+    pts[::7] = (b + lo * (b - a))[::7]
+    pts = np.ascontiguousarray(pts)
+    circ = rng.normal(size=m.n_surfaces)
+    want = O.point_velocity(t, pos, circ, pts, 1e-6)
+    got = m.point_velocity(1e-6, pos, circ, pts)
+    assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
+
+
+def test_noalloc_holds_meshes_near_its_scratch_limit():
+    """Line records alone near the fixed scratch: the smaller chunk count is taken, by both entry
+    points, and the call is not refused."""
+    _lib.call("pvl_init", 0)
+    pos, el = G.uv_sphere(512, 300, sigma=1e-4, seed=1)
+    m, rng = Mesh(pos.shape[0], el), np.random.default_rng(2)
+    assert 88 * m.n_lines + 24 * 512 * 1000 > (32 << 20) > 88 * m.n_lines + 24 * 128 * 1000
+    pts = DeviceArray.from_numpy(rng.normal(0.0, 1.5, (1000, 3)))
+    dpos, circ = DeviceArray.from_numpy(pos), DeviceArray.from_numpy(rng.normal(size=m.n_surfaces))
+    out = []
+    for name in ("pvl_point_velocity", "pvl_point_velocity_noalloc"):
+        v = DeviceArray((1000, 3))
+        _lib.check(getattr(_lib.load(), name)(m._device(), C.c_double(1e-6), dpos.cptr, circ.cptr, C.c_uint(1000),
+                                              pts.cptr, v.cptr, C.c_int(0), C.c_int(_lib.PVL_FP64)), name)
+        out.append(v.numpy())
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
