@@ -229,16 +229,21 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // Normal-reduced assembly (induction_matrix3), out[n_cpts][n_surf]: one lane per control
-// point, one wave per run of up to kAsmGroups groups of kAsmSurfaces consecutive surfaces,
+// point, one wave per run of one to kAsmGroups groups of kAsmSurfaces consecutive surfaces,
 // executing the run's program (build_assembly_program): each line of the run is evaluated
 // once, as n . K, and kept in an LDS slot while a later surface of the run needs it; a
 // surface's value is the sum of its lines' +-n.K in CSR order (src/core/flow_solver.c:188-202
 // sums the vectors first and then dots with the normal: the same terms, another association).
 // Program entries are wave-uniform (scalar loads and branches); per lane the inner step is one
 // K and one LDS access at most.  Each group's results are staged in LDS and stored as rows of
-// kAsmSurfaces consecutive doubles.
+// kAsmSurfaces consecutive doubles.  Bound by FP64 issue where the chip is full (~60 slots per line
+// in the far form, which all but 1 % of the waves' lines take at 16,384 surfaces: 1.50 ms, 2.10 in
+// the general form) and by the latency of a wave's chain of evaluations where it is not.  A pair's
+// program words are loaded one pair ahead; loading its lines ahead as well (two records more in
+// scalar registers, or one with everything copied to VGPRs first) spilled and was slower (2.1 ms).
+// Four waves per SIMD, which the LDS allows, leave the registers for the coefficients.
 template <int PREC>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
     assembly_kernel(unsigned n_cpts, unsigned n_surf, unsigned n_runs, const uint32_t *__restrict__ run_off,
                     const uint32_t *__restrict__ run_grp, const uint32_t *__restrict__ prog,
                     const LineGeom *__restrict__ geom, const double *__restrict__ cpts,
@@ -288,15 +293,20 @@ __global__ void __launch_bounds__(kBlock)
         }
     };
     // groups have even entry counts (padded), so a group ends on a pair boundary
+    if (k0 >= k1)
+        return;
+    const uint4 *words = (const uint4 *)prog;
+    uint4 next = words[k0 / 2];
     for (uint32_t k = k0; k < k1; k += 2)
     {
         // a kAsmNone entry names line 0 (the geometry buffer always has one element)
-        const uint32_t ea = prog[2 * k], opa = prog[2 * k + 1], eb = prog[2 * k + 2], opb = prog[2 * k + 3];
+        const uint32_t ea = next.x, opa = next.y, eb = next.z, opb = next.w;
         const LineGeom ga = geom[ea & kInvalidId], gb = geom[eb & kInvalidId];
+        next = words[min(k + 2, k1 - 2) / 2];
         // both geometries in SGPRs here (the compiler would otherwise sink the second load
         // into the branch that uses it, after the first evaluation)
         asm volatile("" ::"s"(ga.r1x), "s"(ga.r2x), "s"(ga.ex), "s"(ga.len), "s"(gb.r1x), "s"(gb.r2x), "s"(gb.ex),
-                     "s"(gb.len));
+                     "s"(gb.len), "s"(next.x));
         step(ea, opa, ga);
         step(eb, opb, gb);
         if (sl == ns)
@@ -896,7 +906,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
             const SegRec *sg = segs + hd.first_seg;
             const double *gg = seg_gamma + hd.first_seg;
             // one segment in the general form, and on to its end node
-            auto general = [&](unsigned j, const double *table) {
+            auto general = [&](unsigned j, AtanTable table) {
                 const double nx = sg[j].nx, ny = sg[j].ny, nz = sg[j].nz;
                 const double ex = sg[j].ex, ey = sg[j].ey, ez = sg[j].ez, len = sg[j].len, gamma = gg[j];
 #pragma unroll
@@ -960,7 +970,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
             }
             else
             {
-                const double *table = PREC == PVL_FP64 ? atan_table() : nullptr;
+                AtanTable table = PREC == PVL_FP64 ? atan_table() : nullptr;
                 for (unsigned j = 0; j < n; ++j)
                     general(j, table);
             }

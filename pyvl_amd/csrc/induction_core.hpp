@@ -39,57 +39,42 @@ enum
 // pyvl_amd/csrc/tools/fit_atan.py (Lawson iteration in 60-digit arithmetic): P of degree 16
 // for FP64 (maximum relative error of the polynomial 1.1e-15, ~5 ulp: the pair's other
 // rounding errors are of that order), degree 7 for FP32 (1.7e-8).
-// SGPR_COEF: the Horner steps as one inline-asm block of v_fma_f64 with the coefficients in
-// SGPRs.  In kernels whose loop has enough control flow around the evaluation the compiler
-// otherwise keeps the loop-invariant coefficients in VGPRs and emits every step as a copy
-// plus the two-address v_fmac_f64 (twice the instructions); the same 15 FMAs in the same
+// VGPR_COEF: every Horner step as one three-address v_fma_f64 with the coefficient in VGPRs, where
+// the kernel has those to spare.  In loops with enough control flow around the evaluation the
+// compiler otherwise keeps the loop-invariant coefficients in VGPRs all the same and emits every
+// step as a copy plus the two-address v_fmac_f64 (twice the instructions); the same FMAs in the same
 // order, so the results are bit-identical.
-template <bool SGPR_COEF = false> __device__ __forceinline__ double atan_poly64(double a)
+template <bool VGPR_COEF> __device__ __forceinline__ double fma_step(double p, double s, double c)
+{
+    if constexpr (VGPR_COEF)
+    {
+        double r;
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(s), "v"(c));
+        return r;
+    }
+    else
+        return fma(p, s, c);
+}
+template <bool V = false> __device__ __forceinline__ double atan_poly64(double a)
 {
     const double s = a * a;
     double p = -4.7926633120228785553e-5;
-    p = fma(p, s, 4.800660567800612957e-4);
-    if constexpr (SGPR_COEF)
-    {
-        asm("v_fma_f64 %0, %0, %1, %2\n\t"
-            "v_fma_f64 %0, %0, %1, %3\n\t"
-            "v_fma_f64 %0, %0, %1, %4\n\t"
-            "v_fma_f64 %0, %0, %1, %5\n\t"
-            "v_fma_f64 %0, %0, %1, %6\n\t"
-            "v_fma_f64 %0, %0, %1, %7\n\t"
-            "v_fma_f64 %0, %0, %1, %8\n\t"
-            "v_fma_f64 %0, %0, %1, %9\n\t"
-            "v_fma_f64 %0, %0, %1, %10\n\t"
-            "v_fma_f64 %0, %0, %1, %11\n\t"
-            "v_fma_f64 %0, %0, %1, %12\n\t"
-            "v_fma_f64 %0, %0, %1, %13\n\t"
-            "v_fma_f64 %0, %0, %1, %14\n\t"
-            "v_fma_f64 %0, %0, %1, %15\n\t"
-            "v_fma_f64 %0, %0, %1, %16"
-            : "+v"(p)
-            : "v"(s), "s"(-2.2725728333658927666e-3), "s"(6.8183912427924839848e-3),
-              "s"(-1.4739706399322470277e-2), "s"(2.4909137877934616446e-2), "s"(-3.5142229350564300719e-2),
-              "s"(4.3938991765738211806e-2), "s"(-5.1356486201903778769e-2), "s"(5.8483233451193392607e-2),
-              "s"(-6.6598275562737410628e-2), "s"(7.6913027337110721971e-2), "s"(-9.090805442522420044e-2),
-              "s"(1.1111104041852547122e-1), "s"(-1.4285713995249626285e-1), "s"(1.9999999993898812193e-1),
-              "s"(-3.3333333333288106455e-1));
-        return fma(a * s, p, a);
-    }
-    p = fma(p, s, -2.2725728333658927666e-3);
-    p = fma(p, s, 6.8183912427924839848e-3);
-    p = fma(p, s, -1.4739706399322470277e-2);
-    p = fma(p, s, 2.4909137877934616446e-2);
-    p = fma(p, s, -3.5142229350564300719e-2);
-    p = fma(p, s, 4.3938991765738211806e-2);
-    p = fma(p, s, -5.1356486201903778769e-2);
-    p = fma(p, s, 5.8483233451193392607e-2);
-    p = fma(p, s, -6.6598275562737410628e-2);
-    p = fma(p, s, 7.6913027337110721971e-2);
-    p = fma(p, s, -9.090805442522420044e-2);
-    p = fma(p, s, 1.1111104041852547122e-1);
-    p = fma(p, s, -1.4285713995249626285e-1);
-    p = fma(p, s, 1.9999999993898812193e-1);
-    p = fma(p, s, -3.3333333333288106455e-1);
+    p = fma_step<V>(p, s, 4.800660567800612957e-4);
+    p = fma_step<V>(p, s, -2.2725728333658927666e-3);
+    p = fma_step<V>(p, s, 6.8183912427924839848e-3);
+    p = fma_step<V>(p, s, -1.4739706399322470277e-2);
+    p = fma_step<V>(p, s, 2.4909137877934616446e-2);
+    p = fma_step<V>(p, s, -3.5142229350564300719e-2);
+    p = fma_step<V>(p, s, 4.3938991765738211806e-2);
+    p = fma_step<V>(p, s, -5.1356486201903778769e-2);
+    p = fma_step<V>(p, s, 5.8483233451193392607e-2);
+    p = fma_step<V>(p, s, -6.6598275562737410628e-2);
+    p = fma_step<V>(p, s, 7.6913027337110721971e-2);
+    p = fma_step<V>(p, s, -9.090805442522420044e-2);
+    p = fma_step<V>(p, s, 1.1111104041852547122e-1);
+    p = fma_step<V>(p, s, -1.4285713995249626285e-1);
+    p = fma_step<V>(p, s, 1.9999999993898812193e-1);
+    p = fma_step<V>(p, s, -3.3333333333288106455e-1);
     return fma(a * s, p, a);
 }
 
@@ -102,13 +87,14 @@ static __constant__ double kAtanTable[17] = {
     -5.1356486201903778769e-2, 5.8483233451193392607e-2, -6.6598275562737410628e-2, 7.6913027337110721971e-2,
     -9.090805442522420044e-2,  1.1111104041852547122e-1, -1.4285713995249626285e-1, 1.9999999993898812193e-1,
     -3.3333333333288106455e-1};
-__device__ __forceinline__ const double *atan_table()
+using AtanTable = const __attribute__((address_space(4))) double *; // constant memory: scalar loads
+__device__ __forceinline__ AtanTable atan_table()
 {
-    const double *t = kAtanTable;
+    AtanTable t = (AtanTable)kAtanTable;
     asm volatile("" : "+s"(t));
     return t;
 }
-__device__ __forceinline__ double atan_poly64_table(double a, const double *t)
+__device__ __forceinline__ double atan_poly64_table(double a, AtanTable t)
 {
     const double s = a * a;
     double p = t[0];
@@ -153,7 +139,7 @@ __device__ __forceinline__ double pvl_atan2(double y, double x)
 // atan2(-ay, x) for ay >= 0 (the segment's angle below: its sine is never positive), as
 // pvl_atan2 without the sign transfer.
 template <int COEF = 0>
-__device__ __forceinline__ double pvl_atan2_neg(double ay, double x, const double *table = nullptr)
+__device__ __forceinline__ double pvl_atan2_neg(double ay, double x, AtanTable table = nullptr)
 {
     const double ax = fabs(x);
     const double mn = fmin(ax, ay), mx = fmax(ax, ay);
@@ -199,7 +185,7 @@ __device__ __forceinline__ double pvl_rsqrt(double x)
 template <int PREC, int COEF = 0>
 __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double len, double d1x, double d1y,
                                          double d1z, double q1, double d2x, double d2y, double d2z, double q2,
-                                         double tol, double tol2, bool &cut, const double *table = nullptr)
+                                         double tol, double tol2, bool &cut, AtanTable table = nullptr)
 {
     const double t1 = ex * d1x + ey * d1y + ez * d1z;
     const double t2 = ex * d2x + ey * d2y + ez * d2z;
@@ -258,7 +244,7 @@ __device__ __forceinline__ double pair_m(double ex, double ey, double ez, double
 template <int PREC, int COEF = 0>
 __device__ __forceinline__ double cross_m(double ex, double ey, double ez, double len, double d1x, double d1y,
                                           double d1z, double tol2, double &cx, double &cy, double &cz, bool &cut,
-                                          const double *table = nullptr)
+                                          AtanTable table = nullptr)
 {
     cx = fma(d1y, ez, -(d1z * ey));
     cy = fma(d1z, ex, -(d1x * ez));
@@ -311,7 +297,7 @@ __device__ __forceinline__ double far_rcp(double b)
 }
 
 // Scalar factor of K (angle / h; the cut-off is decided here) and dr1 = p - r1.
-template <int PREC, int COEF = 0>
+template <int PREC>
 __device__ __forceinline__ double line_m(const LineGeom &g, double px, double py, double pz, double tol, double tol2,
                                          double &d1x, double &d1y, double &d1z, bool &cut)
 {
@@ -319,7 +305,7 @@ __device__ __forceinline__ double line_m(const LineGeom &g, double px, double py
     const double d2x = px - g.r2x, d2y = py - g.r2y, d2z = pz - g.r2z;
     const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
     const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
-    return pair_m<PREC, COEF>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2, tol, tol2, cut);
+    return pair_m<PREC>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2, tol, tol2, cut);
 }
 
 // K(line, p).  The reference form keeps the reference's cross product and products; the
@@ -352,9 +338,58 @@ __device__ __forceinline__ void line_k(const LineGeom &g, double px, double py, 
     }
 }
 
+// The far form for a line tested by itself, for points in no particular order (boxes are useless
+// there): from two lengths off the midpoint on B >= 3.75 len^2 and s <= 0.2845, over which the
+// degree-10 P has a relative error of 3.2e-16 (tools/fit_atan.py 10 double 0.2844).  Returns
+// angle / h (negative, as K's factor) from q = len / B and h^2.
+template <bool VGPR_COEF> __device__ __forceinline__ double mid_far(double q, double h2)
+{
+    const double u = (h2 * q) * q;
+    double p = -1.0530409925033454105e-2;
+    if constexpr (VGPR_COEF)
+    {
+        p = fma_step<true>(p, u, 2.9501554043661432491e-2);
+        p = fma_step<true>(p, u, -4.6025268387594494587e-2);
+        p = fma_step<true>(p, u, 5.7199422485590436944e-2);
+        p = fma_step<true>(p, u, -6.6394999569895820257e-2);
+        p = fma_step<true>(p, u, 7.6892308217604938091e-2);
+        p = fma_step<true>(p, u, -9.0906782661688777695e-2);
+        p = fma_step<true>(p, u, 1.1111100144380131558e-1);
+        p = fma_step<true>(p, u, -1.4285713981516674141e-1);
+        p = fma_step<true>(p, u, 1.9999999995777831413e-1);
+        p = fma_step<true>(p, u, -3.3333333333312912204e-1);
+    }
+    else
+        asm("v_fma_f64 %0, %0, %1, %2\n\t"
+            "v_fma_f64 %0, %0, %1, %3\n\t"
+            "v_fma_f64 %0, %0, %1, %4\n\t"
+            "v_fma_f64 %0, %0, %1, %5\n\t"
+            "v_fma_f64 %0, %0, %1, %6\n\t"
+            "v_fma_f64 %0, %0, %1, %7\n\t"
+            "v_fma_f64 %0, %0, %1, %8\n\t"
+            "v_fma_f64 %0, %0, %1, %9\n\t"
+            "v_fma_f64 %0, %0, %1, %10\n\t"
+            "v_fma_f64 %0, %0, %1, %11"
+            : "+v"(p)
+            : "v"(u), "s"(2.9501554043661432491e-2), "s"(-4.6025268387594494587e-2), "s"(5.7199422485590436944e-2),
+              "s"(-6.6394999569895820257e-2), "s"(7.6892308217604938091e-2), "s"(-9.0906782661688777695e-2),
+              "s"(1.1111100144380131558e-1), "s"(-1.4285713981516674141e-1), "s"(1.9999999995777831413e-1),
+              "s"(-3.3333333333312912204e-1));
+    return -fma(q * u, p, q);
+}
+
+// q = len / B also decides: 0 <= q len <= 1 / 3.75, as one unsigned comparison of the product's
+// upper word, which negative values, infinities and NaN fail.  A line cut by length has q = 0 and
+// adds 0.
+__device__ __forceinline__ bool mid_holds(double q, double len)
+{
+    return (unsigned)(__double_as_longlong(q * len) >> 32) < 0x3FD11111u; // upper word of 1 / 3.75
+}
+
 // n . K(line, p) for the normal-reduced assembly.  The reference form dots the reference's K
 // (reference rounding of every product); the others form m (n . c) with c = dr1 x e and the
-// dot as FMAs, and decide the cut-off once for the scalar.
+// dot as FMAs, decide the cut-off once for the scalar, and take the far form when it holds for all
+// points of the wave.
 template <int PREC>
 __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double py, double pz, double nx, double ny,
                                           double nz, double tol, double tol2)
@@ -367,24 +402,33 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     }
     else
     {
-        double d1x, d1y, d1z;
-        bool cut;
-        const double m = line_m<PREC, 1>(g, px, py, pz, tol, tol2, d1x, d1y, d1z, cut);
+        const double d1x = px - g.r1x, d1y = py - g.r1y, d1z = pz - g.r1z;
+        const double d2x = px - g.r2x, d2y = py - g.r2y, d2z = pz - g.r2z;
+        const double q = g.len * far_rcp(fma(d1x, d2x, fma(d1y, d2y, d1z * d2z)));
         const double cx = fma(d1y, g.ez, -(d1z * g.ey));
         const double cy = fma(d1z, g.ex, -(d1x * g.ez));
         const double cz = fma(d1x, g.ey, -(d1y * g.ex));
         const double nc = fma(cx, nx, fma(cy, ny, cz * nz));
-        return cut ? 0.0 : m * nc;
+        if (__builtin_amdgcn_ballot_w64(!mid_holds(q, g.len)) == 0)
+        {
+            const double h2 = fma(cx, cx, fma(cy, cy, cz * cz));
+            const double v = nc * mid_far<true>(q, h2);
+            return h2 < tol2 ? 0.0 : v;
+        }
+        const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
+        const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
+        bool cut;
+        const double v = nc * pair_m<PREC, 1>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2, tol, tol2,
+                                              cut);
+        return cut ? 0.0 : v;
     }
 }
 
 // The accurate forms of the point-velocity sums, from line records about the midpoint: m = p - mid,
 // c = m x e (= dr1 x e: K's direction, |c| = h), B = dr1 . dr2 = |m|^2 - len^2 / 4, three operations
 // fewer per pair than from the end points.  From two lengths off the midpoint on
-// (B >= far_b = 3.75 len^2, for all points of a wave) the far form above holds with s <= 0.2845 and a
-// degree-10 P (relative error 3.2e-16: tools/fit_atan.py 10 double 0.2844); points in no particular
-// order make boxes useless, and the test costs one comparison per line.  Otherwise the whole wave
-// takes the general form, from the line's own end points (its h^2 is the reference's, rounding
+// (B >= far_b = 3.75 len^2, for all points of a wave, one comparison per line) the far form above
+// holds.  Otherwise the whole wave takes the general form, from the line's own end points (its h^2 is the reference's, rounding
 // included, which is what separates the two near a line).  43 issue slots per far pair, against
 // ~102 of the general form.
 struct LineMid
@@ -397,30 +441,6 @@ struct LineMid
     double gamma; // the line's circulation (point-velocity sums)
 };
 static_assert(sizeof(LineMid) == sizeof(LineGeom), "one scratch size for both records");
-
-// angle / h (negative, as K's factor).
-__device__ __forceinline__ double mid_far(double b, double h2, double len)
-{
-    const double q = len * far_rcp(b);
-    const double u = (h2 * q) * q;
-    double p = -1.0530409925033454105e-2;
-    asm("v_fma_f64 %0, %0, %1, %2\n\t"
-        "v_fma_f64 %0, %0, %1, %3\n\t"
-        "v_fma_f64 %0, %0, %1, %4\n\t"
-        "v_fma_f64 %0, %0, %1, %5\n\t"
-        "v_fma_f64 %0, %0, %1, %6\n\t"
-        "v_fma_f64 %0, %0, %1, %7\n\t"
-        "v_fma_f64 %0, %0, %1, %8\n\t"
-        "v_fma_f64 %0, %0, %1, %9\n\t"
-        "v_fma_f64 %0, %0, %1, %10\n\t"
-        "v_fma_f64 %0, %0, %1, %11"
-        : "+v"(p)
-        : "v"(u), "s"(2.9501554043661432491e-2), "s"(-4.6025268387594494587e-2), "s"(5.7199422485590436944e-2),
-          "s"(-6.6394999569895820257e-2), "s"(7.6892308217604938091e-2), "s"(-9.0906782661688777695e-2),
-          "s"(1.1111100144380131558e-1), "s"(-1.4285713981516674141e-1), "s"(1.9999999995777831413e-1),
-          "s"(-3.3333333333312912204e-1));
-    return -fma(q * u, p, q);
-}
 
 // v[j] += gamma K(line, p[j]): the point-velocity inner step.  The non-reference forms scale once
 // and accumulate with FMAs.
@@ -464,13 +484,13 @@ __device__ __forceinline__ void line_k_acc(const LineMid &g, const uint32_t *ab,
         for (int j = 0; j < PPL; ++j)
         {
             const double h2 = fma(cx[j], cx[j], fma(cy[j], cy[j], cz[j] * cz[j]));
-            const double f = g.gamma * mid_far(b[j], h2, g.len);
+            const double f = g.gamma * mid_far<false>(g.len * far_rcp(b[j]), h2);
             w[j] = h2 < tol2 ? 0.0 : f;
         }
     }
     else
     {
-        const double *table = PREC == PVL_FP64 ? atan_table() : nullptr;
+        AtanTable table = PREC == PVL_FP64 ? atan_table() : nullptr;
         const double *r1 = pos + 3 * (size_t)(ab[0] & pvl::kInvalidId), *r2 = pos + 3 * (size_t)(ab[1] & pvl::kInvalidId);
 #pragma unroll
         for (int j = 0; j < PPL; ++j)

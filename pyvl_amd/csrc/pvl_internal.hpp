@@ -241,8 +241,7 @@ namespace pvl
 // The assembly (induction_matrix3) walks its surfaces in groups of kAsmSurfaces consecutive
 // surfaces (group g: surfaces 8g .. 8g + 7) and its groups in runs of up to kAsmGroups, one
 // run per wave; a run's groups are chosen by shared lines (on a structured body: the same
-// columns of kAsmGroups neighbouring rows), so that most lines of a run serve two of its
-// surfaces.  Inside a run each line's n . K is evaluated once and kept in one of kAsmSlots
+// columns of neighbouring rows), so that most lines of a run serve two of its surfaces.  Inside a run each line's n . K is evaluated once and kept in one of kAsmSlots
 // per-lane LDS slots while a later surface of the run still needs it.  The program lists,
 // per run, group by group and in CSR order, one entry per surface line: word 0 the line with
 // the orientation bit, word 1 the operation (kAsmEval / kAsmEvalStore / kAsmLoad / kAsmNone,
@@ -253,6 +252,18 @@ namespace pvl
 constexpr unsigned kAsmSurfaces = 8;
 constexpr unsigned kAsmGroups = 4;
 constexpr unsigned kAsmSlots = 10;
+// Long runs evaluate fewer lines (2.4 per quadrilateral with four groups, 2.6 with two, 3.1 with one),
+// short ones give more waves, and a wave with few others beside it waits out every evaluation's
+// latency (~0.5 us).  So the longest runs that give four waves per SIMD (4,096) with a control point
+// per surface: four groups from about 2,900 surfaces, two from 2,048, else one.  Measured with 4 / 2 / 1
+// groups: the whole matrix of 2,048 surfaces 49 / 40 / 46 us, of 16,384 1.50 / 1.58 / 1.78 ms, the
+// steady solve of 64 surfaces 160 / 144 / 132 us.
+constexpr unsigned assembly_groups_per_run(unsigned n_surfaces)
+{
+    const unsigned long long groups = (n_surfaces + 7ull) / kAsmSurfaces, points = (n_surfaces + 63ull) / 64;
+    return groups * points >= 4 * 4096 ? 4 : groups * points >= 2 * 4096 ? 2 : 1;
+}
+static_assert(assembly_groups_per_run(0xFFFFFFFFu) == kAsmGroups, "longest run");
 constexpr uint32_t kAsmEval = 0, kAsmEvalStore = 1, kAsmLoad = 2, kAsmNone = 3, kAsmEnd = 1u << 8;
 constexpr uint32_t kAsmNoGroup = 0xFFFFFFFFu;
 void build_assembly_program(unsigned n_surfaces, const uint32_t *offsets, const uint32_t *entries,

@@ -217,7 +217,8 @@ void pvl::build_assembly_program(unsigned n_surfaces, const uint32_t *offsets, c
                 it->second.second = g;
         }
     // runs: from the first unassigned group, repeatedly the unassigned group sharing the most
-    // lines with the run's last group (ties: the lowest index), up to kAsmGroups
+    // lines with the run's last group (ties: the lowest index), up to per_run
+    const unsigned per_run = assembly_groups_per_run(n_surfaces);
     std::vector<char> assigned(n_groups, 0);
     std::vector<uint32_t> runs; // kAsmGroups entries per run
     std::unordered_map<uint32_t, unsigned> shared;
@@ -229,7 +230,7 @@ void pvl::build_assembly_program(unsigned n_surfaces, const uint32_t *offsets, c
         unsigned nr = 0;
         run[nr++] = g0;
         assigned[g0] = 1;
-        while (nr < kAsmGroups)
+        while (nr < per_run)
         {
             shared.clear();
             const uint32_t last = run[nr - 1];

@@ -99,3 +99,18 @@ def test_noalloc_holds_meshes_near_its_scratch_limit():
                                               pts.cptr, v.cptr, C.c_int(0), C.c_int(_lib.PVL_FP64)), name)
         out.append(v.numpy())
     assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n_span,n_chord", [(1, 1), (9, 7), (64, 31), (32, 64), (59, 50)])
+def test_assembly_at_every_run_length(n_span, n_chord):
+    """The normal-reduced matrix on both sides of the surface counts where the groups per wave change
+    (2,048 and about 2,900), a single surface, and a last group that is not full."""
+    rng = np.random.default_rng(n_span)
+    pos, el, _ = G.flat_wing(n_span, n_chord, 8.0, 1.0)
+    pos[:, 2] += 0.1 * np.sin(3.0 * pos[:, 0]) + 0.002 * rng.normal(size=pos.shape[0])
+    m, t = Mesh(pos.shape[0], el), O.mesh_from_elements(pos.shape[0], el)
+    nrm, cps = O.surface_normal(t, pos), O.surface_center(t, pos)
+    rows = rng.permutation(m.n_surfaces)[:200]
+    c, n = np.ascontiguousarray(cps[rows]), np.ascontiguousarray(nrm[rows])
+    got, want = m.induction_matrix3(1e-6, pos, c, n), O.induction_matrix3(t, pos, c, n, 1e-6)
+    assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
