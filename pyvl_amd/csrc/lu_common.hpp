@@ -61,6 +61,18 @@ __device__ __forceinline__ unsigned wave_min_u32(unsigned v)
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+// max over the wave of a 32-bit unsigned value, in every lane.
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
+{
+    v = max(v, dpp_u32<0x111, 0xF>(0u, v));
+    v = max(v, dpp_u32<0x112, 0xF>(0u, v));
+    v = max(v, dpp_u32<0x114, 0xF>(0u, v));
+    v = max(v, dpp_u32<0x118, 0xF>(0u, v));
+    v = max(v, dpp_u32<0x142, 0xA>(0u, v));
+    v = max(v, dpp_u32<0x143, 0xC>(0u, v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
 // Order-preserving key of a pivot candidate: the bits of |a| (monotonic for non-negative
 // doubles); NaN maps to 0 and never wins (its row is excluded from the tie-break below).
 __device__ __forceinline__ unsigned long long pivot_key(double v)
@@ -72,8 +84,19 @@ __device__ __forceinline__ unsigned long long pivot_key(double v)
 // Wave-wide idamax over (key, row) pairs: the largest key, then the smallest row among the
 // lanes holding it (rows of excluded candidates are 0xFFFFFFFF).  Returns the row (or
 // 0xFFFFFFFF if no lane has a candidate) and the key through *kmax.
+// The keys' upper words decide unless two lanes share the largest: one chain of six 32-bit steps, where
+// the 64-bit maximum and the rows' minimum are a chain of some seventy dependent instructions, twice
+// per column of a panel.
 __device__ __forceinline__ unsigned wave_argmax(unsigned long long key, unsigned row, unsigned long long *kmax)
 {
+    const unsigned hi = (unsigned)(key >> 32), mh = wave_max_u32(hi);
+    const unsigned long long who = __builtin_amdgcn_ballot_w64(hi == mh);
+    if ((who & (who - 1)) == 0)
+    {
+        const int l = (int)__builtin_ctzll(who);
+        *kmax = ((unsigned long long)mh << 32) | (unsigned)__builtin_amdgcn_readlane((unsigned)key, l);
+        return __builtin_amdgcn_readlane(row, l);
+    }
     const unsigned long long m = wave_max_u64(key);
     *kmax = m;
     return wave_min_u32(key == m ? row : 0xFFFFFFFFu);
