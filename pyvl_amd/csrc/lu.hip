@@ -108,14 +108,6 @@ __device__ __forceinline__ void xstore_u64(unsigned long long *p, unsigned long 
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ unsigned xload_u32(const unsigned *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void xstore_u32(unsigned *p, unsigned v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // Bounded waits: a wait that has not ended after kWaitTicks of the 100 MHz real-time
 // counter (or once another wave has flagged a timeout) gives up and flags *err.
@@ -129,30 +121,47 @@ __device__ __forceinline__ bool wait_expired(unsigned &spins, unsigned long long
 
 constexpr int kRecBytes = 256;
 
-// Exchange area for the panel kernel, double buffered by the parity of the exchange round
-// (one round per column).  There is no grid barrier: a group's record of a round is the
-// signal that its published rows of that round are complete, and every word of a record
-// carries a tag bit (bit 1 of the round number), so that a reader tells the record of this
-// round from the one two rounds earlier in the same buffer.  A group can run at most one
-// round ahead of the slowest (it needs every group's record of the round before), so two
-// buffers and one tag bit suffice.
-// Each record sits in a cache line of its own: every group polls every record, and records
-// packed into a few lines queue those loads (and the stores behind them) on one memory channel.
+// Exchange area for the panel kernel.  There is no grid barrier and no wait for a store to complete:
+// every 64-bit word carries 32 bits of payload and, above them, the tag of the round it belongs to
+// (the number of the column in the factorisation, from 1), so that a reader takes a word only when it
+// is of its round, whatever the order in which words arrive.  The area is cleared (tag 0) before a
+// factorisation.
+// A slot, one per group and parity of the round (a group can run at most one round ahead of the
+// slowest, as it needs every group's slot of the round before): the candidate's |a| (two words), its
+// panel position (all ones: none), its columns of the current sub-block.  Each slot in cache lines of its
+// own: every group polls every slot, and slots packed into a few lines queue those loads (and the
+// stores behind them) on one memory channel.
+constexpr int kPanelKB = 8; // columns of a sub-block
 struct alignas(kRecBytes) PanelSlot
 {
-    unsigned long long key; // bit 63: tag; bits 0-62: the candidate's |a| (double bits)
-    unsigned pos;           // bit 31: tag; bits 0-30: its panel position (INT_MAX: none)
+    unsigned long long w[32];
 };
-struct PanelRec
+struct PanelX
 {
     PanelSlot slot[2][kMaxGroups];
+    PanelSlot rowj[2]; // row j's columns of the current sub-block
+    // the rows that a sub-block's interchanges move, all columns: the rows that become its pivot rows,
+    // and the rows that stood there before
+    unsigned long long row[2][kPanelKB][NB][2];
 };
-template <typename T> struct PanelX
+template <typename T> constexpr int kHalves = sizeof(T) / 4; // words per value
+__device__ __forceinline__ void put_halves(unsigned *d, double v)
 {
-    PanelRec rec;
-    T crow[2][kMaxGroups][NB];
-    T rowj[2][NB];
-};
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    d[0] = (unsigned)u, d[1] = (unsigned)(u >> 32);
+}
+__device__ __forceinline__ void put_halves(unsigned *d, float v) { d[0] = __float_as_uint(v); }
+template <typename T> __device__ __forceinline__ T get_halves(const unsigned *d)
+{
+    if constexpr (sizeof(T) == 8)
+        return __longlong_as_double((long long)(((unsigned long long)d[1] << 32) | d[0]));
+    else
+        return __uint_as_float(d[0]);
+}
+template <int P> __device__ __forceinline__ unsigned quad_u32(unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)v, P * 0x55, 0xF, 0xF, true);
+}
 
 // ---------------------------------------------------------------------------------------
 // The panel's columns [c0, jb) of local rows [rb, nr) take a sub-block's update,
@@ -245,37 +254,59 @@ __device__ __forceinline__ void subblock_update(T *__restrict__ L, const T (*__r
 // ---------------------------------------------------------------------------------------
 // Panel factorisation of P (m x jb, row stride lda), rows k.. of the matrix.  Group g owns
 // panel positions g, g + G, g + 2G, ... (at most R of them).  Per column j: local argmax
-// over positions >= j; publish the candidate's row and the current row j, then the
-// candidate's record (|value|, position); read every group's record; every group picks the
+// over positions >= j; publish the candidate; read every group's; every group picks the
 // same winner (largest |a|, first position on ties: LAPACK idamax), swaps, scales by the
 // reciprocal pivot and applies the rank-1 update to its rows.
+// Bound by latency, 3.2 us per column: about 1.1 us the exchange (one trip through memory: only the
+// eight columns of the sub-block travel with the candidate, in tagged words that need no wait for a
+// store's completion, and the interchanges of the columns outside it are made once per sub-block), the
+// rest the chain of wave and workgroup reductions, the division and a sub-block's update.  A panel of 64
+// FP64 columns takes 210 us with 12 groups and 250 with 64 (240 and 270 with whole rows published, their
+// stores waited for and the winner's row fetched after its record; a factorisation of a random matrix,
+// where every column interchanges, 18.3 instead of 21.1 ms at n = 4,096 and 136 instead of 144 at 16,384).
 template <typename T>
 __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, int m, int jb, int R, int row_base,
-                                                    int *__restrict__ piv, PanelX<T> *__restrict__ X, unsigned base,
+                                                    int *__restrict__ piv, PanelX *__restrict__ X, unsigned base,
                                                     int *__restrict__ status)
 {
     main_stream_priority<2>();
     extern __shared__ __align__(16) unsigned char smem_raw[];
     constexpr int LDP = NB + 1;
+    constexpr int KB = kPanelKB, H = kHalves<T>, VW = KB * H; // words of a sub-block's row
+    constexpr int NK = (3 + VW + 3) / 4;                      // words of a slot per lane of a quad
+    constexpr unsigned NONE = 0xFFFFFFFFu;
     T *L = (T *)smem_raw;
-    __shared__ T prow[NB], srowj[NB], s_invj;
-    __shared__ double red_v[4];
-    __shared__ int red_p[4];
-    __shared__ int s_pos, s_grp;
+    __shared__ unsigned long long red_k[4];
+    __shared__ unsigned red_p[4];
+    __shared__ unsigned wsub[4][VW], rowj_sub[VW]; // each wave's candidate's sub-block columns; row j's, if owned
+    __shared__ unsigned long long win_k[4];        // the winner among the groups that a wave reads
+    __shared__ unsigned win_p[4], win_v[4][VW], srowj[VW]; // its position and columns; row j's columns
+    __shared__ int s_piv[KB]; // the sub-block's pivots
     // pivots collected in LDS and stored once at the end: a global store before a barrier
     // makes the barrier wait for it
     __shared__ int spiv[NB];
     int first_zero = 0;
 
     const int tid = threadIdx.x, g = blockIdx.x, G = gridDim.x;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     // rows dealt cyclically: group g holds panel positions g, g + G, g + 2G, ... (at most R),
     // so row j, its owner's extra publishing and the sub-block's pivot rows rotate over the
     // groups instead of all falling to the first
     const int nr = g < m ? (m - 1 - g) / G + 1 : 0;
-    for (int idx = tid; idx < nr * jb; idx += 256)
+    // position / G for positions below 2^16 (exact: the error of the product is below 2^-16 < 1 / G)
+    const unsigned magic = G > 1 ? (unsigned)((0x100000000ull + G - 1) / G) : 0u;
+    const auto local_row = [&](int position) { return G > 1 ? (int)__umulhi((unsigned)position, magic) : position; };
+    // a wave per row, a lane per column, sixteen loads in flight (one at a time they took 40 us)
+    for (int r0 = 0; r0 < nr; r0 += 64)
     {
-        const int r = idx / jb, c = idx - r * jb;
-        L[r * LDP + c] = P[(size_t)(g + r * G) * lda + c];
+        T x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            x[k] = P[(size_t)(g + min(r0 + w + 4 * k, nr - 1) * G) * lda + min(lane, jb - 1)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            if (r0 + w + 4 * k < nr && lane < jb)
+                L[(r0 + w + 4 * k) * LDP + lane] = x[k];
     }
     __syncthreads();
 
@@ -284,12 +315,8 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
     // updated once per sub-block from the sub-block's pivot rows (U12 of the sub-block,
     // formed by every group from the published pivot rows) -- per element the same FMAs in the
     // same order as the column-by-column sweep, so factors and pivots are unchanged, with an
-    // eighth of the LDS traffic.  Rows published for the exchange carry the sub-block's
-    // columns from registers and the columns right of it as they stand (not yet updated by the
-    // sub-block): every consumer (the interchange, U12) treats them the same way.
-    constexpr int KB = 8;
+    // eighth of the LDS traffic.
     __shared__ T ucur[KB][NB]; // the sub-block's pivot rows as published, then U12 in place
-    __shared__ T wsub[4][KB], rowj_sub[KB]; // each wave's candidate's sub-block columns; row j's
     const int r = tid; // this thread's row (R <= 256 rows per group)
     const bool has_row = r < nr;
     const int pos = g + r * G;
@@ -301,95 +328,149 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
         for (int t = 0; t < KB; ++t)
             v[t] = (has_row && t < kb) ? L[r * LDP + j0 + t] : T(0);
         unsigned zm = 0; // bit t: column j0 + t had an exactly-zero pivot (no update applied)
-#pragma unroll
-        for (int t = 0; t < KB; ++t)
+        unsigned tag = 0;
+        int owner_j = j0 - local_row(j0) * G; // the group owning row j
+        // A rotating window: at step t slot i holds column j0 + (t + i) % KB, so the steps are one loop's
+        // body with static register indexes (unrolled: 62 KB of code, no faster).
+#pragma unroll 1
+        for (int t = 0; t < kb; ++t)
         {
-            if (t >= kb)
-                break;
             const int j = j0 + t;
-            const unsigned rnd = base + (unsigned)j; // exchange round
-            const int par = (int)(rnd & 1u);
-            const unsigned tagbit = (rnd >> 1) & 1u;
-            const unsigned long long ktag = (unsigned long long)tagbit << 63;
-            const unsigned ptag = tagbit << 31;
+            tag = base + (unsigned)j + 1u;
+            const int par = (int)(tag & 1u);
+            const unsigned long long tagged = (unsigned long long)tag << 32;
             // 1. local candidate: per lane, then over the wave (DPP moves), then over the waves;
             // each wave's winner stages its sub-block columns beside the wave's record, and the
             // owner of row j its own, before the one barrier
-            const int oj = j % G; // the group owning row j
-            const bool own_j = g == oj;
+            const bool own_j = g == owner_j;
+            owner_j = owner_j + 1 == G ? 0 : owner_j + 1;
             {
                 unsigned long long key = 0;
-                unsigned row = 0xFFFFFFFFu;
+                unsigned row = NONE;
                 if (has_row && pos >= j)
                 {
-                    const double vv = fabs((double)v[t]);
+                    const double vv = fabs((double)v[0]);
                     if (vv == vv)
                         key = pivot_key(vv), row = (unsigned)pos;
                 }
                 unsigned long long km;
                 const unsigned wrow = wave_argmax(key, row, &km);
-                if ((tid & 63) == 0)
-                {
-                    const bool none = wrow == 0xFFFFFFFFu;
-                    red_v[tid >> 6] = none ? -1.0 : __longlong_as_double((long long)km);
-                    red_p[tid >> 6] = none ? INT_MAX : (int)wrow;
-                }
+                if (lane == 0)
+                    red_k[w] = km, red_p[w] = wrow; // no candidate: key 0, position NONE
                 if (has_row && (unsigned)pos == wrow)
                 {
 #pragma unroll
                     for (int i = 0; i < KB; ++i)
-                        wsub[tid >> 6][i] = v[i];
+                        put_halves(&wsub[w][i * H], v[i]);
                 }
             }
             if (has_row && pos == j)
             {
 #pragma unroll
                 for (int i = 0; i < KB; ++i)
-                    rowj_sub[i] = v[i];
+                    put_halves(&rowj_sub[i * H], v[i]);
             }
             __syncthreads();
-            double bv = red_v[0];
-            int bp = red_p[0], bw = 0;
-            for (int w = 1; w < 4; ++w)
-                if (better(red_v[w], red_p[w], bv, bp))
-                    bv = red_v[w], bp = red_p[w], bw = w;
-            // 2. publish the candidate's row and row j (if owned); once those stores are
-            // complete, the tagged record that signals them
-            // (a candidate that is row j itself is not published twice: readers take row j)
-            if (bp != INT_MAX && bp != j)
-                for (int c = tid; c < jb; c += 256)
-                    xstore(&X->crow[par][g][c],
-                           (c >= j0 && c < j0 + kb) ? wsub[bw][c - j0] : L[(bp / G) * LDP + c]);
-            if (own_j)
-                for (int c = tid; c < jb; c += 256)
-                    xstore(&X->rowj[par][c], (c >= j0 && c < j0 + kb) ? rowj_sub[c - j0] : L[(j / G) * LDP + c]);
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (tid == 0)
+            // 2. publish the candidate and, if owned, row j
             {
-                xstore_u64(&X->rec.slot[par][g].key,
-                           (bp == INT_MAX ? 0ull : (unsigned long long)__double_as_longlong(bv)) | ktag);
-                xstore_u32(&X->rec.slot[par][g].pos, (unsigned)bp | ptag);
+                // (all four records in one batch of LDS reads, compared without branches)
+                unsigned long long k4[4];
+                unsigned p4[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    k4[q] = red_k[q], p4[q] = red_p[q];
+                unsigned long long kv = k4[0];
+                unsigned bp = p4[0];
+                int bw = 0;
+#pragma unroll
+                for (int q = 1; q < 4; ++q)
+                {
+                    const bool take = (k4[q] > kv) | ((k4[q] == kv) & (p4[q] < bp));
+                    kv = take ? k4[q] : kv, bp = take ? p4[q] : bp, bw = take ? q : bw;
+                }
+                if (tid < 4 * NK)
+                {
+                    const unsigned x = tid == 0   ? (unsigned)kv
+                                       : tid == 1 ? (unsigned)(kv >> 32)
+                                       : tid == 2 ? bp
+                                                  : (tid < 3 + VW ? wsub[bw][min(tid - 3, VW - 1)] : 0u);
+                    xstore_u64(&X->slot[par][g].w[tid], tagged | x);
+                }
+                else if (own_j && tid >= 64 && tid < 64 + VW)
+                    xstore_u64(&X->rowj[par].w[tid - 64], tagged | rowj_sub[tid - 64]);
             }
-            // 3. every group's record of this round (wave 0, a group per lane) and the winner,
-            // identical in every group; wave 1 fetches row j as soon as its owner's record is
-            // in -- it is the pivot row whenever no interchange is due (the usual case)
-            if (tid < 64)
+            // 3. every group's candidate: a quad of lanes per slot, sixteen slots per wave, and the
+            // winner among them; the last wave row j's columns as well
             {
                 unsigned long long key = 0;
-                unsigned row = 0xFFFFFFFFu;
-                int bq = 0;
-                for (int q = tid; q < G; q += 64)
+                unsigned row = NONE;
+                unsigned pay[NK];
+#pragma unroll
+                for (int k = 0; k < NK; ++k)
+                    pay[k] = 0u;
+                for (int q = 16 * w + (lane >> 2); q < G; q += 64)
                 {
-                    unsigned long long kw;
-                    unsigned pw;
+                    const unsigned long long *slot = &X->slot[par][q].w[lane & 3];
+                    unsigned long long x[NK];
+                    unsigned spins = 0;
+                    bool late = false;
+                    const unsigned long long t0 = wall_clock64();
+                    for (;;)
+                    {
+                        bool ok = true;
+#pragma unroll
+                        for (int k = 0; k < NK; ++k)
+                            x[k] = xload_u64(slot + 4 * k);
+#pragma unroll
+                        for (int k = 0; k < NK; ++k)
+                            ok = ok && (unsigned)(x[k] >> 32) == tag;
+                        if (ok)
+                            break;
+                        if (wait_expired(spins, t0, &status[1]))
+                        {
+                            xstore_i(&status[1], 1);
+                            late = true;
+                            break;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    // a slot that came too late holds no candidate (the call fails)
+                    const unsigned head = (unsigned)x[0];
+                    const bool any_late = (quad_u32<0>(late) | quad_u32<1>(late) | quad_u32<2>(late) | quad_u32<3>(late)) != 0;
+                    const unsigned long long kk = ((unsigned long long)quad_u32<1>(head) << 32) | quad_u32<0>(head);
+                    const unsigned qp = any_late ? NONE : quad_u32<2>(head);
+                    if ((qp != NONE) & ((kk > key) | ((kk == key) & (qp < row))))
+                    {
+                        key = kk, row = qp;
+#pragma unroll
+                        for (int k = 0; k < NK; ++k)
+                            pay[k] = (unsigned)x[k];
+                    }
+                }
+                unsigned long long km;
+                const bool first = (lane & 3) == 0;
+                const unsigned wrow = wave_argmax(first ? key : 0ull, first ? row : NONE, &km);
+                if (lane == 0)
+                    win_k[w] = km, win_p[w] = wrow;
+                if (row == wrow && wrow != NONE)
+                {
+#pragma unroll
+                    for (int k = 0; k < NK; ++k)
+                    {
+                        const int i = (lane & 3) + 4 * k - 3;
+                        if (i >= 0 && i < VW)
+                            win_v[w][i] = pay[k];
+                    }
+                }
+                if (w == 3 && lane < VW)
+                {
+                    unsigned long long x;
                     unsigned spins = 0;
                     const unsigned long long t0 = wall_clock64();
                     for (;;)
                     {
-                        kw = xload_u64(&X->rec.slot[par][q].key);
-                        pw = xload_u32(&X->rec.slot[par][q].pos);
-                        if ((kw >> 63) == (ktag >> 63) && (pw >> 31) == (ptag >> 31))
+                        x = xload_u64(&X->rowj[par].w[lane]);
+                        if ((unsigned)(x >> 32) == tag)
                             break;
                         if (wait_expired(spins, t0, &status[1]))
                         {
@@ -398,115 +479,82 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
                         }
                         __builtin_amdgcn_s_sleep(1);
                     }
-                    const unsigned long long kk = kw & ~(1ull << 63);
-                    const unsigned qp = pw & 0x7FFFFFFFu;
-                    if (qp != (unsigned)INT_MAX && (kk > key || (kk == key && qp < row)))
-                        key = kk, row = qp, bq = q;
-                }
-                unsigned long long km;
-                const unsigned wrow = wave_argmax(key, row, &km);
-                const unsigned long long who = __ballot(wrow != 0xFFFFFFFFu && row == wrow);
-                const int wl = who ? (int)__builtin_ctzll(who) : 0;
-                const int wgq = __builtin_amdgcn_readlane(bq, wl);
-                if (tid == 0)
-                    s_pos = wrow == 0xFFFFFFFFu ? INT_MAX : (int)wrow, s_grp = wgq;
-            }
-            else if (tid < 128)
-            {
-                unsigned pw;
-                unsigned spins = 0;
-                const unsigned long long t0 = wall_clock64();
-                for (;;)
-                {
-                    pw = xload_u32(&X->rec.slot[par][oj].pos);
-                    if ((pw >> 31) == (ptag >> 31))
-                        break;
-                    if (wait_expired(spins, t0, &status[1]))
-                    {
-                        xstore_i(&status[1], 1);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-                if (tid - 64 < jb)
-                {
-                    const T rj = xload(&X->rowj[par][tid - 64]);
-                    srowj[tid - 64] = rj;
-                    // the reciprocal of row j's diagonal, ready for the usual case that row j
-                    // is the pivot row (the division runs while wave 0 still polls)
-                    if (tid - 64 == j)
-                        s_invj = rj != T(0) ? T(1) / rj : T(0);
+                    srowj[lane] = (unsigned)x;
                 }
             }
             __syncthreads();
-            int p = s_pos;
-            const int wg = s_grp;
-            const bool none = (p == INT_MAX); // every candidate NaN: keep row j in place
-            if (none)
-                p = j;
-            // the pivot row: row j itself when p == j (its owner does not publish it as a
-            // candidate), else the winner's published row
-            const T *prow_p = srowj;
-            if (p != j)
+            // 4. the winner of all groups, identical in every group
+            unsigned long long k4[4];
+            unsigned p4[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                k4[q] = win_k[q], p4[q] = win_p[q];
+            unsigned long long bk = k4[0];
+            unsigned bp = p4[0];
+            int bw = 0;
+#pragma unroll
+            for (int q = 1; q < 4; ++q)
             {
-                for (int c = tid; c < jb; c += 256)
-                    prow[c] = xload(&X->crow[par][wg][c]);
-                __syncthreads();
-                prow_p = prow;
+                const bool take = (k4[q] > bk) | ((k4[q] == bk) & (p4[q] < bp));
+                bk = take ? k4[q] : bk, bp = take ? p4[q] : bp, bw = take ? q : bw;
             }
-            // 5. interchange: LDS rows outside the sub-block, the owners' registers inside
-            const bool own_p = p % G == g;
-            if (p != j)
+            const bool none = bp == NONE; // every candidate NaN: keep row j in place
+            const int p = none ? j : (int)bp;
+            const unsigned *uw = none ? srowj : win_v[bw];
+            T u[KB];
+#pragma unroll
+            for (int i = 0; i < KB; ++i)
+                u[i] = get_halves<T>(&uw[i * H]);
+            // 5. interchange of the sub-block's columns, in the owners' registers
+            if (p != j && has_row)
             {
-                if (own_j)
-                    for (int c = tid; c < jb; c += 256)
-                        if (c < j0 || c >= j0 + kb)
-                            L[(j / G) * LDP + c] = prow_p[c];
-                if (own_p)
-                    for (int c = tid; c < jb; c += 256)
-                        if (c < j0 || c >= j0 + kb)
-                            L[(p / G) * LDP + c] = srowj[c];
-                if (has_row && pos == j)
+                if (pos == j)
                 {
 #pragma unroll
                     for (int i = 0; i < KB; ++i)
-                        v[i] = (i < kb) ? prow_p[j0 + i] : v[i];
+                        v[i] = u[i];
                 }
-                else if (has_row && pos == p)
+                else if (pos == p)
                 {
 #pragma unroll
                     for (int i = 0; i < KB; ++i)
-                        v[i] = (i < kb) ? srowj[j0 + i] : v[i];
+                        v[i] = get_halves<T>(&srowj[i * H]);
                 }
             }
-            for (int c = tid; c < jb; c += 256)
-                ucur[t][c] = prow_p[c];
+            if (tid < KB && ((t + tid) & (KB - 1)) < kb)
+                ucur[t][j0 + ((t + tid) & (KB - 1))] = get_halves<T>(&uw[tid * H]);
             if (tid == 0)
-                spiv[j] = row_base + p; // global store deferred: see the end of the kernel
+                spiv[j] = row_base + p, s_piv[t] = p; // global store deferred: see the end of the kernel
             // 6. scale by the reciprocal pivot and update the sub-block's columns (registers)
-            const T pv = prow_p[j];
-            if (pv != T(0))
-            {
-                const T inv = p == j ? s_invj : T(1) / pv;
-                if (has_row && pos > j)
-                {
-                    const T l = v[t] * inv;
-                    v[t] = l;
+            const T pv = u[0];
+            const bool zero = !(pv != T(0));
+            const bool below = has_row && pos > j && !zero;
+            const T l = below ? v[0] * (T(1) / pv) : v[0];
 #pragma unroll
-                    for (int t2 = t + 1; t2 < KB; ++t2)
-                        if (t2 < kb)
-                            v[t2] = fma(-l, prow_p[j0 + t2], v[t2]);
-                }
+            for (int i = 1; i < KB; ++i)
+            {
+                const T x = fma(-l, u[i], v[i]);
+                v[i - 1] = below && t + i < kb ? x : v[i];
             }
-            else
+            v[KB - 1] = l;
+            if (zero)
             {
                 zm |= 1u << t;
                 if (tid == 0 && first_zero == 0)
                     first_zero = row_base + j + 1; // first exactly-zero pivot (1-based global column)
             }
         }
-        // 7. the sub-block's columns back to LDS; U12 of the sub-block for the columns right
-        // of it, pivot row by pivot row in elimination order
+        for (int t = kb; t < KB; ++t) // back to slot i = column i
+        {
+            const T first = v[0];
+#pragma unroll
+            for (int i = 1; i < KB; ++i)
+                v[i - 1] = v[i];
+            v[KB - 1] = first;
+        }
+        // 7. the sub-block's columns back to LDS, and its interchanges as one permutation, in every wave:
+        // lane t < KB stands for position j0 + t, the lanes above for the positions below the sub-block
+        // whose rows go up (each becomes one pivot row); at[.] is the row now at a lane's position
         if (has_row)
         {
 #pragma unroll
@@ -515,6 +563,118 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
                     L[r * LDP + j0 + t] = v[t];
         }
         __syncthreads();
+        int where = lane < kb ? j0 + lane : -1, at = where;
+        {
+            const int piv_l = s_piv[lane & (KB - 1)];
+            int free_lane = KB;
+            for (int t = 0; t < kb; ++t)
+            {
+                const int p = __builtin_amdgcn_readlane(piv_l, t);
+                const unsigned long long found = __builtin_amdgcn_ballot_w64(where == p);
+                int x = free_lane;
+                if (found)
+                    x = (int)__builtin_ctzll(found);
+                else
+                {
+                    ++free_lane;
+                    if (lane == x)
+                        where = p, at = p;
+                }
+                const int a = __builtin_amdgcn_readlane(at, t), b = __builtin_amdgcn_readlane(at, x);
+                at = lane == x ? a : at;
+                at = lane == t ? b : at;
+            }
+        }
+        // The rows that move, published by their owners (columns outside the sub-block, a lane each), and
+        // read back: the pivot rows right of the sub-block by every group, left of it by their new
+        // owners, and the displaced rows by theirs.  Wave w handles pivot rows w and w + 4: the row that
+        // becomes one and the row that takes that one's place, so that what a wave overwrites it has
+        // itself published.
+        const unsigned long long rtag = (unsigned long long)tag << 32;
+        const bool outside = lane < jb && (lane < j0 || lane >= j0 + kb);
+        const auto publish = [&](unsigned long long *dst, int row) {
+            if (outside)
+            {
+                unsigned h[2];
+                put_halves(h, L[row * LDP + lane]);
+#pragma unroll
+                for (int i = 0; i < H; ++i)
+                    xstore_u64(dst + i, rtag | h[i]);
+            }
+        };
+        {
+            const unsigned long long *src[4];
+            bool need[4];
+            int dst[4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+            {
+                const int t = w + 4 * i;
+                need[i] = need[2 + i] = false;
+                src[i] = src[2 + i] = &X->row[0][t][lane][0];
+                dst[i] = dst[2 + i] = 0;
+                if (t < kb) // uniform
+                {
+                    const int from = __builtin_amdgcn_readlane(at, t); // becomes pivot row t
+                    const int fr = local_row(from), tr = local_row(j0 + t);
+                    const bool own_from = from == fr * G + g, own_t = j0 + t == tr * G + g;
+                    if (own_from)
+                        publish(&X->row[0][t][lane][0], fr);
+                    if (own_t && from != j0 + t)
+                        publish(&X->row[1][t][lane][0], tr);
+                    need[i] = outside && (lane >= j0 + kb || (own_t && from != j0 + t));
+                    dst[i] = tr;
+                    if (own_from && from >= j0 + kb) // its place is taken by a row of the sub-block
+                    {
+                        const int x = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(lane >= KB && where == from));
+                        need[2 + i] = outside;
+                        src[2 + i] = &X->row[1][__builtin_amdgcn_readlane(at, x) - j0][lane][0];
+                        dst[2 + i] = fr;
+                    }
+                }
+            }
+            unsigned long long x[4][H];
+            unsigned spins = 0;
+            const unsigned long long t0 = wall_clock64();
+            for (;;)
+            {
+                bool ok = true;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int h = 0; h < H; ++h)
+                        x[i][h] = need[i] ? xload_u64(src[i] + h) : rtag;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int h = 0; h < H; ++h)
+                        ok = ok & ((unsigned)(x[i][h] >> 32) == tag);
+                if (ok)
+                    break;
+                if (wait_expired(spins, t0, &status[1]))
+                {
+                    xstore_i(&status[1], 1);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                unsigned hv[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+                    hv[h] = (unsigned)x[i][h];
+                const T val = get_halves<T>(hv);
+                if (need[i] && i < 2 && lane >= j0 + kb)
+                    ucur[w + 4 * i][lane] = val;
+                else if (need[i])
+                    L[dst[i] * LDP + lane] = val;
+            }
+        }
+        __syncthreads();
+        // 8. U12 of the sub-block for the columns right of it, pivot row by pivot row in elimination
+        // order
         for (int c = j0 + kb + tid; c < jb; c += 256)
         {
             T u[KB];
@@ -534,7 +694,7 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
             }
         }
         __syncthreads();
-        // 8. the columns right of the sub-block: rows below its pivots take its kb updates,
+        // 9. the columns right of the sub-block: rows below its pivots take its kb updates,
         // its pivot rows their U12 rows
         if (j0 + kb < jb)
         {
@@ -569,10 +729,11 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
         if (tid == 0 && first_zero)
             atomicCAS(&status[0], 0, first_zero); // LAPACK info
     }
-    for (int idx = tid; idx < nr * jb; idx += 256)
+    if (lane < jb)
     {
-        const int r = idx / jb, c = idx - r * jb;
-        P[(size_t)(g + r * G) * lda + c] = L[r * LDP + c];
+#pragma unroll 8
+        for (int r = w; r < nr; r += 4)
+            P[(size_t)(g + r * G) * lda + lane] = L[r * LDP + lane];
     }
 }
 
@@ -1980,17 +2141,14 @@ rocblas_handle g_blas = nullptr;
 volatile int *g_status_host = nullptr;
 int *g_status_host_dev = nullptr;
 
-__global__ void factor_reset_kernel(PanelRec *__restrict__ rec, int *__restrict__ status)
+// Clears the status words and, for a factorisation with grouped panels, the exchange area's tags.
+__global__ void __launch_bounds__(256) factor_reset_kernel(unsigned long long *__restrict__ x, size_t words,
+                                                           int *__restrict__ status)
 {
     main_stream_priority();
-    // records tagged 1: never taken for rounds 0 and 1 (tag 0), and overwritten before the
-    // rounds with tag 1 (2 and 3) read them
-    for (int i = threadIdx.x; i < 2 * kMaxGroups; i += blockDim.x)
-    {
-        (&rec->slot[0][0])[i].key = 1ull << 63;
-        (&rec->slot[0][0])[i].pos = 1u << 31;
-    }
-    if (threadIdx.x == 0)
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < words; i += gridDim.x * (size_t)256)
+        x[i] = 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
     {
         status[0] = 0;        // first zero pivot
         status[1] = 0;        // a bounded wait timed out
@@ -2027,7 +2185,7 @@ int ensure_ws()
 {
     if (!g_ws.panelx)
     {
-        PVL_HIP(hipMalloc(&g_ws.panelx, sizeof(PanelX<double>)));
+        PVL_HIP(hipMalloc(&g_ws.panelx, sizeof(PanelX)));
         PVL_HIP(hipMalloc(&g_ws.err, 8 * sizeof(int)));
         PVL_HIP(hipMemset(g_ws.err, 0, 8 * sizeof(int)));
         void *h = nullptr;
@@ -2143,9 +2301,11 @@ template <typename T> int factor_impl(int n, T *A, int *piv, int *info_out, bool
                                     (int)(sizeof(T) * nopiv_lds_elems())));
         attr_set[sizeof(T) == 8] = true;
     }
-    PanelX<T> *X = (PanelX<T> *)g_ws.panelx;
+    PanelX *X = (PanelX *)g_ws.panelx;
     int *status = g_ws.err;
-    factor_reset_kernel<<<1, 256, 0, stream()>>>(&X->rec, status);
+    const bool grouped = pivoting && n > panel_wg_rows(sizeof(T));
+    const size_t words = grouped ? sizeof(PanelX) / sizeof(unsigned long long) : 0;
+    factor_reset_kernel<<<grouped ? 64 : 1, 256, 0, stream()>>>((unsigned long long *)X, words, status);
     PVL_HIP(hipGetLastError());
     unsigned base = 0;
     // Panel width: 32 up to n = 2048, where single-workgroup register panels cover every

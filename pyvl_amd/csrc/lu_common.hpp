@@ -5,13 +5,6 @@
 
 namespace pvl
 {
-// Pivot order of LAPACK's idamax: larger |a| first, the smaller row on ties (a NaN never
-// wins, so a column of NaNs keeps its diagonal row).
-__device__ __forceinline__ bool better(double v1, int p1, double v2, int p2)
-{
-    return v1 > v2 || (v1 == v2 && p1 < p2);
-}
-
 // Wave-wide reductions through DPP lane moves (no LDS round trips).  Each step combines a
 // lane with the lane 1, 2, 4, 8 places below it inside its row of 16 (row_shr), then rows
 // 0 -> 1 and 2 -> 3 (row_bcast:15), then rows 0-1 -> 2-3 (row_bcast:31); lane 63 ends with
