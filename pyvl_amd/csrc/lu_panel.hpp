@@ -36,6 +36,7 @@ __global__ void __launch_bounds__(512) panel_wg_kernel(T *__restrict__ P, int ld
     constexpr unsigned NONE = 0xFFFFFFFFu;
     __shared__ T prow[2][NBP];
     __shared__ T rowj[2][NBP];
+    __shared__ T urow[2][NBP]; // the pivot row's trailing columns, zero in its L slots
     __shared__ unsigned long long red_k[2][NT / 64];
     __shared__ unsigned red_p[2][NT / 64];
     // pivots stay in LDS until the end: a global store inside the loop would make every
@@ -83,16 +84,22 @@ __global__ void __launch_bounds__(512) panel_wg_kernel(T *__restrict__ P, int ld
     {
         const int par = J & 1;
         __syncthreads();
-        unsigned long long bk = 0;
-        unsigned br = NONE;
+        // the waves' records in one batch of LDS reads, compared without branches (eight reads one after
+        // the other were a fifth of the step)
+        unsigned long long k8[NT / 64];
+        unsigned r8[NT / 64];
 #pragma unroll
         for (int q = 0; q < NT / 64; ++q)
-        {
-            const unsigned long long k = red_k[par][q];
-            const unsigned r = red_p[par][q];
-            if (k > bk || (k == bk && r < br))
-                bk = k, br = r;
-        }
+            k8[q] = red_k[par][q], r8[q] = red_p[par][q];
+#pragma unroll
+        for (int d = NT / 128; d > 0; d /= 2)
+#pragma unroll
+            for (int q = 0; q < d; ++q)
+            {
+                const bool take = (k8[q + d] > k8[q]) | ((k8[q + d] == k8[q]) & (r8[q + d] < r8[q]));
+                k8[q] = take ? k8[q + d] : k8[q], r8[q] = take ? r8[q + d] : r8[q];
+            }
+        const unsigned br = r8[0];
         const int p = br == NONE ? J : (int)br; // every candidate NaN: keep row J in place
         // row J lives in thread J (J < NBP <= 512), slot 0; the pivot row in thread p % 512,
         // slot p / 512.  Both windows are in the same state (both rows are still active).
@@ -103,6 +110,9 @@ __global__ void __launch_bounds__(512) panel_wg_kernel(T *__restrict__ P, int ld
 #pragma unroll
                 for (int c = 0; c < NBP; ++c)
                     prow[par][c] = a[s][c];
+#pragma unroll
+                for (int c = 1; c < NBP; ++c)
+                    urow[par][c] = c < NBP - J ? a[s][c] : T(0);
             }
         if (tid == J)
         {
@@ -150,8 +160,7 @@ __global__ void __launch_bounds__(512) panel_wg_kernel(T *__restrict__ P, int ld
                 for (int c = 0; c + 1 < NBP; ++c)
                 {
                     // slot c + 1 is a trailing column while c + 1 < NBP - J, else an L entry
-                    const T u = (c + 1 < NBP - J) ? prow[par][c + 1] : T(0);
-                    a[s][c] = fma(-l, u, a[s][c + 1]);
+                    a[s][c] = fma(-l, urow[par][c + 1], a[s][c + 1]);
                 }
                 a[s][NBP - 1] = l;
             }
