@@ -47,7 +47,7 @@ void gmres_release_workspace();
 void set_error(const char *fmt, ...);
 hipStream_t stream();
 hipStream_t side_stream(); // nullptr (error set) if it cannot be created
-int side_groups(int per_cu = 5); // workgroup cap for grid-stride kernels on the side stream
+int side_groups(int per_cu); // workgroup cap for grid-stride kernels on the side stream
 
 // Kernels on the library stream's critical path raise their waves' issue priority above
 // the side stream's (priority 0), which shares their SIMDs.
@@ -157,8 +157,16 @@ struct alignas(32) ChainHead
     double start[3];
     SegBox box;
 };
-// Workgroups per CU of the self-induction on the side stream.
-constexpr int kChainSideGroups = 3;
+// Workgroups per CU of the self-induction on the side stream: three where it is what a step waits for,
+// two where the library stream's work is (the assembly and the solve, which grow with the square of
+// the bound surfaces).  Five steps with two / three groups: 1,024 bound surfaces and 12,800 to 25,600
+// wake panels (pairs / n_bound^2 from 320 to 1,290) 5.07 / 5.25, 5.06 / 5.30, 6.38 / 6.14, 8.11 / 7.89,
+// 10.0 / 9.5 ms; 2,048 and 19,200 to 32,000 (180 to 500) 7.4 / 8.6, 9.2 / 10.1, 11.3 / 12.0,
+// 16.4 / 16.4 ms; 256 and 3,200 1.86 / 1.95 ms.
+constexpr int chain_side_groups(double pairs, unsigned n_bound)
+{
+    return pairs > 550.0 * n_bound * n_bound ? 3 : 2;
+}
 // Line circulations gamma_l = sum of +-Gamma over the surfaces holding line l, lines < n_active.
 int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, double *gamma, hipStream_t s);
 // SegRec and circulation (seg_gamma) of n_seg segments (seg_ab: node pairs; seg_line: mesh line |

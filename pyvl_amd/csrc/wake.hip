@@ -35,6 +35,7 @@ struct pvl_wake
     unsigned n_shed = 0, R = 0, n_te = 0;
     double tol = 0, current_time = 0;
     unsigned step_count = 0;
+    unsigned n_bound = 0;              // surfaces of the last update's bound mesh
     std::vector<uint32_t> col;         // [n_shed*2] column of (strip, side)
     std::vector<uint32_t> te_nodes;    // [n_te] bound node per column
     std::vector<uint32_t> nl_prefix;   // [R+1] lines used by ring rows < r
@@ -617,7 +618,8 @@ int pvl_wake_begin_update(pvl_wake *w, int mode, int precision)
     // wake nodes (pvl_wake_update evaluates at a copy of the same values)
     PVL_HIP(hipEventRecord(w->ev_ready, stream()));
     PVL_HIP(hipStreamWaitEvent(s, w->ev_ready, 0));
-    if (int st = self_partials(w, n_old, w->d_upos, precision, s, (unsigned)side_groups(kChainSideGroups)))
+    if (int st = self_partials(w, n_old, w->d_upos, precision, s,
+                               (unsigned)side_groups(chain_side_groups((double)n_old * na, w->n_bound))))
         return st;
     PVL_HIP(hipEventRecord(w->ev_done, s));
     w->pending = true;
@@ -649,6 +651,7 @@ int pvl_wake_update_flow(pvl_wake *w, double time, const pvl_mesh *bound, const 
     const unsigned n_te = w->n_te;
     const double dt = time - w->current_time;
     w->current_time = time;
+    w->n_bound = bound->n_surfaces;
     if (w->step_count == 0)
     {
         pin_row0_kernel<<<(n_te + 255) / 256, 256, 0, stream()>>>(w->d_upos, n_te, bound_pos_dev, w->d_te_nodes);
