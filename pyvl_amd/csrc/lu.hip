@@ -30,6 +30,7 @@
 
 #include <climits>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -1826,7 +1827,9 @@ __global__ void __launch_bounds__(kTrsvWgThreads) __attribute__((amdgpu_waves_pe
 // lane = row, coefficients from LDS eight columns ahead, x_k broadcast with readlane.  The upper
 // block's columns are scaled by 1/u_kk beforehand (u_ik / u_kk, off the critical path), so that the
 // chain has no division and the quotients are formed once at the end: one more rounding per
-// coefficient, a relative perturbation of U by half an ulp.
+// coefficient, a relative perturbation of U by half an ulp.  That holds while the scaled
+// coefficients stay normal numbers; a block with rows so unlike in scale that one does not keeps
+// its columns as they are and divides at every step.
 // Bound by the chain of blocks, ~2.5 us each: poll, last block's dot products, 64 substitution
 // steps, store.  At n = 1,024 in FP64 a solve took 420 us in one workgroup per triangle (bound by
 // how fast one CU streams the factor).
@@ -1908,18 +1911,34 @@ __global__ void __launch_bounds__(256)
     }
     __syncthreads();
     const T diag = D[lane][lane];
+    bool scaled = true;
     if constexpr (!LOWER)
     {
-        __syncthreads(); // diag is read by every wave before the columns are scaled
-        T u[16];
+        T u[16], c[16];
+        bool normal = true;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             u[i] = D[q + 4 * i][q + 4 * i];
-        __syncthreads();
 #pragma unroll
         for (int i = 0; i < 16; ++i)
+        {
+            c[i] = D[row][q + 4 * i];
             if (q + 4 * i > row)
-                D[row][q + 4 * i] = D[row][q + 4 * i] / u[i];
+            {
+                // a zero stays zero: its column's diagonal entry has to be an ordinary number
+                const T num = c[i];
+                c[i] = num / u[i];
+                const T m = fabs(num == T(0) ? u[i] : c[i]);
+                normal = normal && m >= std::numeric_limits<T>::min() && m <= std::numeric_limits<T>::max();
+            }
+        }
+        scaled = __syncthreads_and(normal);
+        if (scaled)
+        {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                D[row][q + 4 * i] = c[i];
+        }
     }
     T acc = T(0);
     bool ok = true;
@@ -1973,33 +1992,41 @@ __global__ void __launch_bounds__(256)
     if (w != 0)
         return;
     T x = live ? bv - sums[lane] : T(0), res = T(0);
-    constexpr int KC = 8;
-    T lc[KC], ln[KC];
+    auto substitute = [&](auto divide) {
+        constexpr int KC = 8;
+        T lc[KC], ln[KC];
 #pragma unroll
-    for (int u = 0; u < KC; ++u)
-        lc[u] = D[lane][LOWER ? u : BS - 1 - u];
-    for (int kc = 0; kc < BS; kc += KC)
-    {
-        if (kc + KC < BS)
+        for (int u = 0; u < KC; ++u)
+            lc[u] = D[lane][LOWER ? u : BS - 1 - u];
+        for (int kc = 0; kc < BS; kc += KC)
         {
+            if (kc + KC < BS)
+            {
+#pragma unroll
+                for (int u = 0; u < KC; ++u)
+                    ln[u] = D[lane][LOWER ? kc + KC + u : BS - 1 - (kc + KC + u)];
+            }
 #pragma unroll
             for (int u = 0; u < KC; ++u)
-                ln[u] = D[lane][LOWER ? kc + KC + u : BS - 1 - (kc + KC + u)];
-        }
+            {
+                const int k = LOWER ? kc + u : BS - 1 - (kc + u);
+                // the lane's own value is final at its step; what later steps do to it is not used
+                if constexpr (divide)
+                    x = lane == k ? x / diag : x;
+                const T xk = bcast_lane(x, k);
+                res = lane == k ? x : res;
+                x = fma(-lc[u], xk, x);
+            }
 #pragma unroll
-        for (int u = 0; u < KC; ++u)
-        {
-            const int k = LOWER ? kc + u : BS - 1 - (kc + u);
-            // the lane's own value is final at its step; what later steps do to it is not used
-            const T xk = bcast_lane(x, k);
-            res = lane == k ? x : res;
-            x = fma(-lc[u], xk, x);
+            for (int u = 0; u < KC; ++u)
+                lc[u] = ln[u];
         }
-#pragma unroll
-        for (int u = 0; u < KC; ++u)
-            lc[u] = ln[u];
-    }
-    if constexpr (!LOWER)
+    };
+    if (LOWER || scaled)
+        substitute(std::false_type{});
+    else
+        substitute(std::true_type{});
+    if (!LOWER && scaled)
         res = res / diag;
     if (!s_ok)
         res = T(NAN);
