@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(256) line_geom_kernel(unsigned n_lines, const 
     out[i] = g;
 }
 
-// Record of the accurate forms (LineMid) with the line's circulation, the sum over the surfaces
+// Record of the FP64 form (LineMid) with the line's circulation, the sum over the surfaces
 // holding the line of +-Gamma_s in increasing surface order.  A line cut by
 // length takes the far form everywhere (direction 0: every pair's c and h^2 are 0 and it is cut);
 // lengths whose squares could leave the range of a double never do.
@@ -102,6 +102,10 @@ __global__ void __launch_bounds__(256) line_mid_kernel(unsigned n_lines, const u
 template <int PREC> struct LineRecord
 {
     using type = LineMid;
+};
+template <> struct LineRecord<PVL_FP32>
+{
+    using type = LineGeom;
 };
 template <> struct LineRecord<PVL_FP64_REF_FORM>
 {
@@ -442,7 +446,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
         for (unsigned l = a; l < b; ++l)
         {
             const auto g = geom[l];
-            if constexpr (PREC == PVL_FP64_REF_FORM)
+            if constexpr (PREC != PVL_FP64)
                 line_k_acc<PREC, PPL>(g, gamma[l], px, py, pz, tol, tol2, vx, vy, vz);
             else
                 line_k_acc<PREC, PPL>(g, lines + 2 * l, pos, px, py, pz, tol, tol2, vx, vy, vz);
@@ -1037,7 +1041,7 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
                             const double *pts, int precision, unsigned n_active, const char *prof_name,
                             hipStream_t s, void *geom, double *gamma, double *partial, unsigned max_groups)
 {
-    if (precision == PVL_FP64_REF_FORM)
+    if (precision == PVL_FP32 || precision == PVL_FP64_REF_FORM)
     {
         line_geom_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, (LineGeom *)geom);
         PVL_HIP(hipGetLastError());

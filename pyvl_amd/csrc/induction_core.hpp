@@ -388,8 +388,8 @@ __device__ __forceinline__ bool mid_holds(double q, double len)
 
 // n . K(line, p) for the normal-reduced assembly.  The reference form dots the reference's K
 // (reference rounding of every product); the others form m (n . c) with c = dr1 x e and the
-// dot as FMAs, decide the cut-off once for the scalar, and take the far form when it holds for all
-// points of the wave.
+// dot as FMAs and decide the cut-off once for the scalar; FP64 takes the far form when it holds for
+// all points of the wave (FP32 keeps its single-precision angle at every distance).
 template <int PREC>
 __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double py, double pz, double nx, double ny,
                                           double nz, double tol, double tol2)
@@ -404,16 +404,19 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     {
         const double d1x = px - g.r1x, d1y = py - g.r1y, d1z = pz - g.r1z;
         const double d2x = px - g.r2x, d2y = py - g.r2y, d2z = pz - g.r2z;
-        const double q = g.len * far_rcp(fma(d1x, d2x, fma(d1y, d2y, d1z * d2z)));
         const double cx = fma(d1y, g.ez, -(d1z * g.ey));
         const double cy = fma(d1z, g.ex, -(d1x * g.ez));
         const double cz = fma(d1x, g.ey, -(d1y * g.ex));
         const double nc = fma(cx, nx, fma(cy, ny, cz * nz));
-        if (__builtin_amdgcn_ballot_w64(!mid_holds(q, g.len)) == 0)
+        if constexpr (PREC == PVL_FP64)
         {
-            const double h2 = fma(cx, cx, fma(cy, cy, cz * cz));
-            const double v = nc * mid_far<true>(q, h2);
-            return h2 < tol2 ? 0.0 : v;
+            const double q = g.len * far_rcp(fma(d1x, d2x, fma(d1y, d2y, d1z * d2z)));
+            if (__builtin_amdgcn_ballot_w64(!mid_holds(q, g.len)) == 0)
+            {
+                const double h2 = fma(cx, cx, fma(cy, cy, cz * cz));
+                const double v = nc * mid_far<true>(q, h2);
+                return h2 < tol2 ? 0.0 : v;
+            }
         }
         const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
         const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
@@ -424,7 +427,7 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     }
 }
 
-// The accurate forms of the point-velocity sums, from line records about the midpoint: m = p - mid,
+// The FP64 form of the point-velocity sums, from line records about the midpoint: m = p - mid,
 // c = m x e (= dr1 x e: K's direction, |c| = h), B = dr1 . dr2 = |m|^2 - len^2 / 4, three operations
 // fewer per pair than from the end points.  From two lengths off the midpoint on
 // (B >= far_b = 3.75 len^2, for all points of a wave, one comparison per line) the far form above
@@ -442,8 +445,8 @@ struct LineMid
 };
 static_assert(sizeof(LineMid) == sizeof(LineGeom), "one scratch size for both records");
 
-// v[j] += gamma K(line, p[j]): the point-velocity inner step.  The non-reference forms scale once
-// and accumulate with FMAs.
+// v[j] += gamma K(line, p[j]): the point-velocity inner step.  The FP32 form scales once and
+// accumulates with FMAs.
 template <int PREC, int PPL>
 __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, const double (&px)[PPL],
                                            const double (&py)[PPL], const double (&pz)[PPL], double tol, double tol2,
@@ -452,11 +455,24 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
 #pragma unroll
     for (int j = 0; j < PPL; ++j)
     {
-        double kx, ky, kz;
-        line_k<PREC>(g, px[j], py[j], pz[j], tol, tol2, kx, ky, kz);
-        vx[j] = vx[j] + gamma * kx;
-        vy[j] = vy[j] + gamma * ky;
-        vz[j] = vz[j] + gamma * kz;
+        if constexpr (PREC == PVL_FP64_REF_FORM)
+        {
+            double kx, ky, kz;
+            line_k<PREC>(g, px[j], py[j], pz[j], tol, tol2, kx, ky, kz);
+            vx[j] = vx[j] + gamma * kx;
+            vy[j] = vy[j] + gamma * ky;
+            vz[j] = vz[j] + gamma * kz;
+        }
+        else
+        {
+            double d1x, d1y, d1z;
+            bool cut;
+            const double m = line_m<PREC>(g, px[j], py[j], pz[j], tol, tol2, d1x, d1y, d1z, cut);
+            const double wm = cut ? 0.0 : gamma * m;
+            vx[j] = fma(wm, fma(d1y, g.ez, -(d1z * g.ey)), vx[j]);
+            vy[j] = fma(wm, fma(d1z, g.ex, -(d1x * g.ez)), vy[j]);
+            vz[j] = fma(wm, fma(d1x, g.ey, -(d1y * g.ex)), vz[j]);
+        }
     }
 }
 // ab: the line's two end points in the mesh (read only when near), pos: their coordinates.
