@@ -410,9 +410,9 @@ __global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines,
 // into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.70 ms (1.45 ms
 // in the general form with one point per lane; one point per lane in this form 0.74 ms).
 // SITE only gives the free-wake self-induction launch its own symbol for profilers.
-constexpr int kPvPPL = 2;
-
-template <int PREC, int SITE>
+// Where items of two points per lane would leave SIMDs short of waves, FP32 and the reference form take
+// one (point_velocity_ppl): a wave's chain of lines takes half the time.
+template <int PREC, int SITE, int PPL>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
     point_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, unsigned n_lines,
                           const typename LineRecord<PREC>::type *__restrict__ geom, const double *__restrict__ gamma,
@@ -421,7 +421,6 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
 {
     if constexpr (SITE == 0)
         main_stream_priority();
-    constexpr int PPL = kPvPPL;
     __shared__ double red[4][3][kWave * PPL];
     const unsigned w = wave_id(), lane = lane_id();
     const double tol2 = tol * tol;
@@ -494,6 +493,7 @@ __global__ void __launch_bounds__(256) chunk_reduce_kernel(unsigned n_pts, unsig
     if (i >= 3 * n_pts)
         return;
     double s = accumulate ? out[i] : 0.0;
+#pragma unroll 8
     for (unsigned c = 0; c < n_chunks; ++c)
         s = s + partial[(size_t)c * 3 * n_pts + i];
     out[i] = s;
@@ -655,8 +655,7 @@ __global__ void __launch_bounds__(256) chain_segment_kernel(unsigned n_seg, cons
                                                             const uint32_t *__restrict__ seg_line,
                                                             const double *__restrict__ nodes,
                                                             const double *__restrict__ gamma, unsigned n_active,
-                                                            double tol, SegRec *__restrict__ out,
-                                                            double *__restrict__ seg_gamma)
+                                                            double tol, SegRec *__restrict__ out)
 {
     const unsigned j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n_seg)
@@ -675,7 +674,7 @@ __global__ void __launch_bounds__(256) chain_segment_kernel(unsigned n_seg, cons
     const uint32_t l = ln & kInvalidId;
     double g = l < n_active ? gamma[l] : 0.0;
     g = (ln & kReversed) ? -g : g;
-    r.pad = 0.0;
+    r.gamma = g;
     const double l2 = r.len * r.len;
     constexpr double fa[kFarTerms] = {kFar1, kFar2, kFar3, kFar4, kFar5, kFar6, kFar7};
     double q = r.len * g;
@@ -687,7 +686,6 @@ __global__ void __launch_bounds__(256) chain_segment_kernel(unsigned n_seg, cons
         r.c[k + 1] = fa[k] * q;
     }
     out[j] = r;
-    seg_gamma[j] = g;
 }
 
 // Segments of a piece that are active at cr filled rows.
@@ -857,12 +855,13 @@ __device__ __forceinline__ void arrived(const SegRec &r)
 // Bound by VALU issue: 37 slots per pair in the far form (induction_core.hpp), 73 in the general
 // one.  A piece whose box is far enough from the box of the wave's points takes the far form for
 // all its segments without any test inside the loop (93 to 95 % of the pairs of a 400-row wake);
-// the end node's dr = p - r is the next segment's dr1.  Work items are (point block, piece chunk)
+// the end node's dr = p - r is the next segment's dr1.  FP32 keeps its single-precision angle at every
+// distance (the far form is more exact, but would move the results by the mode's own rounding).  Work items are (point block, piece chunk)
 // pairs, taken from a grid that may be smaller than their number (side stream).
 template <int PREC, int PPL>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PREC == PVL_FP32 ? 6 : 4)))
     chain_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, const ChainHead *__restrict__ heads,
-                          unsigned n_pieces, const SegRec *__restrict__ segs, const double *__restrict__ seg_gamma,
+                          unsigned n_pieces, const SegRec *__restrict__ segs,
                           unsigned n_chunks, double *__restrict__ partial, double tol, unsigned pblocks,
                           unsigned n_items, unsigned *__restrict__ queue)
 {
@@ -893,7 +892,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
             vx[i] = 0.0, vy[i] = 0.0, vz[i] = 0.0;
         }
         PointBox box;
-        if constexpr (PREC != PVL_FP64_REF_FORM)
+        if constexpr (PREC == PVL_FP64)
             box = point_box<PPL>(px, py, pz);
         for (unsigned k = chunk; k < n_pieces; k += n_chunks)
         {
@@ -908,11 +907,17 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
                 aq[i] = PREC == PVL_FP64_REF_FORM ? ax[i] * ax[i] + ay[i] * ay[i] + az[i] * az[i] : 0.0;
             }
             const SegRec *sg = segs + hd.first_seg;
-            const double *gg = seg_gamma + hd.first_seg;
             // one segment in the general form, and on to its end node
-            auto general = [&](unsigned j, AtanTable table) {
-                const double nx = sg[j].nx, ny = sg[j].ny, nz = sg[j].nz;
-                const double ex = sg[j].ex, ey = sg[j].ey, ez = sg[j].ez, len = sg[j].len, gamma = gg[j];
+            struct Seg
+            {
+                double nx, ny, nz, ex, ey, ez, len, gamma;
+            };
+            auto load = [&](unsigned j) {
+                return Seg{sg[j].nx, sg[j].ny, sg[j].nz, sg[j].ex, sg[j].ey, sg[j].ez, sg[j].len, sg[j].gamma};
+            };
+            auto general = [&](const Seg &r, AtanTable table) {
+                const double nx = r.nx, ny = r.ny, nz = r.nz;
+                const double ex = r.ex, ey = r.ey, ez = r.ez, len = r.len, gamma = r.gamma;
 #pragma unroll
                 for (int i = 0; i < PPL; ++i)
                 {
@@ -942,12 +947,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
                         vy[i] = fma(wm, cy, vy[i]);
                         vz[i] = fma(wm, cz, vz[i]);
                         ax[i] = px[i] - nx, ay[i] = py[i] - ny, az[i] = pz[i] - nz;
-                        __builtin_amdgcn_sched_barrier(0); // one point after the other: fewer registers
+                        if constexpr (PREC == PVL_FP64)
+                            __builtin_amdgcn_sched_barrier(0); // one point after the other: fewer registers
                     }
                 }
             };
             bool far = false;
-            if constexpr (PREC != PVL_FP64_REF_FORM)
+            if constexpr (PREC == PVL_FP64)
                 far = box_far(box, hd.box);
             if (far)
             {
@@ -972,11 +978,26 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
                 if (j < n)
                     work(r);
             }
+            else if constexpr (PREC == PVL_FP32)
+            {
+                // every pair comes here: the next record on its way as above
+                Seg r = load(0);
+                for (unsigned j = 0; j < n; ++j)
+                {
+                    const Seg q = load(j + 1 < n ? j + 1 : j);
+                    __builtin_amdgcn_sched_barrier(0);
+                    general(r, nullptr);
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" ::"s"(q.nx), "s"(q.ny), "s"(q.nz), "s"(q.ex), "s"(q.ey), "s"(q.ez), "s"(q.len),
+                                 "s"(q.gamma));
+                    r = q;
+                }
+            }
             else
             {
                 AtanTable table = PREC == PVL_FP64 ? atan_table() : nullptr;
                 for (unsigned j = 0; j < n; ++j)
-                    general(j, table);
+                    general(load(j), table);
             }
         }
 #pragma unroll
@@ -1006,7 +1027,6 @@ namespace pvl
 // plan would not fit pvl_point_velocity_noalloc's fixed scratch, the chunk count of 2,048 workgroups
 // of one point per lane, which is half as many.  One rule for both entry points: same sums.
 static bool self_site(const char *prof_name) { return std::strcmp(prof_name, "wake_self_velocity") == 0; }
-constexpr unsigned kPvPoints = kWave * kPvPPL; // per workgroup
 
 static void plan_chunks(unsigned n_pts, unsigned n_active, unsigned *n_chunks_out, unsigned *lpc_out)
 {
@@ -1023,9 +1043,17 @@ static void plan_chunks(unsigned n_pts, unsigned n_active, unsigned *n_chunks_ou
         *lpc = (n_active + n_chunks - 1) / n_chunks;
         return (n_active + *lpc - 1) / *lpc;
     };
-    *n_chunks_out = plan(4096, kPvPoints, lpc_out);
+    *n_chunks_out = plan(4096, 2 * kWave, lpc_out);
     if (point_velocity_scratch(n_pts, n_active, *n_chunks_out) > PVL_NOALLOC_SCRATCH_BYTES)
         *n_chunks_out = plan(2048, kWave, lpc_out);
+}
+
+// Points per lane: two where items of 128 points give every SIMD four waves (1,024 workgroups), and
+// always in FP64: the far form is chosen for a wave's points together, the same ones at every size.
+static int point_velocity_ppl(unsigned n_pts, unsigned n_chunks, int precision)
+{
+    const bool general = precision == PVL_FP32 || precision == PVL_FP64_REF_FORM;
+    return !general || (unsigned long long)((n_pts + 2 * kWave - 1) / (2 * kWave)) * n_chunks >= 1024 ? 2 : 1;
 }
 
 unsigned point_velocity_chunks(unsigned n_pts, unsigned n_active)
@@ -1054,21 +1082,30 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
     PVL_HIP(hipGetLastError());
     unsigned n_chunks, lpc;
     plan_chunks(n_pts, n_active, &n_chunks, &lpc);
-    const unsigned pblocks = (n_pts + kPvPoints - 1) / kPvPoints;
+    const unsigned points = kWave * point_velocity_ppl(n_pts, n_chunks, precision);
+    const unsigned pblocks = (n_pts + points - 1) / points;
     const unsigned n_items = pblocks * n_chunks;
     const unsigned grid = max_groups && max_groups < n_items ? max_groups : n_items;
     ProfScope prof(prof_name, (double)n_pts * (double)n_active, s);
     dispatch_precision(precision, [&](auto P) {
-        if (self_site(prof_name))
-            point_velocity_kernel<decltype(P)::value, 1>
+        const auto launch = [&](auto site, auto ppl) {
+            point_velocity_kernel<decltype(P)::value, decltype(site)::value, decltype(ppl)::value>
                 <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active,
-                (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
-                m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
+                                         (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
+                                         m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
+        };
+        const auto at = [&](auto ppl) {
+            if (self_site(prof_name))
+                launch(std::integral_constant<int, 1>{}, ppl);
+            else
+                launch(std::integral_constant<int, 0>{}, ppl);
+        };
+        if constexpr (decltype(P)::value == PVL_FP64)
+            at(std::integral_constant<int, 2>{});
+        else if (points == kWave)
+            at(std::integral_constant<int, 1>{});
         else
-            point_velocity_kernel<decltype(P)::value, 0>
-                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active,
-                (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
-                m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
+            at(std::integral_constant<int, 2>{});
     });
     PVL_HIP(hipGetLastError());
     return PVL_OK;
@@ -1085,13 +1122,12 @@ int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, 
 }
 
 int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_line, const double *nodes,
-                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, double *seg_gamma,
-                   hipStream_t s)
+                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, hipStream_t s)
 {
     if (n_seg == 0)
         return PVL_OK;
     chain_segment_kernel<<<(n_seg + 255) / 256, 256, 0, s>>>(n_seg, seg_ab, seg_line, nodes, gamma, n_active_lines,
-                                                             tol, out, seg_gamma);
+                                                             tol, out);
     PVL_HIP(hipGetLastError());
     return PVL_OK;
 }
@@ -1111,8 +1147,7 @@ unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces)
 }
 
 int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nodes, const ChainPiece *pieces,
-                            unsigned n_pieces, unsigned cr, const SegRec *segs, const double *seg_gamma,
-                            ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial,
+                            unsigned n_pieces, unsigned cr, const SegRec *segs, ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial,
                             unsigned max_groups)
 {
     const unsigned n_chunks = chain_velocity_chunks(n_pts, n_pieces);
@@ -1125,7 +1160,7 @@ int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nod
     ProfScope prof("wake_self_velocity", work, s);
     dispatch_precision(precision, [&](auto P) {
         chain_velocity_kernel<decltype(P)::value, kChainPPL><<<grid, kBlock, 0, s>>>(
-            n_pts, pts, heads, n_pieces, segs, seg_gamma, n_chunks, partial, tol, pblocks, n_items, queue);
+            n_pts, pts, heads, n_pieces, segs, n_chunks, partial, tol, pblocks, n_items, queue);
     });
     PVL_HIP(hipGetLastError());
     return PVL_OK;

@@ -140,7 +140,7 @@ struct alignas(128) SegRec
 {
     double nx, ny, nz;
     double ex, ey, ez;
-    double len, pad;
+    double len, gamma;
     double c[8];
 };
 static_assert(sizeof(SegRec) == 128, "SegRec layout");
@@ -163,24 +163,26 @@ struct alignas(32) ChainHead
 // wake panels (pairs / n_bound^2 from 320 to 1,290) 5.07 / 5.25, 5.06 / 5.30, 6.38 / 6.14, 8.11 / 7.89,
 // 10.0 / 9.5 ms; 2,048 and 19,200 to 32,000 (180 to 500) 7.4 / 8.6, 9.2 / 10.1, 11.3 / 12.0,
 // 16.4 / 16.4 ms; 256 and 3,200 1.86 / 1.95 ms.
-constexpr int chain_side_groups(double pairs, unsigned n_bound)
+constexpr int chain_side_groups(double pairs, unsigned n_bound, int precision)
 {
+    // FP32: every pair takes the general form, whose waves need more others beside them; five
+    // steps of 1,024 surfaces and 24,320 wake panels with three / five / six groups 13.7 / 12.5 / 11.8 ms
+    if (precision == PVL_FP32)
+        return 6;
     return pairs > 550.0 * n_bound * n_bound ? 3 : 2;
 }
 // Line circulations gamma_l = sum of +-Gamma over the surfaces holding line l, lines < n_active.
 int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, double *gamma, hipStream_t s);
-// SegRec and circulation (seg_gamma) of n_seg segments (seg_ab: node pairs; seg_line: mesh line |
+// SegRec of n_seg segments (seg_ab: node pairs; seg_line: mesh line |
 // bit 31 when the chain runs against the line's direction); lines >= n_active_lines carry no
 // circulation.
 int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_line, const double *nodes,
-                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, double *seg_gamma,
-                   hipStream_t s);
+                   const double *gamma, unsigned n_active_lines, double tol, SegRec *out, hipStream_t s);
 unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces);
 // Partial sums per piece chunk (3 n_pts doubles each, in chunk order; point_velocity_reduce adds
 // them); work = pairs evaluated, for the profiler.
 int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nodes, const ChainPiece *pieces,
-                            unsigned n_pieces, unsigned cr, const SegRec *segs, const double *seg_gamma,
-                            ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial, unsigned max_groups);
+                            unsigned n_pieces, unsigned cr, const SegRec *segs, ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial, unsigned max_groups);
 
 // Single-workgroup LU panel (lu_panel_f64.hip / lu_panel_f32.hip): factors the m x jb panel
 // at P (row stride lda; matrix rows row_base..) with partial pivoting, piv[row_base + j]

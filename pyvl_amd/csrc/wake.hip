@@ -67,7 +67,6 @@ struct pvl_wake
     ChainPiece *d_pieces = nullptr;
     std::vector<uint32_t> pieces_at; // [R+1] pieces active with r ring rows filled
     SegRec *d_segrec = nullptr;      // [n_seg] per-step records
-    double *d_seggamma = nullptr;    // [n_seg] their circulations
     ChainHead *d_heads = nullptr;    // [pieces] per-step heads
     bool pending = false;
     int pending_prec = 0;
@@ -362,7 +361,6 @@ int build_chains(pvl_wake *w, const std::vector<uint32_t> &lines)
     PVL_HIP(hipMalloc((void **)&w->d_seg_line, sizeof(uint32_t) * sl.size()));
     PVL_HIP(hipMalloc((void **)&w->d_pieces, sizeof(ChainPiece) * pieces.size()));
     PVL_HIP(hipMalloc((void **)&w->d_segrec, sizeof(SegRec) * sl.size()));
-    PVL_HIP(hipMalloc((void **)&w->d_seggamma, sizeof(double) * sl.size()));
     PVL_HIP(hipMalloc((void **)&w->d_heads, sizeof(ChainHead) * (pieces.size() + 1)));
     PVL_HIP(hipMemcpy(w->d_seg_ab, ab.data(), sizeof(uint32_t) * ab.size(), hipMemcpyHostToDevice));
     PVL_HIP(hipMemcpy(w->d_seg_line, sl.data(), sizeof(uint32_t) * sl.size(), hipMemcpyHostToDevice));
@@ -482,7 +480,6 @@ int pvl_wake_destroy(pvl_wake *w)
     (void)hipFree(w->d_seg_line);
     (void)hipFree(w->d_pieces);
     (void)hipFree(w->d_segrec);
-    (void)hipFree(w->d_seggamma);
     (void)hipFree(w->d_heads);
     pvl_mesh_destroy(w->full);
     pvl_mesh_destroy(w->row0);
@@ -566,10 +563,11 @@ static int self_partials(pvl_wake *w, unsigned n_pts, const double *pts, int pre
     if (int st = line_circulations(w->full, na, w->d_circ[w->cur], w->d_sgamma, s))
         return st;
     if (int st = chain_segments(w->n_seg, w->d_seg_ab, w->d_seg_line, w->d_upos, w->d_sgamma, na, w->tol, w->d_segrec,
-                                w->d_seggamma, s))
+                                s))
         return st;
     return chain_velocity_partials(n_pts, pts, w->d_upos, w->d_pieces, w->pieces_at[ar], ar, w->d_segrec,
-                                   w->d_seggamma, w->d_heads, precision, w->tol, (double)n_pts * (double)na, s, w->d_spartial, max_groups);
+                                   w->d_heads, precision, w->tol, (double)n_pts * (double)na, s, w->d_spartial,
+                                   max_groups);
 }
 
 // Orders the library stream after a started self-induction (its inputs may be overwritten
@@ -619,7 +617,7 @@ int pvl_wake_begin_update(pvl_wake *w, int mode, int precision)
     PVL_HIP(hipEventRecord(w->ev_ready, stream()));
     PVL_HIP(hipStreamWaitEvent(s, w->ev_ready, 0));
     if (int st = self_partials(w, n_old, w->d_upos, precision, s,
-                               (unsigned)side_groups(chain_side_groups((double)n_old * na, w->n_bound))))
+                               (unsigned)side_groups(chain_side_groups((double)n_old * na, w->n_bound, precision))))
         return st;
     PVL_HIP(hipEventRecord(w->ev_done, s));
     w->pending = true;

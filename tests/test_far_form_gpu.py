@@ -114,3 +114,17 @@ def test_assembly_at_every_run_length(n_span, n_chord):
     c, n = np.ascontiguousarray(cps[rows]), np.ascontiguousarray(nrm[rows])
     got, want = m.induction_matrix3(1e-6, pos, c, n), O.induction_matrix3(t, pos, c, n, 1e-6)
     assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("n_pts", [65, 3968, 3969, 4100])
+def test_point_velocity_fp32_points_per_lane(n_pts):
+    """FP32 on both sides of the point count where a lane takes two points (32 chunks of lines: 32
+    blocks of 128), against FP64: a pair's angle is a few 2^-24 off, a sum of terms of either sign some
+    ten times that, so 1e-5 of the largest velocity."""
+    pos, el = G.uv_sphere(64, 64, sigma=1e-3, seed=3)
+    m, rng = Mesh(pos.shape[0], el), np.random.default_rng(n_pts)
+    assert (m.n_lines + 255) // 256 == 32
+    pts, circ = rng.normal(0.0, 1.5, (n_pts, 3)), rng.normal(size=m.n_surfaces)
+    want = m.point_velocity(1e-6, pos, circ, pts)
+    got = m.point_velocity(1e-6, pos, circ, pts, precision=_lib.PVL_FP32)
+    assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
