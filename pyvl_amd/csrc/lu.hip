@@ -23,6 +23,7 @@
 // (trsv_flow_kernel).
 #include "pvl_internal.hpp"
 #include "lu_common.hpp"
+#include "lu_exchange.hpp"
 
 #include <rocblas/rocblas.h>
 
@@ -588,9 +589,9 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
         }
         // The rows that move, published by their owners (columns outside the sub-block, a lane each), and
         // read back: the pivot rows right of the sub-block by every group, left of it by their new
-        // owners, and the displaced rows by theirs.  Wave w handles pivot rows w and w + 4: the row that
-        // becomes one and the row that takes that one's place, so that what a wave overwrites it has
-        // itself published.
+        // owners, and the displaced rows by theirs.  Wave w handles pivot rows w and w + 4 (row_move): a
+        // position that it overwrites is published by no other wave of the group, so nothing but its own
+        // order stands between the two.
         const unsigned long long rtag = (unsigned long long)tag << 32;
         const bool outside = lane < jb && (lane < j0 || lane >= j0 + kb);
         const auto publish = [&](unsigned long long *dst, int row) {
@@ -619,10 +620,12 @@ __global__ void __launch_bounds__(256) panel_kernel(T *__restrict__ P, int lda, 
                     const int from = __builtin_amdgcn_readlane(at, t); // becomes pivot row t
                     const int fr = local_row(from), tr = local_row(j0 + t);
                     const bool own_from = from == fr * G + g, own_t = j0 + t == tr * G + g;
-                    if (own_from)
+                    const RowMove mv = row_move(t, from, j0, kb);
+                    if (own_from && mv.up)
                         publish(&X->row[0][t][lane][0], fr);
-                    if (own_t && from != j0 + t)
+                    if (own_t && mv.down)
                         publish(&X->row[1][t][lane][0], tr);
+                    src[i] = &X->row[mv.buf][mv.idx][lane][0];
                     need[i] = outside && (lane >= j0 + kb || (own_t && from != j0 + t));
                     dst[i] = tr;
                     if (own_from && from >= j0 + kb) // its place is taken by a row of the sub-block
