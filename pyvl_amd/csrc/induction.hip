@@ -37,15 +37,10 @@ constexpr int kCptTile = 64; // control points per workgroup (one per lane)
 // and length are stored as 0 (instead of the 0/0 of a zero-length line), so that its angle
 // and the fused accumulation (0 * direction) are 0.  With tol <= 0 nothing is cut by length
 // and the reference's values, NaN included, are kept.
-__global__ void __launch_bounds__(256) line_geom_kernel(unsigned n_lines, const uint32_t *__restrict__ lines,
-                                                       const double *__restrict__ pos, double tol,
-                                                       LineGeom *__restrict__ out)
+__device__ __forceinline__ LineGeom line_geom(const uint32_t *__restrict__ ab, const double *__restrict__ pos,
+                                              double tol)
 {
-    main_stream_priority();
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_lines)
-        return;
-    const uint32_t p1 = lines[2 * i] & kInvalidId, p2 = lines[2 * i + 1] & kInvalidId;
+    const uint32_t p1 = ab[0] & kInvalidId, p2 = ab[1] & kInvalidId;
     LineGeom g;
     g.r1x = pos[3 * p1 + 0], g.r1y = pos[3 * p1 + 1], g.r1z = pos[3 * p1 + 2];
     g.r2x = pos[3 * p2 + 0], g.r2y = pos[3 * p2 + 1], g.r2z = pos[3 * p2 + 2];
@@ -56,61 +51,17 @@ __global__ void __launch_bounds__(256) line_geom_kernel(unsigned n_lines, const 
     g.ez = dz / g.len;
     if (g.len < tol)
         g.ex = g.ey = g.ez = g.len = 0.0;
-    out[i] = g;
+    return g;
 }
-
-// Record of the FP64 form (LineMid) with the line's circulation, the sum over the surfaces
-// holding the line of +-Gamma_s in increasing surface order.  A line cut by
-// length takes the far form everywhere (direction 0: every pair's c and h^2 are 0 and it is cut);
-// lengths whose squares could leave the range of a double never do.
-__global__ void __launch_bounds__(256) line_mid_kernel(unsigned n_lines, const uint32_t *__restrict__ lines,
-                                                      const double *__restrict__ pos, double tol,
-                                                      const uint32_t *__restrict__ loff,
-                                                      const uint32_t *__restrict__ lsurf,
-                                                      const double *__restrict__ circ, LineMid *__restrict__ out)
+__global__ void __launch_bounds__(256) line_geom_kernel(unsigned n_lines, const uint32_t *__restrict__ lines,
+                                                       const double *__restrict__ pos, double tol,
+                                                       LineGeom *__restrict__ out)
 {
     main_stream_priority();
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_lines)
-        return;
-    const uint32_t p1 = lines[2 * i] & kInvalidId, p2 = lines[2 * i + 1] & kInvalidId;
-    const double ax = pos[3 * p1 + 0], ay = pos[3 * p1 + 1], az = pos[3 * p1 + 2];
-    const double bx = pos[3 * p2 + 0], by = pos[3 * p2 + 1], bz = pos[3 * p2 + 2];
-    const double dx = bx - ax, dy = by - ay, dz = bz - az;
-    LineMid g;
-    g.mx = 0.5 * (ax + bx), g.my = 0.5 * (ay + by), g.mz = 0.5 * (az + bz);
-    g.len = sqrt(dx * dx + dy * dy + dz * dz);
-    g.ex = dx / g.len;
-    g.ey = dy / g.len;
-    g.ez = dz / g.len;
-    const bool cut = g.len < tol;
-    if (cut)
-        g.ex = g.ey = g.ez = g.len = 0.0;
-    g.quarter = 0.25 * (g.len * g.len);
-    g.far_b = cut ? 0.0 : (g.len >= 1e-100 && g.len <= 1e100) ? 3.75 * (g.len * g.len) : __builtin_inf();
-    g.gamma = 0.0;
-    for (uint32_t k = loff[i]; k < loff[i + 1]; ++k)
-    {
-        const uint32_t e = lsurf[k];
-        const double c = circ[e & kInvalidId];
-        g.gamma = (e & kReversed) ? g.gamma - c : g.gamma + c;
-    }
-    out[i] = g;
+    if (i < n_lines)
+        out[i] = line_geom(lines + 2 * i, pos, tol);
 }
-
-// The record each precision's kernels read.
-template <int PREC> struct LineRecord
-{
-    using type = LineMid;
-};
-template <> struct LineRecord<PVL_FP32>
-{
-    using type = LineGeom;
-};
-template <> struct LineRecord<PVL_FP64_REF_FORM>
-{
-    using type = LineGeom;
-};
 
 __device__ __forceinline__ unsigned wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
 __device__ __forceinline__ unsigned lane_id() { return threadIdx.x % kWave; }
@@ -380,15 +331,10 @@ __global__ void __launch_bounds__(kBlock)
 // ---------------------------------------------------------------------------------------
 // Point-velocity sums.  Line circulation gamma_l = sum over the surfaces holding line l
 // of +-Gamma_s, in increasing surface order (deterministic).
-__global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines, const uint32_t *__restrict__ loff,
-                                                               const uint32_t *__restrict__ lsurf,
-                                                               const double *__restrict__ circ,
-                                                               double *__restrict__ gamma)
+__device__ __forceinline__ double line_circulation(unsigned i, const uint32_t *__restrict__ loff,
+                                                   const uint32_t *__restrict__ lsurf,
+                                                   const double *__restrict__ circ)
 {
-    main_stream_priority();
-    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_lines)
-        return;
     double g = 0.0;
     for (uint32_t k = loff[i]; k < loff[i + 1]; ++k)
     {
@@ -396,7 +342,32 @@ __global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines,
         const double c = circ[e & kInvalidId];
         g = (e & kReversed) ? g - c : g + c;
     }
-    gamma[i] = g;
+    return g;
+}
+__global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines, const uint32_t *__restrict__ loff,
+                                                               const uint32_t *__restrict__ lsurf,
+                                                               const double *__restrict__ circ,
+                                                               double *__restrict__ gamma)
+{
+    main_stream_priority();
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_lines)
+        gamma[i] = line_circulation(i, loff, lsurf, circ);
+}
+// Both in one launch, for the point-velocity sums.
+__global__ void __launch_bounds__(256) line_record_kernel(unsigned n_lines, const uint32_t *__restrict__ lines,
+                                                          const double *__restrict__ pos, double tol,
+                                                          const uint32_t *__restrict__ loff,
+                                                          const uint32_t *__restrict__ lsurf,
+                                                          const double *__restrict__ circ, LineGeom *__restrict__ geom,
+                                                          double *__restrict__ gamma)
+{
+    main_stream_priority();
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_lines)
+        return;
+    geom[i] = line_geom(lines + 2 * i, pos, tol);
+    gamma[i] = line_circulation(i, loff, lsurf, circ);
 }
 
 // PPL points per lane (64 PPL per wave, point j * 64 + lane of the block); the workgroup's
@@ -405,18 +376,18 @@ __global__ void __launch_bounds__(256) line_circulation_kernel(unsigned n_lines,
 // does not depend on scheduling.  Work items are (64 PPL-point block, line chunk) pairs,
 // item = chunk * pblocks + block; workgroup b takes items b, b + gridDim.x, .. (a grid
 // smaller than the item count leaves CU slots to other work on the device; each item's
-// arithmetic is the same either way).  Bound by FP64 issue: 43 slots per far pair.  With PPL = 2
+// arithmetic is the same either way).  Bound by FP64 issue: 46 slots per far pair.  With PPL = 2
 // each lane runs two independent evaluation chains per line and every line's record, loaded once
-// into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.70 ms (1.45 ms
-// in the general form with one point per lane; one point per lane in this form 0.74 ms).
+// into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.75 ms (1.45 ms
+// in the general form with one point per lane).
 // SITE only gives the free-wake self-induction launch its own symbol for profilers.
 // Where items of two points per lane would leave SIMDs short of waves, FP32 and the reference form take
 // one (point_velocity_ppl): a wave's chain of lines takes half the time.
 template <int PREC, int SITE, int PPL>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
     point_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, unsigned n_lines,
-                          const typename LineRecord<PREC>::type *__restrict__ geom, const double *__restrict__ gamma,
-                          const uint32_t *__restrict__ lines, const double *__restrict__ pos, unsigned lines_per_chunk, double *__restrict__ partial, double tol, unsigned pblocks,
+                          const LineGeom *__restrict__ geom, const double *__restrict__ gamma,
+                          unsigned lines_per_chunk, double *__restrict__ partial, double tol, unsigned pblocks,
                           unsigned n_items)
 {
     if constexpr (SITE == 0)
@@ -444,11 +415,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))
         const unsigned b = (a + per_wave) < l1 ? (a + per_wave) : l1;
         for (unsigned l = a; l < b; ++l)
         {
-            const auto g = geom[l];
-            if constexpr (PREC != PVL_FP64)
-                line_k_acc<PREC, PPL>(g, gamma[l], px, py, pz, tol, tol2, vx, vy, vz);
-            else
-                line_k_acc<PREC, PPL>(g, lines + 2 * l, pos, px, py, pz, tol, tol2, vx, vy, vz);
+            const LineGeom g = geom[l];
+            line_k_acc<PREC, PPL>(g, gamma[l], px, py, pz, tol, tol2, vx, vy, vz);
         }
 #pragma unroll
         for (int j = 0; j < PPL; ++j)
@@ -1022,7 +990,7 @@ namespace pvl
 // entry point; the wake passes the prefix of lines its filled rows use -- the other lines
 // carry zero circulation).
 // Chunking: aim for 4,096 workgroups of two points per lane while keeping >= 64 lines per wave.  Half
-// of that left the last round of waves half empty (30,000 points: 0.80 against 0.72 ms); twice of
+// of that left the last round of waves half empty (30,000 points: 11 % more time); twice of
 // it gains 3 % there and costs 1 % in a wake of 3,200 panels, in partial sums.  Where the partial sums and the line records of such a
 // plan would not fit pvl_point_velocity_noalloc's fixed scratch, the chunk count of 2,048 workgroups
 // of one point per lane, which is half as many.  One rule for both entry points: same sums.
@@ -1069,16 +1037,9 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
                             const double *pts, int precision, unsigned n_active, const char *prof_name,
                             hipStream_t s, void *geom, double *gamma, double *partial, unsigned max_groups)
 {
-    if (precision == PVL_FP32 || precision == PVL_FP64_REF_FORM)
-    {
-        line_geom_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, (LineGeom *)geom);
-        PVL_HIP(hipGetLastError());
-        line_circulation_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_line_offsets,
-                                                                         m->d_line_surfs, circ, gamma);
-    }
-    else
-        line_mid_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, m->d_line_offsets,
-                                                               m->d_line_surfs, circ, (LineMid *)geom);
+    const LineGeom *g = (const LineGeom *)geom;
+    line_record_kernel<<<(n_active + 255) / 256, 256, 0, s>>>(n_active, m->d_lines, pos, tol, m->d_line_offsets,
+                                                              m->d_line_surfs, circ, (LineGeom *)geom, gamma);
     PVL_HIP(hipGetLastError());
     unsigned n_chunks, lpc;
     plan_chunks(n_pts, n_active, &n_chunks, &lpc);
@@ -1090,9 +1051,7 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
     dispatch_precision(precision, [&](auto P) {
         const auto launch = [&](auto site, auto ppl) {
             point_velocity_kernel<decltype(P)::value, decltype(site)::value, decltype(ppl)::value>
-                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active,
-                                         (const typename LineRecord<decltype(P)::value>::type *)geom, gamma,
-                                         m->d_lines, pos, lpc, partial, tol, pblocks, n_items);
+                <<<grid, kBlock, 0, s>>>(n_pts, pts, n_active, g, gamma, lpc, partial, tol, pblocks, n_items);
         };
         const auto at = [&](auto ppl) {
             if (self_site(prof_name))

@@ -427,35 +427,21 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
     }
 }
 
-// The FP64 form of the point-velocity sums, from line records about the midpoint: m = p - mid,
-// c = m x e (= dr1 x e: K's direction, |c| = h), B = dr1 . dr2 = |m|^2 - len^2 / 4, three operations
-// fewer per pair than from the end points.  From two lengths off the midpoint on
-// (B >= far_b = 3.75 len^2, for all points of a wave, one comparison per line) the far form above
-// holds.  Otherwise the whole wave takes the general form, from the line's own end points (its h^2 is the reference's, rounding
-// included, which is what separates the two near a line).  43 issue slots per far pair, against
-// ~102 of the general form.
-struct LineMid
-{
-    double mx, my, mz;
-    double quarter; // len^2 / 4
-    double ex, ey, ez;
-    double len;
-    double far_b; // infinity: always the general form
-    double gamma; // the line's circulation (point-velocity sums)
-};
-static_assert(sizeof(LineMid) == sizeof(LineGeom), "one scratch size for both records");
-
-// v[j] += gamma K(line, p[j]): the point-velocity inner step.  The FP32 form scales once and
-// accumulates with FMAs.
+// v[j] += gamma K(line, p[j]): the point-velocity inner step.  FP32 and FP64 scale once and accumulate
+// with FMAs.  FP64 takes the far form when it holds for all points of the wave (mid_holds): 46 issue
+// slots per far pair against ~102 of the general form.  Like the general form it starts from
+// the differences to the end points, so its error does not depend on where the mesh lies; records
+// about the line's midpoint (three slots fewer) carry the midpoint's rounding, of the size of the
+// coordinates: 4e-12 of the velocity for a body 1e5 radii off the origin, where the end points give 2e-15.
 template <int PREC, int PPL>
 __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, const double (&px)[PPL],
                                            const double (&py)[PPL], const double (&pz)[PPL], double tol, double tol2,
                                            double (&vx)[PPL], double (&vy)[PPL], double (&vz)[PPL])
 {
-#pragma unroll
-    for (int j = 0; j < PPL; ++j)
+    if constexpr (PREC == PVL_FP64_REF_FORM)
     {
-        if constexpr (PREC == PVL_FP64_REF_FORM)
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
         {
             double kx, ky, kz;
             line_k<PREC>(g, px[j], py[j], pz[j], tol, tol2, kx, ky, kz);
@@ -463,7 +449,12 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
             vy[j] = vy[j] + gamma * ky;
             vz[j] = vz[j] + gamma * kz;
         }
-        else
+        return;
+    }
+    else if constexpr (PREC == PVL_FP32)
+    {
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
         {
             double d1x, d1y, d1z;
             bool cut;
@@ -473,63 +464,56 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
             vy[j] = fma(wm, fma(d1z, g.ex, -(d1x * g.ez)), vy[j]);
             vz[j] = fma(wm, fma(d1x, g.ey, -(d1y * g.ex)), vz[j]);
         }
-    }
-}
-// ab: the line's two end points in the mesh (read only when near), pos: their coordinates.
-template <int PREC, int PPL>
-__device__ __forceinline__ void line_k_acc(const LineMid &g, const uint32_t *ab, const double *pos,
-                                           const double (&px)[PPL], const double (&py)[PPL], const double (&pz)[PPL],
-                                           double tol, double tol2, double (&vx)[PPL], double (&vy)[PPL],
-                                           double (&vz)[PPL])
-{
-    double cx[PPL], cy[PPL], cz[PPL], b[PPL], w[PPL];
-    bool far = true;
-#pragma unroll
-    for (int j = 0; j < PPL; ++j)
-    {
-        const double mx = px[j] - g.mx, my = py[j] - g.my, mz = pz[j] - g.mz;
-        b[j] = fma(mx, mx, fma(my, my, fma(mz, mz, -g.quarter)));
-        far = far && b[j] >= g.far_b;
-        cx[j] = fma(my, g.ez, -(mz * g.ey));
-        cy[j] = fma(mz, g.ex, -(mx * g.ez));
-        cz[j] = fma(mx, g.ey, -(my * g.ex));
-    }
-    if (__builtin_amdgcn_ballot_w64(!far) == 0)
-    {
-#pragma unroll
-        for (int j = 0; j < PPL; ++j)
-        {
-            const double h2 = fma(cx[j], cx[j], fma(cy[j], cy[j], cz[j] * cz[j]));
-            const double f = g.gamma * mid_far<false>(g.len * far_rcp(b[j]), h2);
-            w[j] = h2 < tol2 ? 0.0 : f;
-        }
+        return;
     }
     else
     {
-        AtanTable table = PREC == PVL_FP64 ? atan_table() : nullptr;
-        const double *r1 = pos + 3 * (size_t)(ab[0] & pvl::kInvalidId), *r2 = pos + 3 * (size_t)(ab[1] & pvl::kInvalidId);
+        double cx[PPL], cy[PPL], cz[PPL], q[PPL], w[PPL];
+        bool far = true;
 #pragma unroll
         for (int j = 0; j < PPL; ++j)
         {
-            const double d1x = px[j] - r1[0], d1y = py[j] - r1[1], d1z = pz[j] - r1[2];
-            const double d2x = px[j] - r2[0], d2y = py[j] - r2[1], d2z = pz[j] - r2[2];
-            const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
-            const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
-            bool cut;
-            const double f = g.gamma * pair_m<PREC, 2>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2,
-                                                       tol, tol2, cut, table);
-            w[j] = cut ? 0.0 : f;
+            const double d1x = px[j] - g.r1x, d1y = py[j] - g.r1y, d1z = pz[j] - g.r1z;
+            const double d2x = px[j] - g.r2x, d2y = py[j] - g.r2y, d2z = pz[j] - g.r2z;
+            q[j] = g.len * far_rcp(fma(d1x, d2x, fma(d1y, d2y, d1z * d2z)));
+            far = far && mid_holds(q[j], g.len);
             cx[j] = fma(d1y, g.ez, -(d1z * g.ey));
             cy[j] = fma(d1z, g.ex, -(d1x * g.ez));
             cz[j] = fma(d1x, g.ey, -(d1y * g.ex));
         }
-    }
+        if (__builtin_amdgcn_ballot_w64(!far) == 0)
+        {
 #pragma unroll
-    for (int j = 0; j < PPL; ++j)
-    {
-        vx[j] = fma(w[j], cx[j], vx[j]);
-        vy[j] = fma(w[j], cy[j], vy[j]);
-        vz[j] = fma(w[j], cz[j], vz[j]);
+            for (int j = 0; j < PPL; ++j)
+            {
+                const double h2 = fma(cx[j], cx[j], fma(cy[j], cy[j], cz[j] * cz[j]));
+                const double f = gamma * mid_far<false>(q[j], h2);
+                w[j] = h2 < tol2 ? 0.0 : f;
+            }
+        }
+        else
+        {
+            AtanTable table = atan_table();
+#pragma unroll
+            for (int j = 0; j < PPL; ++j)
+            {
+                const double d1x = px[j] - g.r1x, d1y = py[j] - g.r1y, d1z = pz[j] - g.r1z;
+                const double d2x = px[j] - g.r2x, d2y = py[j] - g.r2y, d2z = pz[j] - g.r2z;
+                const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
+                const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
+                bool cut;
+                const double f = gamma * pair_m<PREC, 2>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2,
+                                                         tol, tol2, cut, table);
+                w[j] = cut ? 0.0 : f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PPL; ++j)
+        {
+            vx[j] = fma(w[j], cx[j], vx[j]);
+            vy[j] = fma(w[j], cy[j], vy[j]);
+            vz[j] = fma(w[j], cz[j], vz[j]);
+        }
     }
 }
 
