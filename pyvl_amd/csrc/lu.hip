@@ -816,7 +816,8 @@ constexpr size_t nopiv_lds_elems()
 }
 
 // 1/x to half an ulp and a little: the hardware estimate (2^-24 in FP64), one third-order step,
-// and the specials (0, infinities, NaN) as a division gives them.
+// and the specials (0, infinities, NaN) as a division gives them.  In FP32, x or 1/x subnormal gives
+// 0 or NaN.
 __device__ __forceinline__ double fast_recip(double x)
 {
     const double r = __builtin_amdgcn_rcp(x);
@@ -1015,38 +1016,53 @@ __global__ void __launch_bounds__(kNopivThreads) __attribute__((amdgpu_waves_per
                 const int c0 = kSlab * s, row = c0 + lane;
                 const bool ok = row < NB;
                 T v[kSlab];
+                int slab_due = 0;
+                const auto factor = [&](auto recip) {
+                    slab_due = 0;
 #pragma unroll
-                for (int c = 0; c < kSlab; ++c)
-                    v[c] = ok ? S[row * LD + c0 + c] : T(0);
-                T u = bcast_lane(v[0], 0), r = fast_recip(u);
+                    for (int c = 0; c < kSlab; ++c)
+                        v[c] = ok ? S[row * LD + c0 + c] : T(0);
+                    T u = bcast_lane(v[0], 0), r = recip(u);
 #pragma unroll
-                for (int j = 0; j < kSlab; ++j)
-                {
-                    const double pa = fabs((double)u);
-                    const bool below = lane > j;
-                    const T own = below ? v[j] : T(0);
-                    const T l = own * r;
-                    // (identity padding past jb: a pivot of 1 over zeros, never due)
-                    due |= (int)(below & ok & (!(fabs((double)own) <= pa) | !(pa > 0.0)));
-                    asm volatile("" : "+v"(due)); // now, or every column's operands stay in registers for it
-                    if (lane == j)
-                        inv[c0 + j] = r;
-                    if (j + 1 < kSlab)
+                    for (int j = 0; j < kSlab; ++j)
                     {
-                        // the next pivot and its reciprocal first, from its row's entries (the
-                        // same operations as in its own lane): the other columns' updates fill
-                        // that chain's latency
-                        const T ujk = bcast_lane(v[j + 1], j);
-                        u = fma(-(bcast_lane(v[j], j + 1) * r), ujk, bcast_lane(v[j + 1], j + 1));
-                        r = fast_recip(u);
-                        v[j + 1] = fma(-l, ujk, v[j + 1]);
-                    }
+                        const double pa = fabs((double)u);
+                        const bool below = lane > j;
+                        const T own = below ? v[j] : T(0);
+                        const T l = own * r;
+                        // (identity padding past jb: a pivot of 1 over zeros, never due)
+                        slab_due |= (int)(below & ok & (!(fabs((double)own) <= pa) | !(pa > 0.0)));
+                        asm volatile("" : "+v"(slab_due)); // now, or every column's operands stay in registers for it
+                        if (lane == j)
+                            inv[c0 + j] = r;
+                        if (j + 1 < kSlab)
+                        {
+                            // the next pivot and its reciprocal first, from its row's entries (the
+                            // same operations as in its own lane): the other columns' updates fill
+                            // that chain's latency
+                            const T ujk = bcast_lane(v[j + 1], j);
+                            u = fma(-(bcast_lane(v[j], j + 1) * r), ujk, bcast_lane(v[j + 1], j + 1));
+                            r = recip(u);
+                            v[j + 1] = fma(-l, ujk, v[j + 1]);
+                        }
 #pragma unroll
-                    for (int k = j + 2; k < kSlab; ++k)
-                        v[k] = fma(-l, bcast_lane(v[k], j), v[k]);
-                    v[j] = below ? l : v[j];
-                    __builtin_amdgcn_sched_barrier(0); // or the broadcasts of several columns pile up in SGPRs
+                        for (int k = j + 2; k < kSlab; ++k)
+                            v[k] = fma(-l, bcast_lane(v[k], j), v[k]);
+                        v[j] = below ? l : v[j];
+                        __builtin_amdgcn_sched_barrier(0); // or the broadcasts of several columns pile up in SGPRs
+                    }
+                };
+                factor([](T x) { return fast_recip(x); });
+                if constexpr (sizeof(T) == 4)
+                {
+                    // a reciprocal that is no normal number: the estimate flushes subnormals, divisions
+                    // do not (FP64's estimate keeps them)
+                    wave_lds_fence();
+                    const T ri = fabs(inv[c0 + lane % kSlab]);
+                    if (__ballot(!(ri >= std::numeric_limits<T>::min() && ri <= std::numeric_limits<T>::max())))
+                        factor([](T x) { return T(1) / x; });
                 }
+                due |= slab_due;
                 if (ok)
                 {
 #pragma unroll
