@@ -815,24 +815,31 @@ __device__ __forceinline__ void arrived(const SegRec &r)
                  "s"(r.c[2]), "s"(r.c[3]), "s"(r.c[4]), "s"(r.c[5]), "s"(r.c[6]), "s"(r.c[7]));
 }
 
-// A lane has PPL points, a wave 64 PPL, a workgroup four times that; the waves of a workgroup walk
-// the same pieces, a chunk of them (every n_chunks-th piece, so that the pieces near the points are
-// spread over the chunks) per item, so that a segment's record is read into the scalar
+// A lane has PPL points, a wave 64 PPL.  FP64 and the reference form: a workgroup has four times that
+// and its waves walk the same pieces, a chunk of them (every n_chunks-th piece, so that the pieces near
+// the points are spread over the chunks) per item, so that a segment's record is read into the scalar
 // cache once for four waves (with a piece per wave the records' latency held the kernel at twice
-// its issue time).  Sums are written per chunk (no atomics, no exchange between waves).
+// its issue time); sums are written per chunk, with no exchange between waves.
 // Bound by VALU issue: 37 slots per pair in the far form (induction_core.hpp), 73 in the general
 // one.  A piece whose box is far enough from the box of the wave's points takes the far form for
 // all its segments without any test inside the loop (93 to 95 % of the pairs of a 400-row wake);
-// the end node's dr = p - r is the next segment's dr1.  FP32 keeps its single-precision angle at every
-// distance (the far form is more exact, but would move the results by the mode's own rounding).  Work items are (point block, piece chunk)
+// the end node's dr = p - r is the next segment's dr1.  Work items are (point block, piece chunk)
 // pairs, taken from a grid that may be smaller than their number (side stream).
+// FP32 keeps its single-precision angle at every distance (the far form is more exact, but would move
+// the results by the mode's own rounding), 68 slots for every pair, which hide the records' latency:
+// there the four waves share the points and take every fourth piece of the chunk, and add their sums
+// in LDS (chain_split).  Waves on one record wait and issue together; a free-wake step of 1,024 /
+// 2,048 / 2,048 surfaces and 25,600 / 19,200 / 32,000 wake panels took 2.43 / 1.81 / 4.18 ms with the
+// pieces shared and takes 2.36 / 1.63 / 3.74 ms.
+constexpr bool chain_split(int precision) { return precision == PVL_FP32; }
 template <int PREC, int PPL>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PREC == PVL_FP32 ? 6 : 4)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PREC == PVL_FP32 ? 8 : 4)))
     chain_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, const ChainHead *__restrict__ heads,
                           unsigned n_pieces, const SegRec *__restrict__ segs,
                           unsigned n_chunks, double *__restrict__ partial, double tol, unsigned pblocks,
                           unsigned n_items, unsigned *__restrict__ queue)
 {
+    constexpr bool SPLIT = chain_split(PREC);
     const unsigned w = wave_id(), lane = lane_id();
     const double tol2 = tol * tol;
     __shared__ unsigned s_item;
@@ -846,7 +853,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PRE
         if (item >= n_items)
             return;
         const unsigned chunk = item / pblocks;
-        const unsigned w0 = ((item - chunk * pblocks) * 4 + w) * (kWave * PPL);
+        const unsigned pb = item - chunk * pblocks;
+        const unsigned w0 = (SPLIT ? pb : pb * 4 + w) * (kWave * PPL);
         if (w0 >= n_pts)
             continue;
         const unsigned p0 = w0 + lane;
@@ -862,7 +870,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PRE
         PointBox box;
         if constexpr (PREC == PVL_FP64)
             box = point_box<PPL>(px, py, pz);
-        for (unsigned k = chunk; k < n_pieces; k += n_chunks)
+        for (unsigned k = SPLIT ? 4 * chunk + w : chunk; k < n_pieces; k += (SPLIT ? 4 : 1) * n_chunks)
         {
             const ChainHead &hd = heads[k];
             const unsigned n = hd.n_seg;
@@ -967,6 +975,33 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PRE
                 for (unsigned j = 0; j < n; ++j)
                     general(load(j), table);
             }
+        }
+        if constexpr (SPLIT)
+        {
+            // the waves' sums in wave order (red is next written after the next item's barriers)
+            __shared__ double red[3][3][kWave * PPL];
+            if (w > 0)
+            {
+#pragma unroll
+                for (int i = 0; i < PPL; ++i)
+                {
+                    red[w - 1][0][i * kWave + lane] = vx[i];
+                    red[w - 1][1][i * kWave + lane] = vy[i];
+                    red[w - 1][2][i * kWave + lane] = vz[i];
+                }
+            }
+            __syncthreads();
+            if (w > 0)
+                continue;
+#pragma unroll
+            for (int i = 0; i < PPL; ++i)
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+                {
+                    vx[i] = vx[i] + red[u][0][i * kWave + lane];
+                    vy[i] = vy[i] + red[u][1][i * kWave + lane];
+                    vz[i] = vz[i] + red[u][2][i * kWave + lane];
+                }
         }
 #pragma unroll
         for (int i = 0; i < PPL; ++i)
@@ -1092,16 +1127,19 @@ int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_l
 }
 
 constexpr int kChainPPL = 2;
-constexpr unsigned kChainPoints = 4 * kWave * kChainPPL; // per workgroup
 constexpr unsigned kChainItems = 4608;
+// points per workgroup
+constexpr unsigned chain_points(int precision) { return (chain_split(precision) ? 1 : 4) * kWave * kChainPPL; }
 
-unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces)
+unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces, int precision)
 {
+    const unsigned points = chain_points(precision), pblocks = (n_pts + points - 1) / points;
+    const unsigned max_chunks = std::max(1u, (n_pieces + 7) / 8);
+    if (chain_split(precision)) // 2,048 and 7,680 items: up to 4 % more time in the sizes above
+        return std::min(max_chunks, (3840u + pblocks - 1) / pblocks);
     // kChainItems work items (six per workgroup of the side stream: the last ones claimed are
     // the kernel's tail), a chunk of at least 8 pieces each.  More items cost more partial sums
     // (24 bytes per point and chunk, written and read once).
-    const unsigned pblocks = (n_pts + kChainPoints - 1) / kChainPoints;
-    const unsigned max_chunks = std::max(1u, (n_pieces + 7) / 8);
     return std::min(max_chunks, std::max(1u, kChainItems / pblocks));
 }
 
@@ -1109,8 +1147,8 @@ int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nod
                             unsigned n_pieces, unsigned cr, const SegRec *segs, ChainHead *heads, int precision, double tol, double work, hipStream_t s, double *partial,
                             unsigned max_groups)
 {
-    const unsigned n_chunks = chain_velocity_chunks(n_pts, n_pieces);
-    const unsigned pblocks = (n_pts + kChainPoints - 1) / kChainPoints;
+    const unsigned n_chunks = chain_velocity_chunks(n_pts, n_pieces, precision);
+    const unsigned points = chain_points(precision), pblocks = (n_pts + points - 1) / points;
     const unsigned n_items = pblocks * n_chunks;
     const unsigned grid = max_groups && max_groups < n_items ? max_groups : n_items;
     unsigned *queue = (unsigned *)(heads + n_pieces); // one spare head

@@ -165,10 +165,11 @@ struct alignas(32) ChainHead
 // 16.4 / 16.4 ms; 256 and 3,200 1.86 / 1.95 ms.
 constexpr int chain_side_groups(double pairs, unsigned n_bound, int precision)
 {
-    // FP32: every pair takes the general form, whose waves need more others beside them; five
-    // steps of 1,024 surfaces and 24,320 wake panels with three / five / six groups 13.7 / 12.5 / 11.8 ms
+    // FP32: every pair takes the general form; with four / five / six groups the steps of
+    // chain_velocity_kernel's comment take 2.36 / 2.57 / 2.58, 1.63 / 1.86 / 1.93 and 3.74 / 3.85 / 3.78 ms,
+    // one of 1,024 surfaces and 12,800 wake panels 1.08 / 1.20 / 1.20 ms
     if (precision == PVL_FP32)
-        return 6;
+        return 4;
     return pairs > 550.0 * n_bound * n_bound ? 3 : 2;
 }
 // Line circulations gamma_l = sum of +-Gamma over the surfaces holding line l, lines < n_active.
@@ -178,7 +179,7 @@ int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, 
 // circulation.
 int chain_segments(unsigned n_seg, const uint32_t *seg_ab, const uint32_t *seg_line, const double *nodes,
                    const double *gamma, unsigned n_active_lines, double tol, SegRec *out, hipStream_t s);
-unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces);
+unsigned chain_velocity_chunks(unsigned n_pts, unsigned n_pieces, int precision);
 // Partial sums per piece chunk (3 n_pts doubles each, in chunk order; point_velocity_reduce adds
 // them); work = pairs evaluated, for the profiler.
 int chain_velocity_partials(unsigned n_pts, const double *pts, const double *nodes, const ChainPiece *pieces,

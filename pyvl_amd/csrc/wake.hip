@@ -520,23 +520,23 @@ static unsigned active_rows(const pvl_wake *w)
 // Lines carrying circulation: those of ring rows < active_rows.
 static unsigned active_lines(const pvl_wake *w) { return w->nl_prefix[active_rows(w)]; }
 
-static unsigned self_chunks(const pvl_wake *w, unsigned n_pts)
+static unsigned self_chunks(const pvl_wake *w, unsigned n_pts, int precision)
 {
     if (w->chains)
-        return chain_velocity_chunks(n_pts, w->pieces_at[active_rows(w)]);
+        return chain_velocity_chunks(n_pts, w->pieces_at[active_rows(w)], precision);
     return point_velocity_chunks(n_pts, active_lines(w));
 }
 
 // Buffers of the self-induction: line circulations, segment records (chains) or line
 // geometry, and the per-chunk partial sums (grown on demand; a started sum must have been
 // consumed or dropped before they are regrown).
-static int self_buffers(pvl_wake *w, unsigned n_pts)
+static int self_buffers(pvl_wake *w, unsigned n_pts, int precision)
 {
     if (!w->chains && !w->d_sgeom)
         PVL_HIP(hipMalloc(&w->d_sgeom, line_geom_bytes(w->full->n_lines)));
     if (!w->d_sgamma)
         PVL_HIP(hipMalloc((void **)&w->d_sgamma, sizeof(double) * (w->full->n_lines ? w->full->n_lines : 1)));
-    const size_t pbytes = sizeof(double) * 3 * (size_t)n_pts * self_chunks(w, n_pts);
+    const size_t pbytes = sizeof(double) * 3 * (size_t)n_pts * self_chunks(w, n_pts, precision);
     if (pbytes > w->spartial_bytes)
     {
         // no queued kernel on either library stream may still use the old buffer
@@ -609,9 +609,9 @@ int pvl_wake_begin_update(pvl_wake *w, int mode, int precision)
     if (!w->ev_done)
         PVL_HIP(hipEventCreateWithFlags(&w->ev_done, hipEventDisableTiming));
     // no started sum is pending here: the buffers are free to regrow
-    if (int st = self_buffers(w, n_old))
+    if (int st = self_buffers(w, n_old, precision))
         return st;
-    const unsigned nc = self_chunks(w, n_old);
+    const unsigned nc = self_chunks(w, n_old, precision);
     // the wake state as the library stream leaves it now; the points are the first n_old
     // wake nodes (pvl_wake_update evaluates at a copy of the same values)
     PVL_HIP(hipEventRecord(w->ev_ready, stream()));
@@ -680,11 +680,11 @@ int pvl_wake_update_flow(pvl_wake *w, double time, const pvl_mesh *bound, const 
         {
             if (int st = drop_pending(w))
                 return st;
-            if (int st = self_buffers(w, n_old))
+            if (int st = self_buffers(w, n_old, precision))
                 return st;
             if (int st = self_partials(w, n_old, w->d_old, precision, stream(), 0))
                 return st;
-            if (int st = point_velocity_reduce(n_old, self_chunks(w, n_old), w->d_spartial, w->d_vel, 1, stream()))
+            if (int st = point_velocity_reduce(n_old, self_chunks(w, n_old, precision), w->d_spartial, w->d_vel, 1, stream()))
                 return st;
         }
     }
