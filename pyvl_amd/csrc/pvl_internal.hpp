@@ -162,7 +162,9 @@ struct alignas(32) ChainHead
 // the bound surfaces).  Five steps with two / three groups: 1,024 bound surfaces and 12,800 to 25,600
 // wake panels (pairs / n_bound^2 from 320 to 1,290) 5.07 / 5.25, 5.06 / 5.30, 6.38 / 6.14, 8.11 / 7.89,
 // 10.0 / 9.5 ms; 2,048 and 19,200 to 32,000 (180 to 500) 7.4 / 8.6, 9.2 / 10.1, 11.3 / 12.0,
-// 16.4 / 16.4 ms; 256 and 3,200 1.86 / 1.95 ms.
+// 16.4 / 16.4 ms; 256 and 3,200 1.86 / 1.95 ms.  The reference form, one step with two / three / five
+// groups: 1,024 and 25,600 8.57 / 8.16 / 8.29 ms, 1,024 and 6,400 0.98 / 1.04 / 1.25 ms, 2,048 and
+// 19,200 5.80 / 5.68 / 5.75 ms.  Until the wake's first update n_bound is 0: three.
 constexpr int chain_side_groups(double pairs, unsigned n_bound, int precision)
 {
     // FP32: every pair takes the general form; with four / five / six groups the steps of
@@ -172,6 +174,12 @@ constexpr int chain_side_groups(double pairs, unsigned n_bound, int precision)
         return 4;
     return pairs > 550.0 * n_bound * n_bound ? 3 : 2;
 }
+// The same for strip topologies that are no chains (point_velocity_kernel), whose waves are lighter: one
+// step with two / three / five / six groups, FP64, 1,024 bound surfaces and 25,600 wake panels
+// 3.13 / 2.75 / 2.70 / 2.52 ms, 1,024 and 6,400 0.83 / 0.83 / 0.84 / 0.90, 2,048 and 19,200
+// 1.93 / 1.76 / 1.63 / 1.71; reference form 9.33 / 8.95 / 8.74 / 8.79, 0.97 / 1.00 / 1.08 / 1.16,
+// 6.06 / 5.88 / 5.73 / 5.61; FP32 3.85 / 3.56 / 3.41 / 3.21, 0.82 / 0.83 / 0.84 / 0.85, 2.51 / 2.35 / 2.23 / 2.13.
+constexpr int line_side_groups(int precision) { return precision == PVL_FP32 ? 6 : 5; }
 // Line circulations gamma_l = sum of +-Gamma over the surfaces holding line l, lines < n_active.
 int line_circulations(const pvl_mesh *m, unsigned n_active, const double *circ, double *gamma, hipStream_t s);
 // SegRec of n_seg segments (seg_ab: node pairs; seg_line: mesh line |
