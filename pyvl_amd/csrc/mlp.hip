@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <vector>
 
 using namespace pvl;
@@ -947,7 +948,11 @@ int pvl_mlp_forward(pvl_mlp *h, const float *X_dev, float *Y_dev, int batch)
     if (batch <= 0)
         return PVL_OK;
     ProfScope prof("mlp_forward", (double)batch);
-    if (fused(h, false))
+    // the fused pass's workgroups read their inputs while others write outputs: buffers that share
+    // memory go through the layer buffers (inputs converted before the first output is written)
+    const uintptr_t x = (uintptr_t)X_dev, y = (uintptr_t)Y_dev;
+    const bool shared = x < y + sizeof(float) * (size_t)batch && y < x + sizeof(float) * (size_t)batch * h->d_in;
+    if (fused(h, false) && !shared)
     {
         if (int st = fused_attributes())
             return st;
