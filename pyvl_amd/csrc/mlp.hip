@@ -27,7 +27,7 @@ struct pvl_mlp
     size_t n_params = 0;
     float *d_p = nullptr, *d_g = nullptr, *d_m = nullptr, *d_v = nullptr; // FP32 master, grad, Adam
     bf16 *d_pb = nullptr;           // BF16 mirror
-    int cap_batch = 0;
+    int cap_batch = 0, cap_general = 0; // samples that the batch buffers hold (ensure_batch, ensure_general)
     std::vector<bf16 *> d_act;      // [n_layers] layer inputs A_l (batch x dims[l]) in BF16
     std::vector<float *> d_z;       // [n_layers] pre-activations Z_l (batch x dims[l+1]) FP32
     std::vector<bf16 *> d_delta;    // [n_layers] error of each layer's output (batch x dims[l+1])
@@ -642,32 +642,48 @@ __global__ void adam_kernel(float *__restrict__ p, const float *__restrict__ g, 
     }
 }
 
+// Buffers of a batch: the hidden layers' inputs and every layer's output error.
 int ensure_batch(pvl_mlp *h, int batch)
 {
     if (batch <= h->cap_batch)
         return PVL_OK;
     (void)hipStreamSynchronize(stream());
-    for (auto p : h->d_act)
-        (void)hipFree(p);
-    for (auto p : h->d_z)
-        (void)hipFree(p);
-    for (auto p : h->d_delta)
-        (void)hipFree(p);
-    (void)hipFree(h->d_loss_part);
     const int L = h->n_layers;
+    for (int l = 1; l < L; ++l)
+        (void)hipFree(h->d_act[l]), h->d_act[l] = nullptr;
+    for (auto &p : h->d_delta)
+        (void)hipFree(p), p = nullptr;
+    (void)hipFree(h->d_loss_part);
     h->cap_batch = 0;
     h->d_loss_part = nullptr;
-    h->d_act.assign(L, nullptr);
-    h->d_z.assign(L, nullptr);
-    h->d_delta.assign(L, nullptr);
     for (int l = 0; l < L; ++l)
     {
-        PVL_HIP(hipMalloc(&h->d_act[l], sizeof(bf16) * (size_t)batch * h->dims[l]));
-        PVL_HIP(hipMalloc(&h->d_z[l], sizeof(float) * (size_t)batch * h->dims[l + 1]));
+        if (l > 0)
+            PVL_HIP(hipMalloc(&h->d_act[l], sizeof(bf16) * (size_t)batch * h->dims[l]));
         PVL_HIP(hipMalloc(&h->d_delta[l], sizeof(bf16) * (size_t)batch * h->dims[l + 1]));
     }
     PVL_HIP(hipMalloc(&h->d_loss_part, sizeof(float) * (size_t)((batch + kRows - 1) / kRows)));
     h->cap_batch = batch;
+    return PVL_OK;
+}
+
+// What the general kernels need besides: the network inputs in BF16 and the pre-activations (the fused
+// pass keeps both in LDS).
+int ensure_general(pvl_mlp *h, int batch)
+{
+    if (int st = ensure_batch(h, batch))
+        return st;
+    if (batch <= h->cap_general)
+        return PVL_OK;
+    (void)hipStreamSynchronize(stream());
+    (void)hipFree(h->d_act[0]), h->d_act[0] = nullptr;
+    for (auto &p : h->d_z)
+        (void)hipFree(p), p = nullptr;
+    h->cap_general = 0;
+    PVL_HIP(hipMalloc(&h->d_act[0], sizeof(bf16) * (size_t)batch * h->dims[0]));
+    for (int l = 0; l < h->n_layers; ++l)
+        PVL_HIP(hipMalloc(&h->d_z[l], sizeof(float) * (size_t)batch * h->dims[l + 1]));
+    h->cap_general = batch;
     return PVL_OK;
 }
 
@@ -684,7 +700,7 @@ int launch_gemm(int M, int N, int R, const bf16 *A, long am, long ar, const bf16
 // Forward pass storing every layer's input (BF16) and pre-activation (FP32).
 int forward(pvl_mlp *h, const float *X, int batch)
 {
-    if (int st = ensure_batch(h, batch))
+    if (int st = ensure_general(h, batch))
         return st;
     const long nin = (long)batch * h->d_in;
     f32_to_bf16_kernel<<<256, 256, 0, stream()>>>(X, h->d_act[0], nin);
@@ -750,8 +766,8 @@ FusedNet fused_net(const pvl_mlp *h)
         net.w[l] = h->d_pb + h->w_off[l];
         net.wt[l] = l >= 1 && l + 1 < h->n_layers ? h->d_pt + (size_t)(l - 1) * h->width * h->width : nullptr;
         net.bias[l] = h->d_p + h->b_off[l];
-        net.act[l] = h->d_act.empty() ? nullptr : h->d_act[l];
-        net.delta[l] = h->d_delta.empty() ? nullptr : h->d_delta[l];
+        net.act[l] = h->d_act[l];
+        net.delta[l] = h->d_delta[l];
     }
     return net;
 }
@@ -858,6 +874,9 @@ int pvl_mlp_create(pvl_mlp **out, int d_in, int width, int n_layers)
         off += (size_t)h->dims[l + 1];
     }
     h->n_params = off;
+    h->d_act.assign(n_layers, nullptr);
+    h->d_z.assign(n_layers, nullptr);
+    h->d_delta.assign(n_layers, nullptr);
     int st = PVL_OK;
     auto alloc = [&](void **p, size_t bytes) {
         if (!st)
