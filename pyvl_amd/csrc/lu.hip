@@ -1838,7 +1838,7 @@ __global__ void __launch_bounds__(kTrsvWgThreads) __attribute__((amdgpu_waves_pe
 
 // Single right-hand side (the time loop's solve): one triangle per launch, a workgroup per block of
 // 64 rows.  A block's solution is published in `out`, whose entries hold a signalling NaN until
-// then (kUnsolved, which no arithmetic returns): whoever needs block k polls its 64 values
+// then (Unsolved<T>::bits, which no arithmetic returns): whoever needs block k polls its 64 values
 // themselves, one memory round trip instead of a flag's and the data's.  Every wave streams its 16
 // rows of the factor block by block, the next block's loads in flight while x of this one is
 // polled; a row's part of a block is a dot product of its own, added to the row's sum, and the
@@ -1854,7 +1854,8 @@ __global__ void __launch_bounds__(kTrsvWgThreads) __attribute__((amdgpu_waves_pe
 // how fast one CU streams the factor).
 // Workgroups take solve-order indices from a ticket counter, so every smaller index belongs to a
 // workgroup already running; the one with the last ticket resets the counter.  Each workgroup
-// puts its block of `reset` (the other triangle's buffer) back to kUnsolved.  Waits are bounded: a
+// puts its block of `reset` (the other triangle's buffer; for the upper one that is `in`, whose block it
+// has read by then) back to Unsolved<T>::bits.  Waits are bounded: a
 // timed-out wait is recorded in the pinned host word kAsyncErrorWord and the workgroup writes NaN.
 constexpr int kAsyncErrorWord = 8;
 template <typename T> struct Unsolved;
@@ -1879,8 +1880,8 @@ template <typename T> __global__ void __launch_bounds__(256) unsolved_kernel(T *
 
 template <typename T, bool LOWER>
 __global__ void __launch_bounds__(256)
-    trsv1_kernel(const T *__restrict__ A, int lda, int n, const T *__restrict__ in, const int *__restrict__ perm,
-                 T *__restrict__ out, T *__restrict__ final_out, T *__restrict__ reset,
+    trsv1_kernel(const T *__restrict__ A, int lda, int n, const T *in, const int *__restrict__ perm,
+                 T *__restrict__ out, T *__restrict__ final_out, T *reset,
                  unsigned *__restrict__ ticket, int *__restrict__ host)
 {
     main_stream_priority<3>();
