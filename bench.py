@@ -44,7 +44,9 @@ PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 (vector and MFMA)
 SELF_VELOCITY_HBM_BYTES = 71.82e6
 PEAK_HBM_GBS = 8000.0
 FLOP_PER_PAIR = 87.0  # induction pair (src/core/flow_solver.c:114-135, atan2 counted as 20)
-FLOP_WEIGHT = 6.0  # Gamma weighting of a point-velocity sum
+# Operations of a self-induction pair in the far form, which 93-95 % of a full wake's pairs take:
+# p - r2 3, B 5, cross product 9, h^2 5, 1/B 5, polynomial with the circulation in it 17, accumulation 6.
+FLOP_SELF_PAIR = 50.0
 
 C3 = dict(n_span=64, n_chord=16, span=8.0, chord=1.0, h0=0.1, omega=0.6, dt=1.0 / 16.0, rows=400, tol=1e-6)
 
@@ -109,7 +111,7 @@ def run_c3(mode: str, prec: int, steps: int, warmup: int, profile: bool):
 
 def roofline_from(prof) -> dict:
     ms, cnt, pairs = prof["wake_self_velocity"]
-    flops = pairs * (FLOP_PER_PAIR + FLOP_WEIGHT)
+    flops = pairs * FLOP_SELF_PAIR
     avg_ms = ms / max(cnt, 1)
     achieved = flops / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
     return {
@@ -121,10 +123,12 @@ def roofline_from(prof) -> dict:
         "traffic": SELF_VELOCITY_HBM_BYTES,
         "kernel": "chain_velocity_kernel<FP64> (free-wake self-induction over segment chains)",
         "note": "FP64 vector-ALU bound (peak: MI355X FP64 vector rate, 78.6 TFLOP/s, equal to its FP64 MFMA rate); "
-                f"algorithmic {FLOP_PER_PAIR + FLOP_WEIGHT:.0f} FLOP per (segment, point) pair, "
+                f"{FLOP_SELF_PAIR:.0f} FLOP per (segment, point) pair, those of the far form (the reference's "
+                "expression: 93), "
                 f"{pairs / max(cnt, 1):.4g} pairs per launch, avg {avg_ms:.3f} ms over {cnt} launches "
                 "(HIP events on the side stream the kernel is launched on, around this kernel only, over "
-                "the timed region; it runs beside the bound solve, capped at two or three workgroups per CU)",
+                "the timed region; it runs beside the bound solve, capped at two or three workgroups per CU, four "
+                "in FP32)",
     }
 
 

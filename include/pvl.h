@@ -49,14 +49,25 @@ enum pvl_status
 
 enum pvl_precision
 {
-    /* FP64 throughout.  Dot products, h^2 and the cut-off test in the reference's operation
-     * order without FMA; the subtended angle in the single-angle form
-     * atan2((t2-t1) h, h^2 + t1 t2) with this library's atan2. */
+    /* FP64 throughout.  The subtended angle in the single-angle form
+     * atan2((t2-t1) h, h^2 + t1 t2) with this library's atan2.  The tensors
+     * (pvl_induction_matrix, pvl_line_induction_matrix) take dot products, h^2 and the cut-off
+     * test in the reference's operation order without FMA.  So do pvl_induction_matrix3 and the
+     * point-velocity sums for points near a line; where 64 (matrix) or 128 (sums) points of
+     * consecutive number are all two lengths or more from a line's midpoint, and everywhere in the
+     * wake's self-induction, h^2 is |dr1 x e|^2, and the cut-off is decided by that.  The two decisions
+     * differ only for pairs with |h^2 - tol^2| of the order of the reference's own rounding, a few
+     * 1e-16 |dr1|^2, i.e. beside a line's extension; such a pair's |K| is below
+     * 2 len sqrt(tol^2 + 1e-15 |dr1|^2) / |dr1|^2.  As the form depends on the
+     * points evaluated together, a subset or another order of the points gives results that agree
+     * to rounding (1e-15), not bit for bit. */
     PVL_FP64 = 0,
-    /* mixed: FP64 geometry, cut-off test, h^2 and cross product; FP32 angle (~1e-7). */
+    /* mixed: FP64 geometry, cut-off test, h^2 and cross product; FP32 angle (~1e-7).  h^2 in the
+     * reference's order, in the wake's self-induction |dr1 x e|^2. */
     PVL_FP32 = 1,
     /* FP64 with the reference's own angle expression atan2(t2,h) - atan2(t1,h) (two calls of
-     * the HIP math library's atan2): the literal restatement, kept for cross-checks. */
+     * the HIP math library's atan2) and its h^2 and cut-off everywhere: the literal restatement,
+     * kept for cross-checks. */
     PVL_FP64_REF = 2,
 };
 

@@ -5,12 +5,18 @@
 //   K = cross(dr1, e) * (atan2(t2, h) - atan2(t1, h)) / h   otherwise
 //
 // |K| is the angle the segment subtends from p (no 1/(4 pi) factor).  The file must be
-// compiled with -ffp-contract=off: the dot products, h^2 and the cut-off test below then
+// compiled with -ffp-contract=off: in PVL_FP64_REF, in the tensors, and wherever else the general
+// form is taken from both end points (pair_m), the dot products, h^2 and the cut-off test
 // round exactly as the reference's GCC x86-64 build (left to right, no FMA), so the cut-off
 // branch is decided identically and the cancellation in h^2 near a segment's line (which
 // the reference's values carry) is reproduced.  FMAs appear only where written explicitly:
 // in the angle evaluation and, for the non-reference forms, in the cross product and the
 // circulation-weighted accumulation (1-ulp differences, no effect on the cut-off).
+// Two forms take h^2 = |dr1 x e|^2 with FMAs and decide the cut-off by that: the wake's
+// self-induction (cross_m, far_add) and the far form of the FP64 assembly and point sums (line_nk,
+// line_k_acc).  Its error is of the order of eps |dr1| h + (eps |dr1|)^2, the reference's of eps |dr1|^2, so the
+// decisions differ only where |h^2 - tol^2| is within a few eps |dr1|^2: beside a line's extension,
+// for a pair worth at most 2 len sqrt(tol^2 + 8 eps |dr1|^2) / |dr1|^2.
 //
 // Angle forms:
 //   PVL_FP64_REF  the reference's expression: two FP64 atan2 calls of the HIP math library.
@@ -22,10 +28,10 @@
 //                 whereas the difference of two atan2 values loses digits in the far field
 //                 (|angle| << pi); the two forms agree to that loss (~1e-14 at r/len ~ 100).
 //                 atan2 is this library's own (pvl_atan2 below), 1/h comes from a
-//                 refined reciprocal square root.  The wake's self-induction takes h^2 from
-//                 the cross product instead (cross_m below).
-//   PVL_FP32      as PVL_FP64 with the angle, h and 1/h in FP32 (cut-off, dots, h^2 and
-//                 cross(dr1, e) stay FP64); ~1e-7 relative.
+//                 refined reciprocal square root.  Far from a line (all points of a wave) a
+//                 polynomial in h^2 / B^2 takes the place of both (far forms below).
+//   PVL_FP32      as PVL_FP64's general form at every distance, with the angle, h and 1/h in FP32
+//                 (cut-off, dots, h^2 and cross(dr1, e) stay FP64); ~1e-7 relative.
 #pragma once
 
 #include "pvl_internal.hpp"
