@@ -392,6 +392,16 @@ __device__ __forceinline__ bool mid_holds(double q, double len)
     return (unsigned)(__double_as_longlong(q * len) >> 32) < 0x3FD11111u; // upper word of 1 / 3.75
 }
 
+// B = dr1 . dr2 from which on the far form holds for a line by itself (3.75 len^2; the same for a whole
+// wave, decided before the reciprocal).  Infinite, so never reached, for lines cut by length and for lengths
+// whose squares could leave the range of a double; the length is wave-uniform, its test scalar.
+__device__ __forceinline__ double mid_reach(double len)
+{
+    const unsigned hi = (unsigned)(__double_as_longlong(len) >> 32);
+    const bool in_range = hi - 0x2B300000u < 0x54C00000u - 0x2B300000u; // 2^-332 .. 2^333
+    return in_range ? 3.75 * (len * len) : __builtin_inf();
+}
+
 // n . K(line, p) for the normal-reduced assembly.  The reference form dots the reference's K
 // (reference rounding of every product); the others form m (n . c) with c = dr1 x e and the
 // dot as FMAs and decide the cut-off once for the scalar; FP64 takes the far form when it holds for
@@ -434,7 +444,7 @@ __device__ __forceinline__ double line_nk(const LineGeom &g, double px, double p
 }
 
 // v[j] += gamma K(line, p[j]): the point-velocity inner step.  FP32 and FP64 scale once and accumulate
-// with FMAs.  FP64 takes the far form when it holds for all points of the wave (mid_holds): 46 issue
+// with FMAs.  FP64 takes the far form when it holds for all points of the wave (mid_reach): 46 issue
 // slots per far pair against ~102 of the general form.  Like the general form it starts from
 // the differences to the end points, so its error does not depend on where the mesh lies; records
 // about the line's midpoint (three slots fewer) carry the midpoint's rounding, of the size of the
@@ -474,15 +484,16 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
     }
     else
     {
-        double cx[PPL], cy[PPL], cz[PPL], q[PPL], w[PPL];
+        double cx[PPL], cy[PPL], cz[PPL], b[PPL], w[PPL];
+        const double far_b = mid_reach(g.len);
         bool far = true;
 #pragma unroll
         for (int j = 0; j < PPL; ++j)
         {
             const double d1x = px[j] - g.r1x, d1y = py[j] - g.r1y, d1z = pz[j] - g.r1z;
             const double d2x = px[j] - g.r2x, d2y = py[j] - g.r2y, d2z = pz[j] - g.r2z;
-            q[j] = g.len * far_rcp(fma(d1x, d2x, fma(d1y, d2y, d1z * d2z)));
-            far = far && mid_holds(q[j], g.len);
+            b[j] = fma(d1x, d2x, fma(d1y, d2y, d1z * d2z));
+            far = far && b[j] >= far_b;
             cx[j] = fma(d1y, g.ez, -(d1z * g.ey));
             cy[j] = fma(d1z, g.ex, -(d1x * g.ez));
             cz[j] = fma(d1x, g.ey, -(d1y * g.ex));
@@ -493,7 +504,7 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
             for (int j = 0; j < PPL; ++j)
             {
                 const double h2 = fma(cx[j], cx[j], fma(cy[j], cy[j], cz[j] * cz[j]));
-                const double f = gamma * mid_far<false>(q[j], h2);
+                const double f = gamma * mid_far<false>(g.len * far_rcp(b[j]), h2);
                 w[j] = h2 < tol2 ? 0.0 : f;
             }
         }

@@ -66,3 +66,17 @@ def test_mid_holds_lets_through_two_lengths_and_nothing_else():
     assert holds(0.0) and holds(5e-324) and holds(0.2666)
     for x in (1.0 / 3.75, 0.27, 1.0, np.inf, np.nan, -0.0, -1e-300, -1.0, -np.inf):
         assert not holds(x)
+
+
+def test_mid_reach_takes_lengths_whose_squares_are_normal_numbers():
+    body = SRC[SRC.index("double mid_reach("):]
+    lo, hi, lo2 = (int(x, 16) for x in re.findall(r"(0x[0-9A-F]+)u", body[:body.index(";", body.index("in_range"))]))
+    assert lo == lo2
+
+    def in_range(x):
+        return ((struct.unpack("<Q", struct.pack("<d", x))[0] >> 32) - lo) % 2**32 < hi - lo
+
+    for x in (1e-99, 1e-6, 1.0, 1e99, 2.0**-332, 2.0**332.999):
+        assert in_range(x) and np.finfo(float).tiny < 3.75 * (x * x) < np.inf
+    for x in (0.0, 5e-324, 1e-101, 2.0**333, 1e300, np.inf, np.nan):
+        assert not in_range(x)
