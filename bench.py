@@ -41,7 +41,7 @@ PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 (vector and MFMA)
 # WRITE_SIZE in two runs of this script (--copy-calibration), each scaled by what the same
 # counter reads for the script's own 1 GiB copy (FETCH x 2.0, WRITE x 1.0); the commands and
 # numbers are in profiles/wake_self_velocity_c3_fp64_traffic.md.
-SELF_VELOCITY_HBM_BYTES = 71.82e6
+SELF_VELOCITY_HBM_BYTES = 149.7e6
 PEAK_HBM_GBS = 8000.0
 FLOP_PER_PAIR = 87.0  # induction pair (src/core/flow_solver.c:114-135, atan2 counted as 20)
 # Operations of a self-induction pair in the far form, which 93-95 % of a full wake's pairs take:

@@ -376,7 +376,8 @@ __global__ void __launch_bounds__(256) line_record_kernel(unsigned n_lines, cons
 // does not depend on scheduling.  Work items are (64 PPL-point block, line chunk) pairs,
 // item = chunk * pblocks + block; workgroup b takes items b, b + gridDim.x, .. (a grid
 // smaller than the item count leaves CU slots to other work on the device; each item's
-// arithmetic is the same either way).  Bound by FP64 issue: 46 slots per far pair.  With PPL = 2
+// arithmetic is the same either way).  Bound by FP64 issue: 46 slots per far pair (by counters
+// 50 VALU instructions per pair at 81 % issue, the near ones among them).  With PPL = 2
 // each lane runs two independent evaluation chains per line and every line's record, loaded once
 // into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.75 ms (1.45 ms
 // in the general form with one point per lane).
