@@ -53,7 +53,7 @@ enum pvl_precision
      * atan2((t2-t1) h, h^2 + t1 t2) with this library's atan2.  The tensors
      * (pvl_induction_matrix, pvl_line_induction_matrix) take dot products, h^2 and the cut-off
      * test in the reference's operation order without FMA.  So do pvl_induction_matrix3 and the
-     * point-velocity sums for points near a line; where 64 (matrix) or 128 (sums) points of
+     * point-velocity sums for points near a line; where 64 (matrix, small sums) or 128 points of
      * consecutive number are all two lengths or more from a line's midpoint, and everywhere in the
      * wake's self-induction, h^2 is |dr1 x e|^2, and the cut-off is decided by that.  The two decisions
      * differ only for pairs with |h^2 - tol^2| of the order of the reference's own rounding, a few

@@ -382,8 +382,8 @@ __global__ void __launch_bounds__(256) line_record_kernel(unsigned n_lines, cons
 // into scalar registers, serves twice the points: 30,000 points x 16,256 lines take 0.75 ms (1.45 ms
 // in the general form with one point per lane).
 // SITE only gives the free-wake self-induction launch its own symbol for profilers.
-// Where items of two points per lane would leave SIMDs short of waves, FP32 and the reference form take
-// one (point_velocity_ppl): a wave's chain of lines takes half the time.
+// Where items of two points per lane would leave SIMDs short of waves, each lane takes one
+// (point_velocity_ppl): a wave's chain of lines takes half the time.
 template <int PREC, int SITE, int PPL>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
     point_velocity_kernel(unsigned n_pts, const double *__restrict__ pts, unsigned n_lines,
@@ -1052,12 +1052,12 @@ static void plan_chunks(unsigned n_pts, unsigned n_active, unsigned *n_chunks_ou
         *n_chunks_out = plan(2048, kWave, lpc_out);
 }
 
-// Points per lane: two where items of 128 points give every SIMD four waves (1,024 workgroups), and
-// always in FP64: the far form is chosen for a wave's points together, the same ones at every size.
-static int point_velocity_ppl(unsigned n_pts, unsigned n_chunks, int precision)
+// Points per lane: two where items of 128 points give every SIMD four waves (1,024 workgroups).  FP64 with
+// one / two points per lane: 300 points and 100 lines 21 / 26 us, 2,054 and 960 33 / 44, 28,077 and 410
+// 45 / 50, 1,000 and 7,300 41 / 58; 100 points and 20,100 lines 42 / 36.
+static int point_velocity_ppl(unsigned n_pts, unsigned n_chunks)
 {
-    const bool general = precision == PVL_FP32 || precision == PVL_FP64_REF_FORM;
-    return !general || (unsigned long long)((n_pts + 2 * kWave - 1) / (2 * kWave)) * n_chunks >= 1024 ? 2 : 1;
+    return (unsigned long long)((n_pts + 2 * kWave - 1) / (2 * kWave)) * n_chunks >= 1024 ? 2 : 1;
 }
 
 unsigned point_velocity_chunks(unsigned n_pts, unsigned n_active)
@@ -1079,7 +1079,7 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
     PVL_HIP(hipGetLastError());
     unsigned n_chunks, lpc;
     plan_chunks(n_pts, n_active, &n_chunks, &lpc);
-    const unsigned points = kWave * point_velocity_ppl(n_pts, n_chunks, precision);
+    const unsigned points = kWave * point_velocity_ppl(n_pts, n_chunks);
     const unsigned pblocks = (n_pts + points - 1) / points;
     const unsigned n_items = pblocks * n_chunks;
     const unsigned grid = max_groups && max_groups < n_items ? max_groups : n_items;
@@ -1095,9 +1095,7 @@ int point_velocity_partials(const pvl_mesh *m, double tol, const double *pos, co
             else
                 launch(std::integral_constant<int, 0>{}, ppl);
         };
-        if constexpr (decltype(P)::value == PVL_FP64)
-            at(std::integral_constant<int, 2>{});
-        else if (points == kWave)
+        if (points == kWave)
             at(std::integral_constant<int, 1>{});
         else
             at(std::integral_constant<int, 2>{});

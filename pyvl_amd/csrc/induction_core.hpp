@@ -510,7 +510,9 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
         }
         else
         {
-            AtanTable table = atan_table();
+            // one point per lane has the registers for the coefficients
+            constexpr int COEF = PPL == 1 ? 1 : 2;
+            AtanTable table = COEF == 2 ? atan_table() : nullptr;
 #pragma unroll
             for (int j = 0; j < PPL; ++j)
             {
@@ -519,7 +521,7 @@ __device__ __forceinline__ void line_k_acc(const LineGeom &g, double gamma, cons
                 const double q1 = d1x * d1x + d1y * d1y + d1z * d1z;
                 const double q2 = d2x * d2x + d2y * d2y + d2z * d2z;
                 bool cut;
-                const double f = gamma * pair_m<PREC, 2>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2,
+                const double f = gamma * pair_m<PREC, COEF>(g.ex, g.ey, g.ez, g.len, d1x, d1y, d1z, q1, d2x, d2y, d2z, q2,
                                                          tol, tol2, cut, table);
                 w[j] = cut ? 0.0 : f;
             }
